@@ -186,7 +186,7 @@ int swe_create(const swe_mesh_desc* d, const swe_params* prm, swe_handle** out) 
     Mode md;
     if ((rc = mode_of(*prm, md))) return rc;
     if ((rc = check_sgn_lists(md, d->n_ux_dir, d->n_uy_dir))) return rc;
-    if ((rc = build_layout(*d, sort_window_default(), L))) return rc;
+    if ((rc = build_layout(*d, sort_window_default(), tile_slices_for(((int64_t)d->np + 63) / 64 * 64), L))) return rc;
     PoolCaps caps;
     caps.rows = L.np_pad;
     caps.slots = L.nslot;
@@ -202,7 +202,7 @@ int swe_create(const swe_mesh_desc* d, const swe_params* prm, swe_handle** out) 
     }
     h->P->use_graph = true;
     int id = -1;
-    if ((rc = pool_add(h->P, *d, *prm, nullptr, 0.0, std::numeric_limits<double>::infinity(), LLONG_MAX, &id, &L))) {
+    if ((rc = pool_add(h->P, *d, *prm, nullptr, 0.0, std::numeric_limits<double>::infinity(), LLONG_MAX, &id, &L, true))) {
         free_handle(h);
         return rc;
     }
@@ -371,7 +371,7 @@ int swe_compute_dt(swe_handle* h, const double* un, double* dt) {
     } else if (!h->state_set) {
         return fail(SWE_EINVAL, "no state has been set");
     }
-    launch_compute_dt(*P, U, nullptr, 1);
+    launch_compute_dt(*P, U, nullptr, 1, false);
     launch_finalize_dt(*P, 0);
     int rc = check_flags(P, kId);
     const int rc2 = read_field(P, kId, offsetof(InstDev, dt), dt, sizeof(double));

@@ -130,6 +130,9 @@ int make_consts(const swe_params& p, Consts& K) {
     K.sqrt_2_g = std::sqrt(2 / p.gravity);
     K.g_half = p.gravity / 2;
     K.g16 = 16 * p.gravity;
+    // lambda's quick sign test, where none of its products can overflow or underflow
+    K.lam_w = 1.01 / (2.34 * 2.34 * K.g_half);
+    K.lam_h = (K.g >= 1e-60 && K.g <= 1e60 && K.htiny <= 0x1p+60) ? 0x1p+300 : -1.0;
     K.fric = p.gravity * (p.mannings * p.mannings);
     K.ent_cst = 1.0e-10 * p.gravity * (p.max_water_h * p.max_water_h);
     K.type_test = p.type_test;
@@ -234,93 +237,92 @@ int validate_mesh(const swe_mesh_desc& d) {
 
 namespace {
 
-// Mean |i - j| over the off-diagonal entries of the CSR graph in the numbering `pos`
-// (pos[i] = position of row i; identity when null).
-double mean_offset(const swe_mesh_desc& d, const std::vector<int>* pos) {
-    std::atomic<int64_t> sum{0}, n{0};
-    parallel_for(d.np, [&](int64_t b0, int64_t e0) {
-        int64_t s = 0, c = 0;
-        for (int64_t i = b0; i < e0; ++i)
-            for (int p = d.ia[i] - 1; p < d.ia[i + 1] - 1; ++p) {
-                const int j = d.ja[p] - 1;
-                if (j == (int)i) continue;
-                const int a = pos ? (*pos)[(size_t)i] : (int)i, b = pos ? (*pos)[(size_t)j] : j;
-                s += (a > b) ? a - b : b - a;
-                ++c;
-            }
-        sum += s;
-        n += c;
-    });
-    return n.load() ? (double)sum.load() / (double)n.load() : 0.0;
-}
-
-// Reverse Cuthill-McKee order of the CSR graph (each component from a pseudo-peripheral node, the
-// end of a breadth-first sweep from a node of least degree; neighbours by increasing degree).
-std::vector<int> rcm_order(const swe_mesh_desc& d) {
-    const int np = d.np;
-    auto deg = [&](int i) { return d.ia[i + 1] - d.ia[i]; };
+// Locality order of the CSR graph, for a mesh handed over without coordinates: the rows are bisected
+// recursively, each part in the order of a breadth-first sweep from an end of it, so that every cut goes
+// across the part's longer dimension and runs of consecutive rows are compact in every direction.  Cuts
+// fall on multiples of the largest tile's rows while a part is larger than that, of a slice's below.  (A
+// reverse Cuthill-McKee order makes runs thin strips: the 256 rows of a tile of a 50,000-node mesh then
+// border on about 450 rows instead of 80.)
+struct Bisector {
+    const swe_mesh_desc& d;
     std::vector<int> order;
-    order.reserve((size_t)np);
-    std::vector<char> seen((size_t)np, 0);
-    std::vector<int> level((size_t)np, -1), nb;
-    auto bfs = [&](int s, bool record) {
-        // breadth-first sweep from s; returns the last node reached
-        std::vector<int> q{s};
-        level[(size_t)s] = 0;
-        int last = s;
-        for (size_t h = 0; h < q.size(); ++h) {
-            const int u = q[h];
-            last = u;
-            nb.clear();
-            for (int p = d.ia[u] - 1; p < d.ia[u + 1] - 1; ++p) {
+    std::vector<int> mark;             // stamp of the part or sweep that holds the node
+    std::atomic<int> stamp{0};
+
+    explicit Bisector(const swe_mesh_desc& m) : d(m), order((size_t)m.np), mark((size_t)m.np, -1) {
+        for (int i = 0; i < m.np; ++i) order[(size_t)i] = i;
+    }
+    // Breadth-first sweep from s over the nodes stamped `from`, restamped `to`, appended to seq.
+    void sweep(int s, int from, int to, std::vector<int>& seq) {
+        size_t h = seq.size();
+        seq.push_back(s);
+        mark[(size_t)s] = to;
+        for (; h < seq.size(); ++h)
+            for (int p = d.ia[seq[h]] - 1; p < d.ia[seq[h] + 1] - 1; ++p) {
                 const int v = d.ja[p] - 1;
-                if (v != u && level[(size_t)v] < 0) {
-                    level[(size_t)v] = level[(size_t)u] + 1;
-                    nb.push_back(v);
+                if (mark[(size_t)v] == from) {
+                    mark[(size_t)v] = to;
+                    seq.push_back(v);
                 }
             }
-            std::stable_sort(nb.begin(), nb.end(), [&](int a, int b) { return deg(a) < deg(b); });
-            q.insert(q.end(), nb.begin(), nb.end());
-        }
-        if (record)
-            for (int u : q) {
-                seen[(size_t)u] = 1;
-                order.push_back(u);
-            }
-        else
-            for (int u : q) level[(size_t)u] = -1;
-        return last;
-    };
-    std::vector<int> by_deg((size_t)np);
-    for (int i = 0; i < np; ++i) by_deg[(size_t)i] = i;
-    std::stable_sort(by_deg.begin(), by_deg.end(), [&](int a, int b) { return deg(a) < deg(b); });
-    for (int s : by_deg) {
-        if (seen[(size_t)s]) continue;
-        const int far = bfs(s, false);
-        bfs(far, true);
     }
-    std::reverse(order.begin(), order.end());
-    return order;
+    void run(int b, int e, int depth) {
+        const int n = e - b;
+        if (n <= 64) return;
+        const int part = stamp.fetch_add(3), seen = part + 1, done = part + 2;
+        for (int q = b; q < e; ++q) mark[(size_t)order[(size_t)q]] = part;
+        std::vector<int> seq, first;
+        seq.reserve((size_t)n);
+        for (int q = b; q < e; ++q) {                      // one connected piece after another
+            if (mark[(size_t)order[(size_t)q]] != part) continue;
+            first.clear();
+            sweep(order[(size_t)q], part, seen, first);
+            sweep(first.back(), seen, done, seq);
+            for (int u : first)                            // (one-way references may leave some behind)
+                if (mark[(size_t)u] == seen) sweep(u, seen, done, seq);
+        }
+        std::copy(seq.begin(), seq.end(), order.begin() + b);
+        std::vector<int>().swap(seq);
+        const int unit = (n > 64 * kMaxTileSlices) ? 64 * kMaxTileSlices : 64;
+        const int m = b + std::max(1, (n / 2 + unit / 2) / unit) * unit;
+        if (m >= e) return;
+        if (depth < 5 && n > (1 << 15)) {
+            std::thread t([=] { run(b, m, depth + 1); });
+            run(m, e, depth + 1);
+            t.join();
+        } else {
+            run(b, m, depth + 1);
+            run(m, e, depth + 1);
+        }
+    }
+};
+
+std::vector<int> locality_order(const swe_mesh_desc& d) {
+    Bisector B(d);
+    B.run(0, d.np, 0);
+    return std::move(B.order);
 }
 
-// SWE_REORDER: 0 keeps the caller's order, 2 always renumbers, otherwise (default) the rows are
-// renumbered by reverse Cuthill-McKee when the caller's numbering scatters neighbours (mean offset
-// above 2*sqrt(np): a lattice numbered row by row has about 0.7*sqrt(np), the loader's first-touch
-// numbering of an unstructured mesh about 3.4*sqrt(np)) and the new order is better.
 }  // namespace
 
-int reorder_mode() {
+bool reorder_enabled() {
     const char* v = std::getenv("SWE_REORDER");
-    const int m = v ? std::atoi(v) : 1;
-    return (m >= 0 && m <= 2) ? m : 1;
+    return !v || std::atoi(v) != 0;
 }
 
-// Internal numbering: a base order of the rows (the caller's, or reverse Cuthill-McKee when the
-// caller's numbering scatters neighbours), then inside consecutive windows of `sort_window` rows
+// Tiles are large where the pool has rows enough for several per CU of a 256-CU device (fewer halo rows per
+// row), small where it has not (more workgroups).  Measured per launch at 1, 2 and 4 slices: k_tile_lo 14.0,
+// 14.6, 15.0 us and k_tile_dt 17.1, 17.9, 18.5 us at 5k rows; k_tile_dt 20.4, 19.4, 18.6 us at 100k, the others
+// within 3%; 8 slices were slower than 4 at 1M and 16.8M rows (k_tile_apply 58.2 against 54.0 us, 864 against
+// 830).
+int tile_slices_for(int64_t rows) { return rows <= 32 * 1024 ? 1 : rows <= 128 * 1024 ? 2 : 4; }
+
+// Internal numbering: a base order of the rows (the locality order, or the caller's under SWE_REORDER=0),
+// then inside consecutive windows of `sort_window` rows
 // of it, rows stably sorted by length, so the 64 rows of a slice (one wave) mostly have equal
 // length.  Only the processing order and placement change; each row keeps its entries in the
 // caller's order, which is the order of every row sum.
-int build_layout(const swe_mesh_desc& d, int sort_window, HostLayout& L) {
+int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostLayout& L) {
     int rc = validate_mesh(d);
     if (rc) return rc;
     const int np = d.np, nnz = d.nnz;
@@ -333,13 +335,7 @@ int build_layout(const swe_mesh_desc& d, int sort_window, HostLayout& L) {
     L.iperm.resize((size_t)np);
     std::vector<int> base((size_t)np);
     for (int i = 0; i < np; ++i) base[(size_t)i] = i;
-    const int mode = reorder_mode();
-    if (mode == 2 || (mode == 1 && mean_offset(d, nullptr) > 2.0 * std::sqrt((double)np))) {
-        std::vector<int> rcm = rcm_order(d);
-        std::vector<int> pos((size_t)np);
-        for (int r = 0; r < np; ++r) pos[(size_t)rcm[(size_t)r]] = r;
-        if (mode == 2 || mean_offset(d, &pos) < mean_offset(d, nullptr)) base.swap(rcm);
-    }
+    if (reorder_enabled()) base = locality_order(d);
     const int W = std::max(1, sort_window);
     const int nwin = (np + W - 1) / W;
     parallel_for(nwin, [&](int64_t b, int64_t e) {
@@ -419,6 +415,45 @@ int build_layout(const swe_mesh_desc& d, int sort_window, HostLayout& L) {
     parallel_for(L.nsl, [&](int64_t b, int64_t e) {
         for (int64_t sl = b; sl < e; ++sl) slice_entries((int)sl, L.elist.data() + L.eoff[(size_t)sl]);
     }, 512);
+    // tiles: the halo of each (sorted), then the columns of its entries within it
+    const int ts = tile_slices, T = 64 * ts;
+    L.tile_slices = ts;
+    L.lcol.assign((size_t)L.nslot, 0);
+    L.halo.assign((size_t)L.nsl * kHaloStride, 0);
+    L.nhalo.assign((size_t)L.nsl, 0);
+    std::atomic<bool> fits{true};
+    std::atomic<int> longest{0};
+    parallel_for((L.nsl + ts - 1) / ts, [&](int64_t tb, int64_t te) {
+        std::vector<int> far;
+        for (int64_t t = tb; t < te; ++t) {
+            const int s0 = (int)t * ts, s1 = std::min(L.nsl, s0 + ts), r0 = s0 * 64, r1 = s1 * 64;
+            far.clear();
+            for (int r = r0; r < r1; ++r)
+                for (int q = 0; q < L.len[(size_t)r]; ++q) {
+                    const int j = L.col[(size_t)(L.sptr[(size_t)(r >> 6)] + (r & 63) + 64 * (int64_t)q)];
+                    if (j < r0 || j >= r1) far.push_back(j);
+                }
+            std::sort(far.begin(), far.end());
+            far.erase(std::unique(far.begin(), far.end()), far.end());
+            if ((int)far.size() > tile_halo_cap(ts, s1 - s0)) {
+                fits = false;
+                return;
+            }
+            for (int cur = longest.load(); (int)far.size() > cur && !longest.compare_exchange_weak(cur, (int)far.size());) {
+            }
+            std::copy(far.begin(), far.end(), L.halo.begin() + (int64_t)s0 * kHaloStride);
+            L.nhalo[(size_t)s0] = (int)far.size();
+            for (int r = r0; r < r1; ++r)
+                for (int q = 0; q < L.len[(size_t)r]; ++q) {
+                    const int64_t slot = L.sptr[(size_t)(r >> 6)] + (r & 63) + 64 * (int64_t)q;
+                    const int j = L.col[(size_t)slot];
+                    L.lcol[(size_t)slot] = (uint16_t)(
+                        (j >= r0 && j < r1) ? j - r0
+                                            : T + (int)(std::lower_bound(far.begin(), far.end(), j) - far.begin()));
+                }
+        }
+    }, 64);
+    L.max_halo = fits ? longest.load() : -1;
     const int* src[3] = {d.h_dir, d.ux_dir, d.uy_dir};
     const int ns[3] = {d.n_h_dir, d.n_ux_dir, d.n_uy_dir};
     for (int k = 0; k < 3; ++k) {
@@ -441,10 +476,11 @@ int dalloc(T** p, size_t n) {
 }
 
 // Device bytes per unit of each capacity.
-constexpr size_t kRowBytes = sizeof(int) + 2 * sizeof(uint8_t) + sizeof(double) * 2 + sizeof(Node) * 4 + sizeof(double) * 3 +
-                             sizeof(double) * 4 + sizeof(double) * 3;   // perm, len dpos, m z, S[3] scratch, ulo, alpha res Rm nwork, stage3
-constexpr size_t kSlotBytes = sizeof(int) + sizeof(int16_t) + sizeof(double2) * 2 + sizeof(double) * 2;  // col dcol c dmu d0 ework
-constexpr size_t kSliceBytes = sizeof(SliceInfo);
+constexpr size_t kRowBytes = sizeof(int) + 3 * sizeof(uint8_t) + sizeof(double) * 2 + sizeof(Node) * 4 + sizeof(double) * 3 +
+                             sizeof(double) * 4 + sizeof(double) * 3;   // perm, len dpos dirm, m z, S[3] scratch, ulo, alpha res Rm nwork, stage3
+constexpr size_t kSlotBytes = sizeof(int) + sizeof(int16_t) + sizeof(uint16_t) + sizeof(double2) * 2 +
+                              sizeof(double) * 2;   // col dcol lcol c dmu d0 ework
+constexpr size_t kSliceBytes = sizeof(SliceInfo) + sizeof(int) * kHaloStride;
 constexpr size_t kInstBytes = sizeof(InstDev) + sizeof(unsigned long long) + sizeof(int);
 constexpr size_t kBcBytes = sizeof(BcEntry) + 3 * sizeof(double);   // entry, value of each stage
 
@@ -454,7 +490,7 @@ void free_pool(Pool* P) {
                     P->elist,   P->S[0],  P->S[1], P->S[2],  P->scratch, P->ulo_h, P->ulo_q, P->d0,    P->dmu,
                     P->ework,   P->alpha, P->res,  P->Rm,    P->nwork, P->stage3, P->tab, P->vmax,
                     P->flags, P->bc,    P->bcv,  P->X[0], P->X[1], P->X[2], P->X[3], P->stage5, P->xscratch,
-                    P->bar};
+                    P->bar,     P->lcol,  P->halo,   P->tact,   P->dirm,  P->done};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (P->act) (void)hipFree(P->act);
@@ -504,6 +540,7 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     if (caps.rows > (int64_t)INT_MAX - 64) return fail(SWE_EINVAL, "at most 2^31 rows per pool");
     Pool* P = new Pool();
     P->sort_window = sort_window_default();
+    P->tile_slices = tile_slices_for(caps.rows);
     const int64_t slices = (caps.rows + 63) / 64;
     P->rows_cap = slices * 64;
     P->slots_cap = caps.slots;
@@ -535,6 +572,7 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     ALLOC(P->sl, (size_t)slices);
     ALLOC(P->len, R);
     ALLOC(P->dpos, R);
+    ALLOC(P->dirm, R);
     ALLOC(P->perm, R);
     ALLOC(P->m, R);
     ALLOC(P->z, R);
@@ -561,11 +599,15 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     P->bcv_stride = std::max<int64_t>(caps.bc, 1);
     ALLOC(P->bcv, 3 * (size_t)P->bcv_stride);
     ALLOC(P->act, (size_t)slices);
+    ALLOC(P->tact, (size_t)slices);
+    ALLOC(P->lcol, S);
+    ALLOC(P->halo, (size_t)slices * kHaloStride);
     ALLOC(P->bar, 2);
+    ALLOC(P->done, (kDoneGroups + 1) * kDoneStride);
 #undef ALLOC
     P->listed.assign((size_t)caps.instances, 0);
     for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        e = hipHostMalloc((void**)&P->act_host[k], sizeof(int) * (size_t)slices, hipHostMallocDefault);
+        e = hipHostMalloc((void**)&P->act_host[k], 2 * sizeof(int) * (size_t)slices, hipHostMallocDefault);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&P->act_ev[k], hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventRecord(P->act_ev[k], P->stream);
     }
@@ -586,7 +628,7 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     }
     // empty tables: every slice free, every instance free; len = 0 marks rows without work
     std::vector<SliceInfo> sl0((size_t)slices);
-    for (auto& s : sl0) s = SliceInfo{0, 0, -1, 0, {0, 0}};
+    for (auto& s : sl0) s = SliceInfo{0, 0, -1, 0, 0, 0};
     std::vector<InstDev> t0((size_t)caps.instances);
     std::memset(t0.data(), 0, sizeof(InstDev) * t0.size());
     e = hipMemcpy(P->sl, sl0.data(), sizeof(SliceInfo) * sl0.size(), hipMemcpyHostToDevice);
@@ -595,6 +637,7 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     if (e == hipSuccess) e = hipMemset(P->vmax, 0, sizeof(unsigned long long) * (size_t)caps.instances);
     if (e == hipSuccess) e = hipMemset(P->flags, 0, sizeof(int) * (size_t)caps.instances);
     if (e == hipSuccess) e = hipMemset(P->bar, 0, 2 * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMemset(P->done, 0, sizeof(unsigned) * (kDoneGroups + 1) * kDoneStride);
     int coop = 0;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, P->device);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&P->num_cu, hipDeviceAttributeMultiprocessorCount, P->device);
@@ -648,7 +691,7 @@ int check_sgn_lists(const Mode& md, int nux, int nuy) {
 }
 
 int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const double* un, double t0, double tfinal,
-             long long max_steps, int* id, HostLayout* keep) {
+             long long max_steps, int* id, HostLayout* keep, bool built) {
     Mode md;
     int rc = mode_of(prm, md);
     if (rc) return rc;
@@ -661,7 +704,7 @@ int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const doubl
     if (md.sgn && (rc = ensure_sgn_buffers(P))) return rc;
     HostLayout Lbuf;
     HostLayout& L = keep ? *keep : Lbuf;
-    if ((rc = build_layout(d, P->sort_window, L))) return rc;
+    if (!built && (rc = build_layout(d, P->sort_window, P->tile_slices, L))) return rc;
     int k = -1;
     for (int q = 0; q < P->inst_cap; ++q)
         if (!P->inst[(size_t)q].used) { k = q; break; }
@@ -682,16 +725,21 @@ int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const doubl
     std::vector<SliceInfo> sls((size_t)L.nsl);
     for (int s = 0; s < L.nsl; ++s)
         sls[(size_t)s] = SliceInfo{p0 + L.sptr[(size_t)s], e0 + L.eoff[(size_t)s], k,
-                                   (int)(L.eoff[(size_t)s + 1] - L.eoff[(size_t)s]), {0, 0}};
+                                   (int)(L.eoff[(size_t)s + 1] - L.eoff[(size_t)s]),
+                                   (s % L.tile_slices) ? 0 : std::min(L.tile_slices, L.nsl - s), L.nhalo[(size_t)s]};
     std::vector<uint8_t> len8(L.len.begin(), L.len.end()), dpos8(L.dpos.begin(), L.dpos.end());
     std::vector<int> colg((size_t)L.nslot);
     for (int64_t q = 0; q < L.nslot; ++q) colg[(size_t)q] = L.col[(size_t)q] + (int)r0;
+    std::vector<int> halog(L.halo);
+    for (int& j : halog) j += (int)r0;
     std::vector<BcEntry> bce((size_t)nbc);
+    std::vector<uint8_t> dirm((size_t)L.np_pad, 0);
     {
         int64_t q = 0;
         for (int comp = 0; comp < 3; ++comp)
             for (int node : L.lists[comp]) {
                 bce[(size_t)q] = BcEntry{node + (int)r0, k, comp, (int)(b0 + q)};
+                dirm[(size_t)node] |= (uint8_t)(1 << comp);
                 ++q;
             }
     }
@@ -704,11 +752,14 @@ int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const doubl
     hipError_t e = hipStreamWaitEvent(cs, P->released, 0);
     if (e == hipSuccess) e = up(P->len + r0, len8.data(), len8.size());
     if (e == hipSuccess) e = up(P->dpos + r0, dpos8.data(), dpos8.size());
+    if (e == hipSuccess) e = up(P->dirm + r0, dirm.data(), dirm.size());
     if (e == hipSuccess) e = up(P->perm + r0, L.perm.data(), sizeof(int) * L.perm.size());
     if (e == hipSuccess) e = up(P->m + r0, L.m.data(), sizeof(double) * L.m.size());
     if (e == hipSuccess) e = up(P->z + r0, L.z.data(), sizeof(double) * L.z.size());
     if (e == hipSuccess) e = up(P->col + p0, colg.data(), sizeof(int) * colg.size());
     if (e == hipSuccess) e = up(P->dcol + p0, L.dcol.data(), sizeof(int16_t) * L.dcol.size());
+    if (e == hipSuccess) e = up(P->lcol + p0, L.lcol.data(), sizeof(uint16_t) * L.lcol.size());
+    if (e == hipSuccess) e = up(P->halo + s0 * kHaloStride, halog.data(), sizeof(int) * halog.size());
     if (e == hipSuccess) e = up(P->c + p0, L.c.data(), sizeof(double2) * L.c.size());
     if (e == hipSuccess) e = up(P->elist + e0, L.elist.data(), sizeof(uint16_t) * L.elist.size());
     if (e == hipSuccess) e = up(P->bc + b0, bce.data(), sizeof(BcEntry) * bce.size());
@@ -742,6 +793,7 @@ int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const doubl
     I.nux = (int)L.lists[1].size();
     I.nuy = (int)L.lists[2].size();
     I.nc = md.sgn ? 5 : 3;
+    I.max_halo = L.max_halo;
     if ((rc = pool_activate(P, k, I, prm, un != nullptr, t0, tfinal, max_steps))) return rc;
     *id = k;
     return SWE_OK;
@@ -798,8 +850,14 @@ int pool_update_active(Pool* P) {
     SWE_HIPCHK(hipEventSynchronize(P->act_ev[b]));
     std::vector<std::pair<int64_t, int64_t>> runs;
     P->any_src = false;
+    P->any_bc_values = false;
+    bool tiles = true;
+    int max_halo = 0;
     for (int k = 0; k < P->inst_cap; ++k)
         if (P->inst[(size_t)k].used && P->listed[(size_t)k]) {
+            P->any_bc_values |= P->inst[(size_t)k].bc_kind >= SWE_BC_VALUES;
+            tiles &= P->inst[(size_t)k].max_halo >= 0;
+            max_halo = std::max(max_halo, P->inst[(size_t)k].max_halo);
             runs.emplace_back(P->inst[(size_t)k].slice0, P->inst[(size_t)k].nslices);
             Consts K;
             if (make_consts(P->inst[(size_t)k].prm, K) == SWE_OK && K.src != SRC_NONE) P->any_src = true;
@@ -808,9 +866,17 @@ int pool_update_active(Pool* P) {
     int n = 0;
     for (const auto& r : runs)
         for (int64_t s = r.first; s < r.first + r.second; ++s) P->act_host[b][n++] = (int)s;
+    int* const th = P->act_host[b] + n;
+    int nt = 0;
+    if (tiles)
+        for (const auto& r : runs)
+            for (int64_t s = r.first; s < r.first + r.second; s += P->tile_slices) th[nt++] = (int)s;
     if (n) SWE_HIPCHK(hipMemcpyAsync(P->act, P->act_host[b], sizeof(int) * (size_t)n, hipMemcpyHostToDevice, P->stream));
+    if (nt) SWE_HIPCHK(hipMemcpyAsync(P->tact, th, sizeof(int) * (size_t)nt, hipMemcpyHostToDevice, P->stream));
     SWE_HIPCHK(hipEventRecord(P->act_ev[b], P->stream));
     P->nact = n;
+    P->ntile = nt;
+    P->tile_nodes = (64 * P->tile_slices + max_halo + 15) / 16 * 16;
     return SWE_OK;
 }
 
@@ -865,6 +931,8 @@ int pool_set_params(Pool* P, int k, const swe_params& prm) {
 int pool_set_bc(Pool* P, int k, int kind, double amp, double period, double level) {
     if (kind < SWE_BC_NONE || kind > SWE_BC_STAGES) return fail(SWE_EINVAL, "unknown bc kind %d", kind);
     if (kind == SWE_BC_INFLOW && !(period != 0.0)) return fail(SWE_EINVAL, "inflow period must be non-zero");
+    P->inst[(size_t)k].bc_kind = kind;
+    if (kind >= SWE_BC_VALUES) P->any_bc_values = true;    // (a list update recomputes it exactly)
     const double v[3] = {amp, period, level};
     int rc = pool_set_field(P, k, offsetof(InstDev, bc_amp), v, sizeof v);
     if (rc) return rc;
@@ -904,8 +972,7 @@ int pool_download_state(Pool* P, int k, const Node* src, double* un) {
 // One SSP-RK3 step of every live instance (SOURCES/main.f90:71-91): A = U^n -> B -> C -> A.
 int record_dt(Pool* P) {
     const bool lam = P->mode.viscosity_type != SWE_GALERKIN;
-    launch_compute_dt(*P, P->S[0], lam ? P->d0 : nullptr, 0);
-    launch_finalize_dt(*P, 1);
+    if (!launch_compute_dt(*P, P->S[0], lam ? P->d0 : nullptr, 0, true)) launch_finalize_dt(*P, 1);
     return SWE_OK;
 }
 
@@ -914,13 +981,14 @@ int record_stages(Pool* P) {
     Node* A = P->S[0];
     Node* B = P->S[1];
     Node* C = P->S[2];
-    int rc;
-    if ((rc = launch_euler_stage(*P, A, A, B, lam ? P->d0 : nullptr, 0))) return rc;
-    launch_bdy(*P, B, 0);
-    if ((rc = launch_euler_stage(*P, B, A, C, nullptr, 1))) return rc;
-    launch_bdy(*P, C, 1);
-    if ((rc = launch_euler_stage(*P, C, A, A, nullptr, 2))) return rc;
-    launch_bdy(*P, A, 2);
+    const bool lists = P->any_bc_values || !bdy_fused(*P);
+    const Node* in[3] = {A, B, C};
+    Node* out[3] = {B, C, A};
+    for (int stage = 0; stage < 3; ++stage) {
+        const int rc = launch_euler_stage(*P, in[stage], A, out[stage], (lam && stage == 0) ? P->d0 : nullptr, stage, true);
+        if (rc) return rc;
+        if (lists) launch_bdy(*P, out[stage], stage);
+    }
     return SWE_OK;
 }
 
@@ -939,7 +1007,7 @@ int64_t tuning_hash(const Tuning& t) {
 
 // The captured step stays valid while the launch extents, the scheme and the schedules stay.
 int ensure_graph(Pool* P) {
-    const int64_t key[6] = {(int64_t)P->nact, (int64_t)P->ninst(), P->nbc(), (int64_t)P->wmax,
+    const int64_t key[6] = {(int64_t)P->nact * 2048 + (P->ntile > 0 ? P->tile_nodes : 0) * 2 + (P->any_bc_values ? 1 : 0), (int64_t)P->ninst(), P->nbc(), (int64_t)P->wmax,
                             (int64_t)(P->mode.viscosity_type * 128 + P->mode.viscous_type * 16 + P->mode.alpha * 4 +
                                       P->mode.roundoff * 2 + (P->any_src ? 1 : 0)),
                             tuning_hash(P->tune)};
@@ -1124,6 +1192,7 @@ int pool_tune(Pool* P, int steps, int trials) {
             const int b = blocks[cand % 3], remap = (cand / 3) % 2, kind = cand / 6;
             {
                 if (!block_supported(kid, b)) continue;
+                if (kid == KID_FCT_LO && kind == 2 && (b != 256 || P->ntile == 0)) continue;   // one workgroup size
                 P->tune.k[kid] = LaunchCfg{b, remap, kind};
                 double ms_min = std::numeric_limits<double>::infinity();
                 for (int t = 0; t < trials && !rc; ++t) {

@@ -33,16 +33,20 @@ extern const char* const kKernelNames[KID_COUNT];
 struct LaunchCfg {
     int block = 256;    // threads per workgroup (whole waves; 4 slices at 256)
     int remap = 1;      // XCD-aware workgroup order
-    int kind = 0;       // schedule kind (k_fct_lo in stages 2-3: 0 lambda per row inline,
-                        // 1 lambda entry-parallel in LDS); 0 for the other kernels
+    int kind = 0;       // schedule kind (k_fct_lo: 0 lambda per row inline, 1 lambda entry-parallel in LDS
+                        // in stages 2-3, 2 tiles); 0 for the other kernels
 };
-// Schedule kinds a kernel has (1 or 2).
+// Schedule kinds a kernel has.
 int kinds_of(int kid);
 struct Tuning {
-    LaunchCfg k[KID_COUNT];   // defaults: 256 threads, XCD-aware order (the tuner refines per mesh)
+    LaunchCfg k[KID_COUNT];   // defaults: 256 threads, XCD-aware order, tiles (the tuner refines per mesh)
+    Tuning() { k[KID_FCT_LO].kind = 2; }
 };
 // Workgroup sizes a kernel can be launched with.
 bool block_supported(int kid, int block);
+
+// Words of Pool::done: one per group of workgroups and one for the groups, a cache line each.
+constexpr unsigned kDoneGroups = 64, kDoneStride = 32;
 
 // ---- first-fit allocator over [0, cap) --------------------------------------------------------
 struct RangeAlloc {
@@ -66,14 +70,20 @@ struct HostLayout {
     std::vector<double> m, z;
     std::vector<uint16_t> elist;
     std::vector<int> lists[3];                        // Dirichlet lists, internal numbering
+    int tile_slices = 0;                              // tiles of this many slices,
+    int max_halo = -1;                                // longest halo; -1: one exceeds tile_halo_cap
+    std::vector<uint16_t> lcol;                       // per slot: column within its tile
+    std::vector<int> halo, nhalo;                     // per slice: kHaloStride rows (local numbering), count
 };
 int validate_mesh(const swe_mesh_desc& d);
-int build_layout(const swe_mesh_desc& d, int sort_window, HostLayout& L);
+int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostLayout& L);
+// Slices per tile for a pool of `rows` rows.
+int tile_slices_for(int64_t rows);
 // Rows sorted by length inside windows of this many rows: SWE_SORT_WINDOW, else 64.
 int sort_window_default();
-// SWE_REORDER: 0 keeps the caller's numbering as the base order, 1 (default) renumbers for locality
-// when the caller's numbering scatters neighbours (mean |i-j| above 2 sqrt(np)), 2 always.
-int reorder_mode();
+// SWE_REORDER: 0 keeps the caller's numbering as the base order; otherwise (default) rows are renumbered
+// for locality, so that tiles are compact.
+bool reorder_enabled();
 int make_consts(const swe_params& p, Consts& K);
 
 // ---- the pool ---------------------------------------------------------------------------------
@@ -86,7 +96,9 @@ struct InstHost {
     int np = 0, nnz = 0, np_pad = 0, wmax = 0;
     int64_t slice0 = 0, nslices = 0, slot0 = 0, nslots = 0, e0 = 0, ne = 0, bc0 = 0, nbc = 0;
     int nh = 0, nux = 0, nuy = 0;
+    int bc_kind = 0;                  // its boundary program (swe_bc_kind), as last queued
     int nc = 3;                       // components of the state: 3, or 5 for the SGN model
+    int max_halo = -1;                // longest halo of its tiles; -1: too long, the gather kernels run it
     swe_params prm{};
 };
 
@@ -129,6 +141,7 @@ struct Pool {
     SliceInfo* sl = nullptr;
     uint8_t* len = nullptr;           // row lengths and diagonal positions (rows hold at most kMaxRow)
     uint8_t* dpos = nullptr;
+    uint8_t* dirm = nullptr;          // Dirichlet components of each row (bdy_row)
     int* perm = nullptr;              // internal row -> caller's node (local numbering)
     double* m = nullptr;
     double* z = nullptr;
@@ -136,13 +149,20 @@ struct Pool {
     int16_t* dcol = nullptr;          // column offsets (read instead of col where they fit)
     double2* c = nullptr;
     uint16_t* elist = nullptr;
+    int tile_slices = 4;              // slices per tile
+    uint16_t* lcol = nullptr;         // per slot: column within the tile
+    int* halo = nullptr;              // per slice: kHaloStride rows
     // the slices the step kernels cover: those of the instances that are (or may be) stepping
     int* act = nullptr;
     int nact = 0;
     int* act_host[2] = {nullptr, nullptr};   // pinned staging, used alternately
     hipEvent_t act_ev[2] = {nullptr, nullptr};
     int act_buf = 0;
+    int* tact = nullptr;                     // first slices of their tiles, when every listed instance
+    int ntile = 0;                           // can be tiled (else 0: the gather kernels run)
+    int tile_nodes = 0;                      // their largest rows + halo: the LDS records of a workgroup
     std::vector<char> listed;                // per instance: its slices are in the list
+    bool any_bc_values = false;              // a listed instance's boundary program takes given values (k_bdy)
     bool any_src = false;                    // a listed instance has a source term (type_test)
     // states and work arrays
     Node* S[3] = {nullptr, nullptr, nullptr};   // S[0] holds U^n between steps
@@ -174,6 +194,7 @@ struct Pool {
     int step_form = 0;                // swe_step_form: 0 launch sequence (graph), 1 persistent (fct)
     bool coop_ok = false;             // the device takes cooperative launches
     int num_cu = 1;
+    unsigned* done = nullptr;         // the dt pass's counts of workgroups that are through (0 between launches)
     unsigned* bar = nullptr;          // the persistent step's barrier word and abort word
     bool use_graph = false;
     hipGraphExec_t gexec = nullptr;
@@ -192,13 +213,13 @@ struct PoolCaps {
     int instances = 1;
 };
 size_t pool_bytes(const PoolCaps& caps);
-int pool_create(const PoolCaps& caps, Pool** out);
+int pool_create(const PoolCaps& caps, Pool** out);   // tile_slices: tile_slices_for(caps.rows)
 void pool_destroy(Pool* P);
 // Admit a mesh: bulk data goes up on the copy stream; the instance starts stepping at the next
 // step queued after this call.  un may be null (state set later).  keep receives the layout
 // when the caller needs its maps (csr2slot, lists).
 int pool_add(Pool* P, const swe_mesh_desc& d, const swe_params& prm, const double* un, double t0,
-             double tfinal, long long max_steps, int* id, HostLayout* keep);
+             double tfinal, long long max_steps, int* id, HostLayout* keep, bool built = false);   // built: *keep is d's layout
 // Make instance k live once its mesh arrays are in place (layout: its ranges and sizes); with
 // packed_state, its state is in stage3 in the caller's numbering.  The instance joins the next step.
 int pool_activate(Pool* P, int k, const InstHost& layout, const swe_params& prm, bool packed_state, double t0,
@@ -260,9 +281,21 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
 
 // ---- launch wrappers (swe_kernels.hip) --------------------------------------------------------
 Mesh mesh_view(const Pool& P);
-void launch_compute_dt(Pool& P, const Node* U, double* d0, int all);
+// COMPUTE_DT's pass; true when it did the step's bookkeeping too (advance, on tiles), which otherwise is
+// launch_finalize_dt's.
+bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance);
 void launch_finalize_dt(Pool& P, int advance);
-int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage);
+// The tile form of k_fct_lo (swe_tiles.hip), where tiles_apply.
+inline bool tiles_apply(const Pool& P) { return P.ntile > 0 && P.tune.k[KID_FCT_LO].kind == 2; }
+void launch_tile_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo);
+void launch_tile_rminus(Pool& P, const Node* U);
+void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
+// The dt pass on tiles; advance: the last workgroup also does finalize_one for every instance.
+void launch_tile_dt(Pool& P, const Node* U, double* d0, int all, bool advance);
+int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage,
+                       bool bdy = false);
+// Whether launch_euler_stage can write the wall and inflow values itself (given values need launch_bdy).
+bool bdy_fused(const Pool& P);
 void launch_bdy(Pool& P, Node* u, int stage);
 // The persistent step form: whether it covers the pool's scheme (fct, three components) on this
 // device, and nsteps steps of every listed instance in cooperative launches.

@@ -18,6 +18,9 @@ namespace swe {
 
 __device__ __forceinline__ double fmaxF(double a, double b) { return (a > b) ? a : b; }
 __device__ __forceinline__ double fminF(double a, double b) { return (a < b) ? a : b; }
+// MAX(x, 0.d0) as one v_max_f64: a NaN x gives 0 there as in (x > 0 ? x : 0), and x is always the
+// result of an operation, so nothing has to be quieted first.
+__device__ __forceinline__ double posF(double x) { return __builtin_fmax(x, 0.0); }
 
 // SQRT of an argument that is a finite double of at least 2^-767: the instructions of the correctly
 // rounded sqrt hipcc emits for gfx950 (reciprocal square root, then Newton corrections in FMA),
@@ -48,6 +51,43 @@ __device__ __forceinline__ double sqrt_rn(double x) {
     return r;
 }
 
+// Divisions that share a divisor.  refined_rcp(b) is the reciprocal the correctly rounded division
+// hipcc emits for gfx950 works with (v_rcp_f64 and two Newton steps); div_shared finishes the
+// same sequence for one dividend (product, exact remainder, correction), so the quotient has the bits
+// of a / b.  The compiler's sequence also scales extreme operands and patches special ones; those
+// (divisor outside [2^-300, 2^300], dividend not 0 and outside [2^-500, 2^500], NaN) take a / b itself
+// in a branch only the waves that hold one take.  (-0 / b gives +0 here; no caller keeps that sign.)
+// Three instructions instead of eleven per further dividend.
+struct Rcp {
+    double b, y;
+    bool ok;
+};
+__device__ __forceinline__ Rcp refined_rcp(double b) {
+    double y = __builtin_amdgcn_rcp(b);
+    double e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    return {b, y, b >= 0x1p-300 && b <= 0x1p+300};
+}
+// The same for a divisor that is uniform per wave: its reciprocal stays in scalar registers.
+__device__ __forceinline__ Rcp uniform_rcp(double b) {
+    Rcp R = refined_rcp(b);
+    const long long v = __double_as_longlong(R.y);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32));
+    R.y = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    return R;
+}
+__device__ __forceinline__ double div_shared(double a, const Rcp& R) {
+    double q = a * R.y;
+    const double e = __builtin_fma(-R.b, q, a);
+    q = __builtin_fma(e, R.y, q);
+    const double m = fabs(a);
+    if (__builtin_expect(!(R.ok && ((m >= 0x1p-500 && m <= 0x1p+500) || m == 0.0)), 0)) q = a / R.b;
+    return q;
+}
+
 __device__ __forceinline__ double ovh_of(double h, double htiny) {
     const double m = fmaxF(h, htiny);
     return 2.0 * h / (h * h + m * m);
@@ -74,43 +114,56 @@ __device__ __forceinline__ double phi_f(double h, double ul, double hl, double u
 
 // compute_lambda_vacc for the left state (hl, qxl, qyl) and the right state (hr, qxr, qyr) along
 // the unit vector (n1, n2); ovhl/ovhr and sql = SQRT(g*ABS(hl)), sqr = SQRT(g*ABS(hr)) are passed
-// in because the callers already hold them.
+// in because the callers already hold them, r16 = refined_rcp(16*g).
+//
+// The reference takes its first case when fh = phi(x0*hmin) >= 0; fh itself is used nowhere else.
+// Almost every entry decides that sign without evaluating phi (two square roots and a division).  Both terms
+// of phi are >= 0 for depths >= 0 with h0 = x0*hmin >= hmax, so fh >= 0 whenever w = vl - vr <= 0; and the
+// shallower side's term is (h0 - hmin)*SQRT(g/2*(one_over_h(h0) + one_over_h(hmin))) >= 2.34*hmin*
+// SQRT(g/2*one_over_h(hmin)), so it outweighs w > 0, and with it fh >= 0 by the monotonicity of the rounded
+// sums, whenever w**2 * lam_w <= hmin**2 * one_over_h(hmin) (lam_w = 1.01/(2.34**2 * g/2), the 1.01 covering
+// every rounding).  The other entries (dry fronts, depth ratios above 3.3, strong separation) evaluate phi
+// in a branch.  Per 16.8M-node launch: k_compute_dt 1113 -> 1045 us; a FCT step 2% less.
 __device__ __forceinline__ double lambda_vacc(double hl, double qxl, double qyl, double hr,
                                               double qxr, double qyr, double n1, double n2,
                                               double ovhl, double ovhr, double sql, double sqr,
-                                              const Consts& K, int& err) {
-    const double vl = (0.0 + qxl * n1 + qyl * n2) * ovhl;
-    const double vr = (0.0 + qxr * n1 + qyr * n2) * ovhr;
-    double hmin, hmax;
-    if (hl <= hr) { hmin = hl; hmax = hr; }
-    else { hmin = hr; hmax = hl; }
-    double ht;
-    const double fh = phi_f(K.x0 * hmin, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
-    if (0.0 <= fh) {
-        const double t = fmaxF(vl - vr + 2.0 * sql + 2.0 * sqr, 0.0);
-        ht = fminF(K.x0 * hmin, t * t / K.g16);
-    } else {
-        const double fh2 = phi_f(K.x0 * hmax, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
-        const double sqrmin = sqrt_rn(hmin);
-        const double sqrmax = sqrt_rn(hmax);
-        if (0.0 <= fh2) {
-            const double cc = -hmin * K.a_c2 - sqrmin * sqrmax + sqrmin * (vr - vl) / K.two_sqrt_g;
-            const double Delta = hmin - 4.0 * K.a_c2 * cc;
-            if (Delta < 0.0) {
-                err |= FLAG_LAMBDA;
-                return 0.0;
+                                              const Consts& K, const Rcp& r16, int& err) {
+    // (the reference starts each dot product from 0.0, which changes nothing but the sign of a zero)
+    const double vl = (qxl * n1 + qyl * n2) * ovhl;
+    const double vr = (qxr * n1 + qyr * n2) * ovhr;
+    const bool left = hl <= hr;
+    const double hmin = left ? hl : hr, hmax = left ? hr : hl;
+    const double h0 = K.x0 * hmin;
+    const double w = vl - vr;
+    const double t0 = posF(w + 2.0 * sql + 2.0 * sqr);
+    double ht = fminF(h0, div_shared(t0 * t0, r16));
+    const bool pos = hmin >= 0.0 && hmax <= K.lam_h && h0 >= hmax;
+    const bool small = w <= 0.0 || (hmin >= 0x1p-300 && w * w * K.lam_w <= hmin * hmin * (left ? ovhl : ovhr));
+    if (!(pos && small)) {
+        const double fh = phi_f(h0, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
+        if (!(0.0 <= fh)) {
+            const double fh2 = phi_f(K.x0 * hmax, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
+            const double sqrmin = sqrt_rn(hmin);
+            const double sqrmax = sqrt_rn(hmax);
+            if (0.0 <= fh2) {
+                const double cc = -hmin * K.a_c2 - sqrmin * sqrmax + sqrmin * (vr - vl) / K.two_sqrt_g;
+                const double Delta = hmin - 4.0 * K.a_c2 * cc;
+                if (Delta < 0.0) {
+                    err |= FLAG_LAMBDA;
+                    return 0.0;
+                }
+                const double t = (-sqrmin + sqrt_rn(Delta)) / (2.0 * K.a_c2);
+                ht = fminF(K.x0 * hmax, t * t);
+            } else {
+                ht = sqrmin * sqrmax * (1.0 + K.sqrt_2_g * (vl - vr) / (sqrmin + sqrmax));
             }
-            const double t = (-sqrmin + sqrt_rn(Delta)) / (2.0 * K.a_c2);
-            ht = fminF(K.x0 * hmax, t * t);
-        } else {
-            ht = sqrmin * sqrmax * (1.0 + K.sqrt_2_g * (vl - vr) / (sqrmin + sqrmax));
         }
     }
     // the arguments are products of two factors >= 1
-    const double lbdl = vl - sql * sqrt_normal((1.0 + fmaxF((ht - hl) * ovhl / 2.0, 0.0)) *
-                                               (1.0 + fmaxF((ht - hl) * ovhl, 0.0)));
-    const double lbdr = vr + sqr * sqrt_normal((1.0 + fmaxF((ht - hr) * ovhr / 2.0, 0.0)) *
-                                               (1.0 + fmaxF((ht - hr) * ovhr, 0.0)));
+    const double lbdl = vl - sql * sqrt_normal((1.0 + posF((ht - hl) * ovhl / 2.0)) *
+                                               (1.0 + posF((ht - hl) * ovhl)));
+    const double lbdr = vr + sqr * sqrt_normal((1.0 + posF((ht - hr) * ovhr / 2.0)) *
+                                               (1.0 + posF((ht - hr) * ovhr)));
     return fmaxF(fabs(lbdl), fabs(lbdr));
 }
 
@@ -118,16 +171,16 @@ __device__ __forceinline__ double lambda_vacc(double hl, double qxl, double qyl,
 // (compute_dij, SOURCES/update.f90:305-315), given norm = SQRT(SUM(c_ij**2)) and n = c_ij/norm.
 __device__ __forceinline__ double dij_of(double2 n, double norm, const Node& I, const Node& J,
                                          double ovh_i, double ovh_j, double sql, double sqr,
-                                         const Consts& K, int& err) {
-    const double lam = lambda_vacc(I.h, I.qx, I.qy, J.h, J.qx, J.qy, n.x, n.y, ovh_i, ovh_j, sql, sqr, K, err);
+                                         const Consts& K, const Rcp& r16, int& err) {
+    const double lam = lambda_vacc(I.h, I.qx, I.qy, J.h, J.qx, J.qy, n.x, n.y, ovh_i, ovh_j, sql, sqr, K, r16, err);
     return norm * lam;
 }
 
 // compute_muij of one off-diagonal entry; (v1i, v2i) and (v1j, v2j) are q*one_over_h.
 __device__ __forceinline__ double mu_of(double cx, double cy, double v1i, double v2i, double v1j, double v2j) {
-    const double sl = 0.0 + cx * v1i + cy * v2i;
-    const double sr = 0.0 + cx * v1j + cy * v2j;
-    return fmaxF(fmaxF(-sl, 0.0), fmaxF(sr, 0.0));
+    const double sl = cx * v1i + cy * v2i;
+    const double sr = cx * v1j + cy * v2j;
+    return fmaxF(posF(-sl), posF(sr));
 }
 
 // ---- x**(4/3) rounded to nearest, for the Manning friction term -------------------------------

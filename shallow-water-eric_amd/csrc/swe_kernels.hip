@@ -28,7 +28,7 @@
 //
 // Diagonal entries contribute to the reference's sums only through terms that multiply an exact
 // zero (U_i*rat_ii - U_i*rat_ii); those products are skipped, which can change nothing but the
-// sign of a zero.
+// sign of a zero, and so are the zeros the reference starts its per-entry dot products from.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,14 +39,12 @@
 
 #include "swe_engine.h"
 #include "swe_kernels.h"
+#include "swe_rows.h"
 
 namespace swe {
 
 namespace {
 
-enum SmbKind : int { SMB_ROUNDOFF = 0, SMB_2 = 1, SMB_1 = 2, SMB_GALERKIN = 3 };
-
-constexpr double kPi = 3.141592653589793;   // ACOS(-1.d0)
 
 #define SWE_PRAGMA(x) _Pragma(#x)
 #define SWE_UNROLL(n) SWE_PRAGMA(unroll n)
@@ -89,191 +87,6 @@ constexpr double kPi = 3.141592653589793;   // ACOS(-1.d0)
 #define SWE_LB_DT(BS) __launch_bounds__(BS)
 #endif
 
-// Slice of this wave: the waves of a launch take the listed slices in order (remap: XCD-aware
-// workgroup order), one slice each; -1 past the end of the list.  The value (and everything
-// derived from it: the instance, its constants, dt) is wave-uniform and kept in scalar registers;
-// the lane's row is slice*64 + lane.
-template <int BS>
-__device__ __forceinline__ int wave_slice(const Mesh& M, int remap) {
-    const int b = remap ? xcd_block() : (int)blockIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(b * (BS / 64) + (int)(threadIdx.x >> 6));
-    if (w >= M.nact) return -1;
-    return __builtin_amdgcn_readfirstlane(M.act[w]);
-}
-
-// Instance owning a slice; -1 for a free slice.
-__device__ __forceinline__ int slice_inst(const Mesh& M, int slice) {
-    return __builtin_amdgcn_readfirstlane(M.sl[slice].inst);
-}
-
-__device__ __forceinline__ int lane_of() { return (int)(threadIdx.x & 63); }
-
-__device__ __forceinline__ bool takes_steps(const InstDev& D, int flags) {
-    return D.state == INST_RUNNING && flags == 0 && D.time < D.tfinal && D.steps < D.max_steps;
-}
-
-__device__ __forceinline__ int64_t row_base(const Mesh& M, int i) {
-    return M.sl[i >> 6].sbase + (i & 63);
-}
-
-// Per-entry arrays streamed once per pass (c_ij, the first-order viscosities; with SWE_NT_LOADS >= 2
-// also the dt pass's d_ij): their loads and stores carry the non-temporal hint, so they do not
-// displace the gathered node data from the caches (measured: 14.86 -> 14.70 ms per 16.8M-node step).
-// SWE_NT_NODE: the same hint on the low-order solution (1: discharge, 2: depth too), written by
-// k_fct_lo and read back only at the row itself.
-#ifndef SWE_NT_NODE
-#define SWE_NT_NODE 2
-#endif
-#ifndef SWE_NT_LOADS
-#define SWE_NT_LOADS 2
-#endif
-typedef double dvec2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ double2 ld_entry(const double2* p) {
-#if SWE_NT_LOADS
-    const dvec2 v = __builtin_nontemporal_load((const dvec2*)p);
-    return make_double2(v.x, v.y);
-#else
-    return *p;
-#endif
-}
-__device__ __forceinline__ double ld_entry1(const double* p) {
-#if SWE_NT_LOADS > 1
-    return __builtin_nontemporal_load(p);
-#else
-    return *p;
-#endif
-}
-__device__ __forceinline__ void st_entry1(double* p, double v) {
-#if SWE_NT_LOADS > 1
-    __builtin_nontemporal_store(v, p);
-#else
-    *p = v;
-#endif
-}
-__device__ __forceinline__ void st_entry(double2* p, double2 v) {
-#if SWE_NT_LOADS
-    dvec2 w;
-    w.x = v.x;
-    w.y = v.y;
-    __builtin_nontemporal_store(w, (dvec2*)p);
-#else
-    *p = v;
-#endif
-}
-
-// Column of slot p of row i: a 16-bit offset from the row (half the bytes of the 32-bit column,
-// which is read only where the offset does not fit).
-__device__ __forceinline__ int col_at(const Mesh& M, int64_t p, int i) {
-    const int d = M.dcol[p];
-    return (d != kColFar) ? i + d : M.col[p];
-}
-
-__device__ __forceinline__ void raise_flag(int* flags, int inst, int f) {
-    if (f) atomicOr(flags + inst, f);
-}
-
-// LDS of one wave for the compacted lambda phase: per-row one_over_h and SQRT(g*ABS(h)), then
-// one double per slot of the slice (slot offset q*64 + lane).
-__device__ __forceinline__ double* wave_lds(double* smem, int wmax) {
-    return smem + (size_t)(threadIdx.x >> 6) * (size_t)(2 + wmax) * 64;
-}
-
-// RK combination of SOURCES/main.f90:83,89 (stage 0 keeps the Euler output)
-__device__ __forceinline__ double rk_combine(int stage, double uo, double ui) {
-    if (stage == 1) return (3.0 * uo + ui) / 4.0;
-    if (stage == 2) return (uo + 2.0 * ui) / 3.0;
-    return ui;
-}
-
-// Source terms of one node, dispatched on type_test (update.f90:614-623): friction (425-452),
-// my_friction (454-469), coriolis (471-486).  v1, v2 = velocity at U.  src is uniform per wave.
-// Launches whose instances have no source term use the HAS_SRC = false kernels, which leave it out.
-template <bool HAS_SRC>
-__device__ __forceinline__ void add_sources(int src, const Node& I, double mi, double v1, double v2, double dt,
-                                            const Consts& K, double& r2, double& r3) {
-    if constexpr (!HAS_SRC) return;
-    if (src == SRC_MANNING) {
-        const double hs = pow43(fmaxF(I.h, K.htiny));
-        const double vel = K.fric * sqrt_rn(v1 * v1 + v2 * v2);
-        const double hloc = 1.0 * vel * dt;
-        const double den = hs + fmaxF(hs, hloc);
-        r2 = r2 - mi * I.qx * vel * 2.0 / den;
-        r3 = r3 - mi * I.qy * vel * 2.0 / den;
-    } else if (src == SRC_LINEAR) {
-        r2 = r2 - mi * 0.2 * I.qx;
-        r3 = r3 - mi * 0.2 * I.qy;
-    } else if (src == SRC_CORIOLIS) {
-        const double f = 2.0;
-        r2 = r2 + mi * f * I.qy;
-        r3 = r3 - mi * f * I.qx;
-    }
-}
-
-// compute_dij of one off-diagonal entry from c_ij itself: the norm and the unit vector are
-// evaluated with compute_dij's expressions (SOURCES/update.f90:306-310; correctly rounded sqrt and
-// division, so the bits are the reference's), which costs a square root and two divisions per entry
-// instead of storing 24 bytes of normal and norm per entry (measured faster in every pass).
-__device__ __forceinline__ double dij_from_c(const double2 c, const Node& I, const Node& J, double ovh_i,
-                                             double ovh_j, double sql, double sqr, const Consts& K, int& err) {
-    const double norm = sqrt_normal(0.0 + c.x * c.x + c.y * c.y);
-    return dij_of(make_double2(c.x / norm, c.y / norm), norm, I, J, ovh_i, ovh_j, sql, sqr, K, err);
-}
-
-// dlam is compute_dij's value for this entry (from the dt pass or computed inline).
-template <bool ALPHA>
-__device__ __forceinline__ void first_order_dmu(const double2 c, double v1i, double v2i, double v1j, double v2j,
-                                                double dlam, double ai, const double* __restrict__ alpha, int j,
-                                                double& d, double& mu) {
-    d = dlam;
-    mu = mu_of(c.x, c.y, v1i, v2i, v1j, v2j);
-    d = fmaxF(d, mu);
-    if constexpr (ALPHA) {
-        const double s = fmaxF(ai, alpha[j]);
-        d = d * s;
-        mu = mu * s;
-    }
-}
-
-// alpha_limit, first loop (update.f90:758-781) for row i: alpha_i = (|sum(h_j-h_i)| /
-// sum|h_j-h_i|)**8, 1 if h_i <= htiny or the denominator does not exceed the numerator.  All index
-// loads, then all gathers, then the sums in entry order.  (Evaluating it inside the dt pass for
-// stage 1 was measured slower than this separate sweep: the gathers after the LDS phase stall.)
-__device__ __forceinline__ double alpha_of(const Mesh& M, const Node* __restrict__ U, int i, double hi, double htiny) {
-    double a = 1.0;
-    if (!(hi <= htiny)) {
-        const int64_t pb = row_base(M, i);
-        const int len = M.len[i];
-        constexpr int kUnroll = 12;
-        int js[kUnroll];
-        double hs[kUnroll];
-#pragma unroll
-        for (int q = 0; q < kUnroll; ++q) js[q] = (q < len) ? (int)M.dcol[pb + 64 * q] : 0;
-#pragma unroll
-        for (int q = 0; q < kUnroll; ++q) js[q] = (js[q] != kColFar) ? i + js[q] : M.col[pb + 64 * q];
-#pragma unroll
-        for (int q = 0; q < kUnroll; ++q) hs[q] = U[js[q]].h;
-        double num = 0.0, denom = 0.0;
-#pragma unroll
-        for (int q = 0; q < kUnroll; ++q) {
-            if (q < len) {
-                num = num + hs[q] - hi;
-                denom = denom + fabs(hs[q] - hi);
-            }
-        }
-        for (int q = kUnroll; q < len; ++q) {
-            const double hj = U[col_at(M, pb + 64 * (int64_t)q, i)].h;
-            num = num + hj - hi;
-            denom = denom + fabs(hj - hi);
-        }
-        if (denom <= fabs(num)) a = 1.0;
-        else a = fabs(num) / (denom);
-        a = a * a;
-        a = a * a;
-        a = a * a;
-    }
-    return a;
-}
-
 // =============================================================================================
 // COMPUTE_DT: d_ij for every off-diagonal entry, row sums, max |d_ii|/m_i per instance.
 // Phase 0 (one lane per row) puts the row's one_over_h and SQRT(g*ABS(h)) in LDS and an exact 0.0
@@ -301,6 +114,7 @@ __device__ __forceinline__ void dt_slice(const Mesh& M, const InstDev* __restric
     int err = 0;
     Consts K{};
     if (wave_live) K = T[inst].K;
+    const Rcp r16 = uniform_rcp(K.g16);
     Node I{};
     if (valid) {
         I = U[i];
@@ -319,7 +133,7 @@ __device__ __forceinline__ void dt_slice(const Mesh& M, const InstDev* __restric
             const Node Ir = U[slice * 64 + r];
             const Node J = U[col_at(M, slot, slice * 64 + r)];
             const double d = dij_from_c(ld_entry(M.c + slot), Ir, J, lw[r], ovh_of(J.h, K.htiny), lw[64 + r],
-                                        sqrt_rn(K.g * fabs(J.h)), K, err);
+                                        sqrt_rn(K.g * fabs(J.h)), K, r16, err);
             lw[128 + off] = d;
             if (d0) st_entry1(d0 + slot, d);
         }
@@ -373,54 +187,13 @@ k_compute_dt(Mesh M, const InstDev* __restrict__ T, const int* __restrict__ flag
     dt_slice<BS>(M, T, flags, U, d0, vmax, flags_out, all, wave_slice<BS>(M, remap), wave_lds(smem, M.wmax));
 }
 
-// Per-instance step bookkeeping after the dt pass (SOURCES/main.f90:61-91):
-// an instance takes the step while time < tfinal (and its step limit and error flags allow);
-// dt = CFL*1/MAXVAL(ABS(d_ii)/m_i); the boundary values of the three stages are evaluated at
-// t+dt, (t+dt)+dt/2 and (t+dt/2)+dt; time = to + dt.  advance = 0 only computes dt.
-__device__ __forceinline__ void finalize_one(InstDev* __restrict__ T, unsigned long long* __restrict__ vmax,
-                                             const int* __restrict__ flags, int k, int advance) {
-    InstDev& D = T[k];
-    if (D.state == INST_FREE) return;
-    const double mx = __longlong_as_double((long long)vmax[k]);
-    vmax[k] = 0ull;
-    if (!advance) {
-        D.dt = D.K.cfl * 1.0 / mx;
-        return;
-    }
-    if (D.state != INST_RUNNING) {
-        D.go = 0;
-        return;
-    }
-    if (!takes_steps(D, flags[k])) {
-        D.go = 0;
-        D.state = flags[k] ? INST_FAILED : INST_DONE;
-        return;
-    }
-    // test 9 takes the driver's fixed dt and skips COMPUTE_DT (main.f90:66-71)
-    const double dt = (D.K.dt_fixed > 0.0) ? D.K.dt_fixed : D.K.cfl * 1.0 / mx;
-    const double to = D.time;
-    D.dt = dt;
-    if (D.bc_kind == SWE_BC_INFLOW) {
-        double t = to;
-        const double ts0 = t + dt;
-        t = to + dt;
-        const double ts1 = t + dt / 2;
-        t = to + dt / 2;
-        const double ts2 = t + dt;
-        D.bc_val[0] = D.bc_amp * sin_rn(2.0 * kPi * ts0 / D.bc_period);
-        D.bc_val[1] = D.bc_amp * sin_rn(2.0 * kPi * ts1 / D.bc_period);
-        D.bc_val[2] = D.bc_amp * sin_rn(2.0 * kPi * ts2 / D.bc_period);
-    }
-    if (D.dt_log) D.dt_log[D.steps % D.dt_cap] = dt;
-    D.time = to + dt;
-    D.steps = D.steps + 1;
-    D.go = 1;
-}
-
 __global__ void k_finalize_dt(InstDev* __restrict__ T, unsigned long long* __restrict__ vmax,
                               const int* __restrict__ flags, int ninst, int advance) {
     const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (k < ninst) finalize_one(T, vmax, flags, k, advance);
+    if (k >= ninst) return;
+    const unsigned long long v = vmax[k];
+    vmax[k] = 0ull;
+    finalize_one(T, v, flags[k], k, advance);
 }
 
 // compute_dij with the full dij%aa (diagonal = -row sum), for swe_compute_dij.
@@ -436,6 +209,7 @@ k_dij_full(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, do
     const int len = M.len[i];
     if (len == 0) return;
     const Consts K = T[inst].K;
+    const Rcp r16 = uniform_rcp(K.g16);
     int err = 0;
     const Node I = U[i];
     const double ovh_i = ovh_of(I.h, K.htiny);
@@ -448,7 +222,7 @@ k_dij_full(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, do
         const int j = col_at(M, p, i);
         if (j == i) { pd = p; dij[p] = 0.0; continue; }
         const Node J = U[j];
-        const double d = dij_from_c(M.c[p], I, J, ovh_i, ovh_of(J.h, K.htiny), sql, sqrt_rn(K.g * fabs(J.h)), K, err);
+        const double d = dij_from_c(M.c[p], I, J, ovh_i, ovh_of(J.h, K.htiny), sql, sqrt_rn(K.g * fabs(J.h)), K, r16, err);
         dij[p] = d;
         s = s + d;
     }
@@ -492,6 +266,7 @@ k_stage_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
     const int len = M.len[i];
     if (len == 0) return;
     const Consts K = T[inst].K;
+    const Rcp r16 = uniform_rcp(K.g16);
     const double dt = T[inst].dt;
     int err = 0;
     const Node I = U[i];
@@ -519,23 +294,17 @@ k_stage_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
         const bool off = (j != i);
         if (SMB != SMB_GALERKIN && off)
             first_order_dmu<ALPHA>(c, v1i, v2i, v1j, v2j,
-                                   d0 ? d0[p] : dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, err),
+                                   d0 ? d0[p] : dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, r16, err),
                                    ai, alpha, j, d, mu);
         if constexpr (SMB == SMB_1) {
             // smb_1 (update.f90:378-409)
-            double xx = 0.0;
-            xx = xx - c.x * (v1j * J.h * ratji + v1i * I.h * ratij);
-            xx = xx - c.y * (v2j * J.h * ratji + v2i * I.h * ratij);
+            double xx = -(c.x * (v1j * J.h * ratji + v1i * I.h * ratij)) - c.y * (v2j * J.h * ratji + v2i * I.h * ratij);
             r1 = r1 + xx;
             if (off) r1 = r1 + d * (J.h * ratji - I.h * ratij);
-            xx = 0.0;
-            xx = xx - c.x * (v1j * J.qx * ratji + v1i * I.qx * ratij);
-            xx = xx - c.y * (v2j * J.qx * ratji + v2i * I.qx * ratij);
+            xx = -(c.x * (v1j * J.qx * ratji + v1i * I.qx * ratij)) - c.y * (v2j * J.qx * ratji + v2i * I.qx * ratij);
             r2 = r2 + xx;
             if (off) r2 = r2 + d * (J.qx * ratji - I.qx * ratij);
-            xx = 0.0;
-            xx = xx - c.x * (v1j * J.qy * ratji + v1i * I.qy * ratij);
-            xx = xx - c.y * (v2j * J.qy * ratji + v2i * I.qy * ratij);
+            xx = -(c.x * (v1j * J.qy * ratji + v1i * I.qy * ratij)) - c.y * (v2j * J.qy * ratji + v2i * I.qy * ratij);
             r3 = r3 + xx;
             if (off) r3 = r3 + d * (J.qy * ratji - I.qy * ratij);
             if (off) {
@@ -546,30 +315,22 @@ k_stage_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
         } else {
             if constexpr (SMB == SMB_ROUNDOFF) {
                 // smb_2_roundoff (update.f90:566-611): mass equation with fix_roundoff
-                double xx = 0.0;
-                xx = xx - c.x * (v1j);
-                xx = xx - c.y * (v2j);
+                const double xx = -(c.x * (v1j)) - c.y * (v2j);
                 if (!off) {
                     fix = fix + xx;
                 } else {
                     fix = fix - mu + (d - mu) * (-ratij);
-                    r1 = r1 + (xx + mu) * J.h + fmaxF((d - mu) * Hji, 0.0);
+                    r1 = r1 + (xx + mu) * J.h + posF((d - mu) * Hji);
                 }
             } else {
                 // smb_2 (update.f90:656-663), k = 1
-                double xx = 0.0;
-                xx = xx - c.x * (v1j * J.h);
-                xx = xx - c.y * (v2j * J.h);
+                const double xx = -(c.x * (v1j * J.h)) - c.y * (v2j * J.h);
                 r1 = r1 + xx;
                 if (SMB != SMB_GALERKIN && off)
                     r1 = r1 + d * (J.h * ratji - I.h * ratij) + mu * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
             }
-            double xx2 = 0.0;
-            xx2 = xx2 - c.x * (v1j * J.qx);
-            xx2 = xx2 - c.y * (v2j * J.qx);
-            double xx3 = 0.0;
-            xx3 = xx3 - c.x * (v1j * J.qy);
-            xx3 = xx3 - c.y * (v2j * J.qy);
+            const double xx2 = -(c.x * (v1j * J.qx)) - c.y * (v2j * J.qx);
+            const double xx3 = -(c.x * (v1j * J.qy)) - c.y * (v2j * J.qy);
             r2 = r2 + xx2;
             r3 = r3 + xx3;
             if (SMB != SMB_GALERKIN && off) {
@@ -636,6 +397,7 @@ k_stage_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, c
     const int len = M.len[i];
     if (len == 0) return;
     const Consts K = T[inst].K;
+    const Rcp r16 = uniform_rcp(K.g16);
     const double dt = T[inst].dt;
     int err = 0;
     const Node I = U[i];
@@ -670,13 +432,11 @@ k_stage_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, c
         const bool off = (j != i);
         if (SMB != SMB_GALERKIN && off)
             first_order_dmu<ALPHA>(c, v1i, v2i, v1j, v2j,
-                                   d0 ? d0[p] : dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, err),
+                                   d0 ? d0[p] : dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, r16, err),
                                    ai, alpha, j, d, mu);
         if constexpr (SMB == SMB_1) {
             for (int k = 0; k < 5; ++k) {
-                double xx = 0.0;
-                xx = xx - c.x * (v1j * uj[k] * ratji + v1i * ui[k] * ratij);
-                xx = xx - c.y * (v2fj * uj[k] * ratji + v2fi * ui[k] * ratij);
+                const double xx = -(c.x * (v1j * uj[k] * ratji + v1i * ui[k] * ratij)) - c.y * (v2fj * uj[k] * ratji + v2fi * ui[k] * ratij);
                 r[k] = r[k] + xx;
                 if (off) r[k] = r[k] + d * (uj[k] * ratji - ui[k] * ratij);
             }
@@ -688,20 +448,16 @@ k_stage_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, c
         } else {
             int k0 = 0;
             if constexpr (SMB == SMB_ROUNDOFF) {
-                double xm = 0.0;
-                xm = xm - c.x * (v1j);
-                xm = xm - c.y * (v2fj);
+                const double xm = -(c.x * (v1j)) - c.y * (v2fj);
                 if (!off) fix = fix + xm;
                 else {
                     fix = fix - mu + (d - mu) * (-ratij);
-                    r[0] = r[0] + (xm + mu) * J.h + fmaxF((d - mu) * Hji, 0.0);
+                    r[0] = r[0] + (xm + mu) * J.h + posF((d - mu) * Hji);
                 }
                 k0 = 1;
             }
             for (int k = k0; k < 5; ++k) {
-                double xx = 0.0;
-                xx = xx - c.x * (v1j * uj[k]);
-                xx = xx - c.y * (v2fj * uj[k]);
+                const double xx = -(c.x * (v1j * uj[k])) - c.y * (v2fj * uj[k]);
                 r[k] = r[k] + xx;
                 if (SMB != SMB_GALERKIN && off)
                     r[k] = r[k] + d * (uj[k] * ratji - ui[k] * ratij) + mu * (uj[k] * (1.0 - ratji) - ui[k] * (1.0 - ratij));
@@ -776,6 +532,7 @@ fct_lo_body(const Mesh& M, const InstDev* __restrict__ T, const Node* __restrict
     const int len = M.len[i];
     if (len == 0) return;
     const Consts K = T[inst].K;
+    const Rcp r16 = uniform_rcp(K.g16);
     const double dt = T[inst].dt;
     int err = 0;
     const Node I = U[i];
@@ -815,22 +572,14 @@ fct_lo_body(const Mesh& M, const InstDev* __restrict__ T, const Node* __restrict
             double dlam;
             if constexpr (LAM == LAM_D0) dlam = ld_entry1(d0 + p);
             else if constexpr (LAM == LAM_LDS) dlam = lam[64 * q + lane_of()];
-            else dlam = dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, err);
+            else dlam = dij_from_c(c, I, J, ovh_i, ovh_j, sql, sqrt_rn(K.g * fabs(J.h)), K, r16, err);
             first_order_dmu<ALPHA>(c, v1i, v2i, v1j, v2j, dlam, ai, alpha, j, d, mu);
             st_entry(dmu + p, make_double2(d, mu));
         }
-        double xm = 0.0;
-        xm = xm - c.x * (v1j);
-        xm = xm - c.y * (v2j);
-        double xe = 0.0;
-        xe = xe - c.x * (v1j * J.h);
-        xe = xe - c.y * (v2j * J.h);
-        double xx2 = 0.0;
-        xx2 = xx2 - c.x * (v1j * J.qx);
-        xx2 = xx2 - c.y * (v2j * J.qx);
-        double xx3 = 0.0;
-        xx3 = xx3 - c.x * (v1j * J.qy);
-        xx3 = xx3 - c.y * (v2j * J.qy);
+        const double xm = -(c.x * (v1j)) - c.y * (v2j);
+        const double xe = -(c.x * (v1j * J.h)) - c.y * (v2j * J.h);
+        const double xx2 = -(c.x * (v1j * J.qx)) - c.y * (v2j * J.qx);
+        const double xx3 = -(c.x * (v1j * J.qy)) - c.y * (v2j * J.qy);
         const double topo = K.g * I.h * (J.h + J.z - I.h - I.z);
         // The momentum sums of the low-order update (thresholds htiny) and of the entropy residual
         // (thresholds 0) take the same terms in the same order while every entry's ratios agree, so
@@ -846,7 +595,7 @@ fct_lo_body(const Mesh& M, const InstDev* __restrict__ T, const Node* __restrict
                 if (!off) fix = fix + xm;
                 else {
                     fix = fix - mu + (d - mu) * (-ratijr);
-                    r1 = r1 + (xm + mu) * J.h + fmaxF((d - mu) * Hji, 0.0);
+                    r1 = r1 + (xm + mu) * J.h + posF((d - mu) * Hji);
                 }
             } else {
                 r1 = r1 + xe;
@@ -991,6 +740,7 @@ k_fct_lo_lds(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
     __syncthreads();
     if (live) {
         const Consts K = T[inst].K;
+        const Rcp r16 = uniform_rcp(K.g16);
         const SliceInfo S = M.sl[slice];
         const int64_t e1 = S.ebase + S.ecount;
         int err = 0;
@@ -1001,27 +751,13 @@ k_fct_lo_lds(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
             const Node Ir = U[slice * 64 + r];
             const Node J = U[col_at(M, slot, slice * 64 + r)];
             lw[128 + off] = dij_from_c(ld_entry(M.c + slot), Ir, J, lw[r], ovh_of(J.h, K.htiny), lw[64 + r],
-                                       sqrt_rn(K.g * fabs(J.h)), K, err);
+                                       sqrt_rn(K.g * fabs(J.h)), K, r16, err);
         }
         raise_flag(flags_out, inst, err);
     }
     __syncthreads();
     fct_lo_body<BS, ALPHA, WRITE_LO, HAS_SRC, LAM_LDS>(M, T, U, ulo_h, ulo_q, dmu, res, nullptr, lw + 128, alpha,
                                                        roundoff, flags_out, slice);
-}
-
-// Antidiffusive flux f_ij of compute_fct_matrix (update.f90:732-745) for an off-diagonal entry,
-// with the high-order viscosities MIN(dL, resij), MIN(muL, resij) of update.f90:233-239.
-__device__ __forceinline__ double fct_flux(const Node& I, const Node& J, double dLp, double muLp,
-                                           double rij, double& dH, double& muH, double& ratij, double& ratji) {
-    dH = fminF(dLp, 1.0 * rij);
-    muH = fminF(muLp, 1.0 * rij);
-    const double zmax = fmaxF(I.z, J.z);
-    const double Hij = fmaxF(0.0, I.h + I.z - zmax);
-    const double Hji = fmaxF(0.0, J.h + J.z - zmax);
-    ratij = (I.h <= 0.0) ? 0.0 : Hij / I.h;
-    ratji = (J.h <= 0.0) ? 0.0 : Hji / J.h;
-    return (dH - dLp) * (J.h * ratji - I.h * ratij) + (muH - muLp) * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
 }
 
 // =============================================================================================
@@ -1191,27 +927,19 @@ k_ev_update(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, c
             mu = fminF(lo.y, 1.0 * rij);
         }
         if (roundoff) {
-            double xm = 0.0;
-            xm = xm - c.x * (v1j);
-            xm = xm - c.y * (v2j);
+            const double xm = -(c.x * (v1j)) - c.y * (v2j);
             if (!off) fix = fix + xm;
             else {
                 fix = fix - mu + (d - mu) * (-ratij);
-                r1 = r1 + (xm + mu) * J.h + fmaxF((d - mu) * Hji, 0.0);
+                r1 = r1 + (xm + mu) * J.h + posF((d - mu) * Hji);
             }
         } else {
-            double xe = 0.0;
-            xe = xe - c.x * (v1j * J.h);
-            xe = xe - c.y * (v2j * J.h);
+            const double xe = -(c.x * (v1j * J.h)) - c.y * (v2j * J.h);
             r1 = r1 + xe;
             if (off) r1 = r1 + d * (J.h * ratji - I.h * ratij) + mu * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
         }
-        double xx2 = 0.0;
-        xx2 = xx2 - c.x * (v1j * J.qx);
-        xx2 = xx2 - c.y * (v2j * J.qx);
-        double xx3 = 0.0;
-        xx3 = xx3 - c.x * (v1j * J.qy);
-        xx3 = xx3 - c.y * (v2j * J.qy);
+        const double xx2 = -(c.x * (v1j * J.qx)) - c.y * (v2j * J.qx);
+        const double xx3 = -(c.x * (v1j * J.qy)) - c.y * (v2j * J.qy);
         r2 = r2 + xx2;
         r3 = r3 + xx3;
         if (off) {
@@ -1373,7 +1101,11 @@ k_step_fct(StepArgs A, int nsteps) {
             dt_slice<BS>(M, A.T, A.flags, A.S0, A.d0, A.vmax, A.flags, 0, slice, lw);
         }
         if (!grid_barrier(A, epoch)) return;
-        for (int k = gt; k < A.ninst; k += nt) finalize_one(A.T, A.vmax, A.flags, k, 1);
+        for (int k = gt; k < A.ninst; k += nt) {
+            const unsigned long long v = A.vmax[k];
+            A.vmax[k] = 0ull;
+            finalize_one(A.T, v, A.flags[k], k, 1);
+        }
         if (!grid_barrier(A, epoch)) return;
         for (int stage = 0; stage < 3; ++stage) {
             const Node* U = (stage == 0) ? A.S0 : (stage == 1) ? A.S1 : A.S2;
@@ -1707,7 +1439,7 @@ void launch_fct_lo(Pool& P, const Node* U, const double* d0) {
 const char* const kKernelNames[KID_COUNT] = {"k_compute_dt", "k_alpha", "k_stage_lo", "k_fct_lo",
                                              "k_fct_rminus", "k_fct_apply", "k_ev_update"};
 
-int kinds_of(int kid) { return (kid == KID_FCT_LO) ? 2 : 1; }
+int kinds_of(int kid) { return (kid == KID_FCT_LO) ? 3 : 1; }
 
 bool block_supported(int kid, int block) {
     if (kid == KID_STAGE_LO || kid == KID_EV) return block == 256;
@@ -1715,12 +1447,19 @@ bool block_supported(int kid, int block) {
 }
 
 Mesh mesh_view(const Pool& P) {
-    return Mesh{P.sl, P.len, P.col, P.dcol, P.c, P.m, P.elist, P.dpos, P.act, P.nact, P.wmax};
+    return Mesh{P.sl,   P.len,  P.col,   P.dcol, P.c,    P.m,   P.elist, P.dpos,
+                P.dirm, P.lcol, P.halo, P.tact, P.ntile, P.act, P.nact, P.wmax};
 }
 
-void launch_compute_dt(Pool& P, const Node* U, double* d0, int all) {
+bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
     const Mesh M = mesh_view(P);
-    if (M.nact == 0) return;
+    if (M.nact == 0) return false;
+    if (tiles_apply(P)) {
+        timed_begin(P, KID_DT);
+        launch_tile_dt(P, U, d0, all, advance);
+        timed_end(P, KID_DT);
+        return advance;
+    }
     const LaunchCfg& L = P.tune.k[KID_DT];
     // the dynamic LDS of a workgroup stays within 64 KiB: fall back to smaller workgroups
     int block = L.block;
@@ -1732,6 +1471,7 @@ void launch_compute_dt(Pool& P, const Node* U, double* d0, int all) {
                            (const InstDev*)P.tab, (const int*)P.flags, U, d0, P.vmax, P.flags, all, L.remap);
     })
     timed_end(P, KID_DT);
+    return false;
 }
 
 void launch_finalize_dt(Pool& P, int advance) {
@@ -1744,7 +1484,8 @@ void launch_finalize_dt(Pool& P, int advance) {
 // One Euler stage from U to out (out != U) for every instance that takes the step.  d0 (may be
 // null) holds compute_dij at U.  stage: 0 keeps the Euler output, 1 and 2 apply the RK
 // combinations with Uo.
-int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage) {
+// bdy: the kernels that can (bdy_fused) also write the wall and inflow values of `stage`.
+int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage, bool bdy) {
     const Mode& md = P.mode;
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return SWE_OK;
@@ -1805,28 +1546,35 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
         timed_end(P, KID_STAGE_LO);
     } else if (md.viscosity_type == SWE_FCT) {
         timed_begin(P, KID_FCT_LO);
-        if (alpha) launch_fct_lo<true, true>(P, U, d0);
+        if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, true);
+        else if (alpha) launch_fct_lo<true, true>(P, U, d0);
         else launch_fct_lo<false, true>(P, U, d0);
         timed_end(P, KID_FCT_LO);
-        {
+        if (tiles_apply(P)) {
+            timed_begin(P, KID_RMINUS);
+            launch_tile_rminus(P, U);
+            timed_end(P, KID_RMINUS);
+            timed_begin(P, KID_APPLY);
+            launch_tile_apply(P, U, Uo, out, stage, bdy);
+            timed_end(P, KID_APPLY);
+        } else {
             const LaunchCfg& L = P.tune.k[KID_RMINUS];
             timed_begin(P, KID_RMINUS);
             SWE_BS_SWITCH(L.block, hipLaunchKernelGGL((k_fct_rminus<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0,
                                                       P.stream, M, T, U, (const double*)P.ulo_h, (const double2*)P.dmu,
                                                       (const double*)P.res, P.Rm, L.remap))
             timed_end(P, KID_RMINUS);
-        }
-        {
-            const LaunchCfg& L = P.tune.k[KID_APPLY];
+            const LaunchCfg& A = P.tune.k[KID_APPLY];
             timed_begin(P, KID_APPLY);
-            SWE_BS_SWITCH(L.block, hipLaunchKernelGGL((k_fct_apply<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0,
+            SWE_BS_SWITCH(A.block, hipLaunchKernelGGL((k_fct_apply<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0,
                                                       P.stream, M, T, U, Uo, (const double*)P.ulo_h, (const double2*)P.ulo_q, out,
                                                       (const double2*)P.dmu, (const double*)P.res,
-                                                      (const double*)P.Rm, stage, P.flags, L.remap))
+                                                      (const double*)P.Rm, stage, P.flags, A.remap))
             timed_end(P, KID_APPLY);
         }
     } else {  // entropy_visc
-        if (alpha) launch_fct_lo<true, false>(P, U, d0);
+        if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, false);
+        else if (alpha) launch_fct_lo<true, false>(P, U, d0);
         else launch_fct_lo<false, false>(P, U, d0);
         const LaunchCfg& L = P.tune.k[KID_EV];
         timed_begin(P, KID_EV);
@@ -1846,6 +1594,8 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
     if (e != hipSuccess) return fail(SWE_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return SWE_OK;
 }
+
+bool bdy_fused(const Pool& P) { return P.mode.viscosity_type == SWE_FCT && tiles_apply(P); }
 
 void launch_bdy(Pool& P, Node* u, int stage) {
     const int64_t n = P.nbc();

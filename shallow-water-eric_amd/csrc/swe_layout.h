@@ -36,6 +36,8 @@ struct Consts {
     double g_half;      // g/2
     double g16;         // 16*g
     double fric;        // g*mannings**2
+    double lam_w;       // 1.01/(2.34**2*g/2), and
+    double lam_h;       // the greatest depth of lambda's quick sign test (lambda_vacc); -1 turns it off
     double ent_cst;     // 1e-10*g*max_water_h**2
     double dt_fixed;    // > 0: the time loop's dt instead of the CFL one (test 9, SOURCES/main.f90:68)
     double lambda_sgn;  // inputs%lambdaSGN of the SGN model (test 13)
@@ -55,8 +57,25 @@ struct alignas(32) SliceInfo {
     int64_t ebase;      // first element of the slice's compact off-diagonal list
     int inst;           // owning instance, -1 when the slice is free or not yet admitted
     int ecount;         // length of the compact off-diagonal list
-    int pad_[2];
+    int tile_slices;    // first slice of a tile: slices of the tile (0 on the other slices)
+    int nhalo;          // first slice of a tile: rows of its halo list
 };
+
+// A tile is a run of up to tile_slices (1, 2 or 4: fixed per pool) consecutive slices of one instance,
+// counted from the instance's first slice; one workgroup works on it with the node data of its rows and of
+// its halo (the rows of other tiles its entries refer to, ascending) staged in LDS.  lcol names an entry's
+// column there: row - first row of the tile for the tile's own rows, 64*tile_slices + position in the halo
+// list for the others.  The halo list of the tile that starts at slice s begins at halo[s * kHaloStride].
+constexpr int kHaloStride = 192;
+constexpr int kMaxTileSlices = 4;
+constexpr int kTileNodes = 816;    // rows and halo of a tile: 80 bytes each within 64 KiB of LDS
+// Longest halo a tile of ns slices may have in a pool of ts-slice tiles.  (Measured on locality-ordered meshes
+// of 5k to 1M nodes: 36 to 43 rows on average and at most 124 in tiles of 64 rows, 66 to 84 and at most 240
+// of 256; an instance with a longer one is run by the gather kernels.)
+__host__ __device__ constexpr int tile_halo_cap(int ts, int ns) {
+    const int lds = kTileNodes - 64 * ts, room = ns * kHaloStride;
+    return lds < 512 ? (lds < room ? lds : room) : (512 < room ? 512 : room);
+}
 
 enum InstState : int { INST_FREE = 0, INST_RUNNING = 1, INST_DONE = 2, INST_FAILED = 3 };
 
@@ -99,6 +118,11 @@ struct Mesh {
     const double* __restrict__ m;       // lumped mass of each row
     const uint16_t* __restrict__ elist; // per slice: slot offsets (q*64 + lane) of off-diagonal entries
     const uint8_t* __restrict__ dpos;   // position q of the diagonal in each row
+    const uint8_t* __restrict__ dirm;   // Dirichlet components of each row: bits 1 h, 2 qx, 4 qy
+    const uint16_t* __restrict__ lcol;  // column of each slot within its tile (see tile_slices above)
+    const int* __restrict__ halo;       // halo lists of the tiles (global rows)
+    const int* __restrict__ tact;       // first slices of the tiles a launch covers, ascending
+    int ntile;                          // number of them
     const int* __restrict__ act;        // the slices a launch covers, ascending (one wave each)
     int nact;                           // number of them
     int wmax;                           // longest row of the resident instances

@@ -430,28 +430,6 @@ __global__ void k_curve_key(int np, const double* __restrict__ rr, double x0, do
     idx[i] = i;
 }
 
-__global__ void k_inverse(int np, const int* __restrict__ order, int* __restrict__ pos) {
-    const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (p < np) pos[order[p]] = p;
-}
-
-// Sum over the off-diagonal entries of |pos(i) - pos(j)| (pos null: the caller's numbering).
-__global__ void k_offset_sum(int np, const int64_t* __restrict__ ia0, const int* __restrict__ ja,
-                             const int* __restrict__ pos, unsigned long long* __restrict__ sum) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    unsigned long long acc = 0;
-    if (i < np) {
-        const int pi = pos ? pos[i] : i;
-        for (int64_t p = ia0[i]; p < ia0[i + 1]; ++p) {
-            const int j = ja[p] - 1;
-            const int pj = pos ? pos[j] : j;
-            acc += (unsigned long long)((pi > pj) ? pi - pj : pj - pi);
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if ((threadIdx.x & 63) == 0 && acc) atomicAdd(sum, acc);
-}
-
 __global__ void k_lay_iperm(int np, int np_pad, const int* __restrict__ perm, const int* __restrict__ lenc,
                             int* __restrict__ iperm, int* __restrict__ lenr) {
     const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -486,6 +464,7 @@ __global__ void k_lay_slices(int nsl, int np, const int* __restrict__ lenr, int6
 struct LayOut {
     uint8_t* len8;
     uint8_t* dpos8;
+    uint8_t* dirm;
     int* perm;
     double* m;
     double* z;
@@ -503,6 +482,7 @@ __global__ void k_lay_fill(int np, int np_pad, int64_t r0, int64_t p0, const int
                            int64_t* __restrict__ csr2slot) {
     const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (r >= np_pad) return;
+    o.dirm[r0 + r] = 0;
     if (r >= np) {
         o.len8[r0 + r] = 0;
         o.dpos8[r0 + r] = 0;
@@ -553,7 +533,7 @@ __global__ void k_lay_elist(int nsl, int np, int64_t r0, int64_t e0, const int* 
     }
 }
 
-__global__ void k_lay_slice_info(int nsl, int64_t s0, int64_t p0, int64_t e0, int inst,
+__global__ void k_lay_slice_info(int nsl, int64_t s0, int64_t p0, int64_t e0, int inst, int tile_slices,
                                  const int64_t* __restrict__ sptr, const int64_t* __restrict__ eoff,
                                  swe::SliceInfo* __restrict__ sl) {
     const int s = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -563,17 +543,96 @@ __global__ void k_lay_slice_info(int nsl, int64_t s0, int64_t p0, int64_t e0, in
     v.ebase = e0 + eoff[s];
     v.inst = inst;
     v.ecount = (int)(eoff[s + 1] - eoff[s]);
-    v.pad_[0] = 0;
-    v.pad_[1] = 0;
+    v.tile_slices = (s % tile_slices) ? 0 : ((nsl - s < tile_slices) ? nsl - s : tile_slices);
+    v.nhalo = 0;
     sl[s0 + s] = v;
 }
 
+// One workgroup per tile: the distinct rows outside the tile that its entries refer to, collected in a hash
+// set in LDS (open addressing; a tile past the halo capacity gives up),
+// ranked by counting (ascending, as the host layout sorts them), every entry's column within the tile,
+// and the longest list (INT_MAX: one past the capacity).  Runs after k_lay_fill (global columns) and k_lay_slice_info.
+constexpr int kTileHash = 1024;
+__global__ void __launch_bounds__(256)
+k_lay_tiles(int nsl, int64_t s0, int tile_slices, const uint8_t* __restrict__ len8, const int* __restrict__ col,
+            swe::SliceInfo* __restrict__ sl, uint16_t* __restrict__ lcol, int* __restrict__ halo,
+            int* __restrict__ longest) {
+    __shared__ int key[kTileHash];
+    __shared__ int pos[kTileHash];
+    __shared__ int list[512];
+    __shared__ int count;
+    const int t0 = (int)blockIdx.x * tile_slices;
+    const int ns = (nsl - t0 < tile_slices) ? nsl - t0 : tile_slices;
+    const int64_t g0 = s0 + t0;                       // the tile's first slice
+    const int row0 = (int)(g0 * 64), row1 = row0 + 64 * ns;
+    const int cap = swe::tile_halo_cap(tile_slices, ns);
+    for (int q = threadIdx.x; q < kTileHash; q += blockDim.x) key[q] = -1;
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    auto slot_of = [&](int j) { return (int)(((unsigned)j * 2654435761u) >> 22); };   // 10 bits
+    static_assert(kTileHash == 1024, "slot_of gives 10 bits");
+    for (int r = threadIdx.x; r < 64 * ns; r += blockDim.x) {
+        const int L = len8[row0 + r];
+        const int64_t base = sl[g0 + (r >> 6)].sbase + (r & 63);
+        for (int q = 0; q < L; ++q) {
+            const int j = col[base + 64 * (int64_t)q];
+            if (j >= row0 && j < row1) continue;
+            for (int h = slot_of(j), n = 0; n < kTileHash; ++n, h = (h + 1) & (kTileHash - 1)) {
+                const int old = atomicCAS(key + h, -1, j);
+                if (old == j) break;
+                if (old == -1) {
+                    atomicAdd(&count, 1);
+                    break;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int n = count;
+    if (threadIdx.x == 0) atomicMax(longest, (n > cap) ? 0x7fffffff : n);
+    if (n > cap) return;
+    __syncthreads();
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    for (int h = threadIdx.x; h < kTileHash; h += blockDim.x)
+        if (key[h] >= 0) list[atomicAdd(&count, 1)] = key[h];
+    __syncthreads();
+    for (int h = threadIdx.x; h < kTileHash; h += blockDim.x) {
+        const int k = key[h];
+        if (k < 0) continue;
+        int rank = 0;
+        for (int q = 0; q < n; ++q) rank += (list[q] < k) ? 1 : 0;
+        pos[h] = rank;
+        halo[g0 * swe::kHaloStride + rank] = k;
+    }
+    if (threadIdx.x == 0) sl[g0].nhalo = n;
+    __syncthreads();
+    for (int r = threadIdx.x; r < 64 * ns; r += blockDim.x) {
+        const int L = len8[row0 + r];
+        const int64_t base = sl[g0 + (r >> 6)].sbase + (r & 63);
+        for (int q = 0; q < L; ++q) {
+            const int64_t p = base + 64 * (int64_t)q;
+            const int j = col[p];
+            int l = j - row0;
+            if (j < row0 || j >= row1) {
+                int h = slot_of(j);
+                while (key[h] != j) h = (h + 1) & (kTileHash - 1);
+                l = 64 * tile_slices + pos[h];
+            }
+            lcol[p] = (uint16_t)l;
+        }
+    }
+}
+
 __global__ void k_lay_bc(int nbc, int nh, int nux, int64_t r0, int64_t b0, int inst, const int* __restrict__ nodes1,
-                         const int* __restrict__ iperm, swe::BcEntry* __restrict__ bc) {
+                         const int* __restrict__ iperm, swe::BcEntry* __restrict__ bc, uint8_t* __restrict__ dirm) {
     const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (q >= nbc) return;
     const int comp = (q < nh) ? 0 : (q < nh + nux) ? 1 : 2;
-    bc[b0 + q] = swe::BcEntry{(int)(r0 + iperm[nodes1[q] - 1]), inst, comp, (int)(b0 + q)};
+    const int row = (int)(r0 + iperm[nodes1[q] - 1]);
+    bc[b0 + q] = swe::BcEntry{row, inst, comp, (int)(b0 + q)};
+    // several entries may share a row and rows share a word: set the row's bit in its aligned word
+    atomicOr((unsigned*)dirm + (row >> 2), 1u << (8 * (row & 3) + comp));
 }
 
 }  // namespace
@@ -585,69 +644,47 @@ hipError_t read_u64(const unsigned long long* d, unsigned long long* h, int n, h
     return (e == hipSuccess) ? hipStreamSynchronize(s) : e;
 }
 
-// The base order of the layout.  *base stays null for the caller's numbering; otherwise it lists the
-// nodes along a Hilbert curve of their coordinates, the device counterpart of the host
-// layout's reverse Cuthill-McKee order, under the same SWE_REORDER policy: 1 when the caller's
-// numbering scatters neighbours (mean |i-j| above 2 sqrt(np)) and the curve brings them closer, 2
-// always.  Only the processing order changes; results do not depend on it.
+// The base order of the layout: the nodes along a Hilbert curve of their coordinates, the device
+// counterpart of the host layout's locality order, or the caller's numbering (*base null) under
+// SWE_REORDER=0.  Only the processing order changes; results do not depend on it.
 hipError_t locality_order(const swe_assembly* a, hipStream_t s, int** base) {
     *base = nullptr;
-    const int mode = swe::reorder_mode();
     const int np = a->np;
-    if (mode == 0 || np < 2 || a->nnz <= np) return hipSuccess;
-    unsigned long long* acc = nullptr;   // [0] offset sum, caller's order; [1] curve order; [2..5] box
-    unsigned long long* keys = nullptr;
-    int *idx = nullptr, *order = nullptr, *pos = nullptr;
-    unsigned long long* keys2 = nullptr;
+    if (!swe::reorder_enabled() || np < 2) return hipSuccess;
+    unsigned long long* box = nullptr;
+    unsigned long long *keys = nullptr, *keys2 = nullptr;
+    int *idx = nullptr, *order = nullptr;
     void* tmp = nullptr;
-    unsigned long long h[6] = {0, 0, ~0ull, 0ull, ~0ull, 0ull};
+    unsigned long long h[4] = {~0ull, 0ull, ~0ull, 0ull};
     const unsigned bl = (unsigned)((np + 255) / 256);
-    const double offdiag = (double)(a->nnz - np);
-    hipError_t e = dalloc(&acc, 6, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(acc, h, sizeof h, hipMemcpyHostToDevice, s);
+    hipError_t e = dalloc(&box, 4, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(box, h, sizeof h, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_offset_sum, dim3(bl), dim3(256), 0, s, np, (const int64_t*)a->ia0, (const int*)a->ja,
-                           (const int*)nullptr, acc);
+        hipLaunchKernelGGL(k_bbox, dim3(bl < 1024u ? bl : 1024u), dim3(256), 0, s, np, (const double*)a->rr, box);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = read_u64(acc, h, 1, s);
-    const double mean0 = (double)h[0] / offdiag;
-    bool take = false;
-    if (e == hipSuccess && (mode == 2 || mean0 > 2.0 * std::sqrt((double)np))) {
-        hipLaunchKernelGGL(k_bbox, dim3(bl < 1024u ? bl : 1024u), dim3(256), 0, s, np, (const double*)a->rr, acc + 2);
+    if (e == hipSuccess) e = read_u64(box, h, 4, s);
+    const double x0 = double_of_ord(h[0]), x1 = double_of_ord(h[1]);
+    const double y0 = double_of_ord(h[2]), y1 = double_of_ord(h[3]);
+    const double top = (double)((1 << kCurveBits) - 1);
+    const double sx = (x1 > x0) ? top / (x1 - x0) : 0.0, sy = (y1 > y0) ? top / (y1 - y0) : 0.0;
+    if (e == hipSuccess) e = dalloc(&keys, (size_t)np, s);
+    if (e == hipSuccess) e = dalloc(&keys2, (size_t)np, s);
+    if (e == hipSuccess) e = dalloc(&idx, (size_t)np, s);
+    if (e == hipSuccess) e = dalloc(&order, (size_t)np, s);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_curve_key, dim3(bl), dim3(256), 0, s, np, (const double*)a->rr, x0, sx, y0, sy, keys, idx);
         e = hipGetLastError();
-        if (e == hipSuccess) e = read_u64(acc + 2, h + 2, 4, s);
-        const double x0 = double_of_ord(h[2]), x1 = double_of_ord(h[3]);
-        const double y0 = double_of_ord(h[4]), y1 = double_of_ord(h[5]);
-        const double top = (double)((1 << kCurveBits) - 1);
-        const double sx = (x1 > x0) ? top / (x1 - x0) : 0.0, sy = (y1 > y0) ? top / (y1 - y0) : 0.0;
-        if (e == hipSuccess) e = dalloc(&keys, (size_t)np, s);
-        if (e == hipSuccess) e = dalloc(&keys2, (size_t)np, s);
-        if (e == hipSuccess) e = dalloc(&idx, (size_t)np, s);
-        if (e == hipSuccess) e = dalloc(&order, (size_t)np, s);
-        if (e == hipSuccess) e = dalloc(&pos, (size_t)np, s);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_curve_key, dim3(bl), dim3(256), 0, s, np, (const double*)a->rr, x0, sx, y0, sy, keys, idx);
-            e = hipGetLastError();
-        }
-        size_t bytes = 0;
-        if (e == hipSuccess)
-            e = hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
-        if (e == hipSuccess) e = hipMallocAsync(&tmp, bytes ? bytes : 1, s);
-        if (e == hipSuccess)   // a radix sort is stable: equal keys keep the caller's order
-            e = hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_inverse, dim3(bl), dim3(256), 0, s, np, (const int*)order, pos);
-            hipLaunchKernelGGL(k_offset_sum, dim3(bl), dim3(256), 0, s, np, (const int64_t*)a->ia0,
-                               (const int*)a->ja, (const int*)pos, acc + 1);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess) e = read_u64(acc + 1, h + 1, 1, s);
-        take = e == hipSuccess && (mode == 2 || h[1] < h[0]);
     }
-    void* bufs[] = {acc, keys, keys2, idx, pos, tmp};
+    size_t bytes = 0;
+    if (e == hipSuccess)
+        e = hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
+    if (e == hipSuccess) e = hipMallocAsync(&tmp, bytes ? bytes : 1, s);
+    if (e == hipSuccess)   // a radix sort is stable: equal keys keep the caller's order
+        e = hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
+    void* bufs[] = {box, keys, keys2, idx, tmp};
     for (void* b : bufs) dfree(b, s);
-    if (take) *base = order;
+    if (e == hipSuccess) *base = order;
     else dfree(order, s);
     return e;
 }
@@ -757,7 +794,11 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
     hipStream_t s = P->copy;
     double* dbath = nullptr;
     int* dnodes = nullptr;
+    int* dlong = nullptr;
+    int longest = 0;
     hipError_t e = dalloc(&dbath, (size_t)np, s);
+    if (e == hipSuccess) e = dalloc(&dlong, 1, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(dlong, &longest, sizeof longest, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = dalloc(&dnodes, (size_t)nbc, s);
     if (e == hipSuccess) e = hipMemcpyAsync(dbath, bath, sizeof(double) * (size_t)np, hipMemcpyHostToDevice, s);
     for (int c = 0, q = 0; c < 3 && e == hipSuccess; q += nlist[c], ++c)
@@ -771,7 +812,7 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
         e = hipMemcpyAsync(st + nc * r0, un, sizeof(double) * nc * (size_t)np, hipMemcpyHostToDevice, s);
     }
     if (e == hipSuccess) {
-        LayOut o{P->len, P->dpos, P->perm, P->m, P->z, P->col, P->dcol, P->c};
+        LayOut o{P->len, P->dpos, P->dirm, P->perm, P->m, P->z, P->col, P->dcol, P->c};
         hipLaunchKernelGGL(k_lay_fill, dim3(grid_of(np_pad, 256)), dim3(256), 0, s, np, np_pad, r0, p0,
                            (const int*)DL.perm, (const int*)DL.iperm, (const int*)DL.len, (const int64_t*)DL.sptr,
                            (const int64_t*)a->ia0, (const int*)a->ja, (const double*)a->cx, (const double*)a->cy,
@@ -780,13 +821,17 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
                            (const int*)DL.len, (const uint8_t*)P->dpos, (const int64_t*)DL.sptr,
                            (const int64_t*)DL.eoff, P->elist);
         hipLaunchKernelGGL(k_lay_slice_info, dim3(grid_of(DL.nsl, 256)), dim3(256), 0, s, DL.nsl, s0, p0, e0, k,
-                           (const int64_t*)DL.sptr, (const int64_t*)DL.eoff, P->sl);
+                           P->tile_slices, (const int64_t*)DL.sptr, (const int64_t*)DL.eoff, P->sl);
+        hipLaunchKernelGGL(k_lay_tiles, dim3(grid_of(DL.nsl, P->tile_slices)), dim3(256), 0, s, DL.nsl, s0,
+                           P->tile_slices, (const uint8_t*)P->len, (const int*)P->col, P->sl, P->lcol, P->halo, dlong);
         if (nbc > 0)
             hipLaunchKernelGGL(k_lay_bc, dim3(grid_of(nbc, 256)), dim3(256), 0, s, (int)nbc, nlist[0], nlist[1], r0, b0,
-                               k, (const int*)dnodes, (const int*)DL.iperm, P->bc);
+                               k, (const int*)dnodes, (const int*)DL.iperm, P->bc, P->dirm);
         e = hipGetLastError();
     }
+    if (e == hipSuccess) e = hipMemcpyAsync(&longest, dlong, sizeof longest, hipMemcpyDeviceToHost, s);
     dfree(dbath, s);
+    dfree(dlong, s);
     dfree(dnodes, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
@@ -812,6 +857,7 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
     I.nh = nlist[0];
     I.nux = nlist[1];
     I.nuy = nlist[2];
+    I.max_halo = (longest == 0x7fffffff) ? -1 : longest;
     if ((rc = pool_activate(P, k, I, prm, un != nullptr, t0, tfinal, max_steps))) return rc;
     *id = k;
     return SWE_OK;

@@ -1,0 +1,603 @@
+// swe_tiles.hip -- the step's passes over tiles: one workgroup per tile (up to 4 consecutive slices of an
+// instance, swe_layout.h), one lane per row as in swe_kernels.hip, with the node data of the tile's rows and
+// of its halo staged in LDS first.
+//
+// What this changes against the gather kernels: an entry's column is a 16-bit LDS index that streams in
+// with c_ij, so no load depends on a loaded index (the gather kernels wait about 1700 cycles for each
+// neighbour record); everything that depends on one node only (one_over_h, SQRT(g h), the entropy, the
+// depth ratio against the node's own bed) is evaluated once per staged node instead of once per entry, about
+// 1.2 instead of 7 times per row; and of the two depth ratios of an entry the one whose bed is the
+// higher is that staged quantity, so one division is left of two.  Every expression is the gather kernels',
+// on the same operands, so the results are the same bits.
+#include <hip/hip_runtime.h>
+
+#include "swe_engine.h"
+#include "swe_kernels.h"
+#include "swe_rows.h"
+
+namespace swe {
+
+namespace {
+
+// First slice of this workgroup's tile.
+__device__ __forceinline__ int block_tile(const Mesh& M, int remap) {
+    return __builtin_amdgcn_readfirstlane(M.tact[remap ? xcd_block() : (int)blockIdx.x]);
+}
+
+// MAX(0, h + zb - zb)/h, the depth ratio of a node against its own bed (smb_2: U_i's ratio where its bed is
+// the higher one).
+__device__ __forceinline__ double own_ratio(double h, double z) { return fmaxF(0.0, h + z - z) / h; }
+
+// The depth ratios of an entry before the dry-node rule: qij = MAX(0, h_i + z_i - zmax)/h_i, qji likewise
+// for j, zmax = MAX(z_i, z_j); qi, qj are own_ratio of the two nodes.
+__device__ __forceinline__ void depth_ratios(double hi, double zi, double qi, double hj, double zj, double qj,
+                                             double& Hji, double& qij, double& qji) {
+    const bool up = zi > zj;
+    const double zmax = up ? zi : zj;
+    const double Hij = fmaxF(0.0, hi + zi - zmax);
+    Hji = fmaxF(0.0, hj + zj - zmax);
+    const double quo = (up ? Hji : Hij) / (up ? hj : hi);
+    qij = up ? qi : quo;
+    qji = up ? quo : qj;
+}
+
+// Sums of one row over its entries, for lo_finish.
+struct LoSums {
+    double r1, r2, r3, fix, e1, e2, e3, emax, emin;
+};
+
+// What k_tile_lo stages per node: 80 bytes, read in 16-byte pieces.
+struct alignas(16) LoNode {
+    double h, z, qx, qy;
+    double ovh, sq;       // one_over_h, SQRT(g*ABS(h))
+    double q, E;          // own_ratio, entropy
+    double alpha, pad;
+};
+
+// The row loop of k_tile_lo (the sums of fct_lo_body in swe_kernels.hip).  WET: every node of the tile and its
+// halo is deeper than the dry-node thresholds of both sums, so the ratios need no selection and the two
+// sums' momentum parts are one.
+template <bool WET, bool ALPHA, bool WRITE_LO, bool D0>
+__device__ __forceinline__ void lo_rows(const LoNode* __restrict__ nodes, const Mesh& M, int64_t pb, int len,
+                                        const Node& I, const Consts& K, const Rcp& r16, const double* __restrict__ d0,
+                                        double2* __restrict__ dmu, int roundoff, LoSums& s, int& err) {
+    const int tid = (int)threadIdx.x;
+    const double ovh_i = nodes[tid].ovh, sql = nodes[tid].sq, qi = nodes[tid].q;
+    const double ai = ALPHA ? nodes[tid].alpha : 1.0;
+    const double v1i = I.qx * ovh_i, v2i = I.qy * ovh_i;
+    const double thr_lo = roundoff ? K.htiny : 0.0;
+    double r1 = 0.0, r2 = 0.0, r3 = 0.0, fix = 0.0, e1 = 0.0, e2 = 0.0, e3 = 0.0, emax = 0.0, emin = 0.0;
+    bool split = false;
+    double2 c_next = ld_entry(M.c + pb);
+    int l_next = M.lcol[pb];
+    double d_next = D0 ? ld_entry1(d0 + pb) : 0.0;
+    for (int q = 0; q < len; ++q) {
+        const int64_t p = pb + 64 * (int64_t)q;
+        const double2 c = c_next;
+        const int l = l_next;
+        const double d0p = d_next;
+        if (q + 1 < len) {
+            c_next = ld_entry(M.c + p + 64);
+            l_next = M.lcol[p + 64];
+            if constexpr (D0) d_next = ld_entry1(d0 + p + 64);
+        }
+        const LoNode& n = nodes[l];
+        const Node J{n.h, n.qx, n.qy, n.z};
+        const double ovh_j = n.ovh;
+        const double v1j = J.qx * ovh_j, v2j = J.qy * ovh_j;
+        double Hji, qij, qji;
+        depth_ratios(I.h, I.z, qi, J.h, J.z, n.q, Hji, qij, qji);
+        const double ratij0 = (!WET && I.h <= 0.0) ? 0.0 : qij;
+        const double ratji0 = (!WET && J.h <= 0.0) ? 0.0 : qji;
+        const double ratijr = (!WET && I.h <= thr_lo) ? 0.0 : qij;
+        const double ratjir = (!WET && J.h <= thr_lo) ? 0.0 : qji;
+        const bool off = (l != tid);
+        double d = 0.0, mu = 0.0;
+        if (off) {
+            d = D0 ? d0p : dij_from_c(c, I, J, ovh_i, ovh_j, sql, n.sq, K, r16, err);
+            mu = mu_of(c.x, c.y, v1i, v2i, v1j, v2j);
+            d = fmaxF(d, mu);
+            if constexpr (ALPHA) {
+                const double a = fmaxF(ai, n.alpha);
+                d = d * a;
+                mu = mu * a;
+            }
+            st_entry(dmu + p, make_double2(d, mu));
+        }
+        const double xm = -(c.x * (v1j)) - c.y * (v2j);
+        const double xe = -(c.x * (v1j * J.h)) - c.y * (v2j * J.h);
+        const double xx2 = -(c.x * (v1j * J.qx)) - c.y * (v2j * J.qx);
+        const double xx3 = -(c.x * (v1j * J.qy)) - c.y * (v2j * J.qy);
+        const double topo = K.g * I.h * (J.h + J.z - I.h - I.z);
+        if (!WET && WRITE_LO && !split && !(ratjir == ratji0 && ratijr == ratij0)) {
+            split = true;
+            e2 = r2;
+            e3 = r3;
+        }
+        if (WRITE_LO) {
+            if (roundoff) {
+                if (!off) fix = fix + xm;
+                else {
+                    fix = fix - mu + (d - mu) * (-ratijr);
+                    r1 = r1 + (xm + mu) * J.h + posF((d - mu) * Hji);
+                }
+            } else {
+                r1 = r1 + xe;
+                if (off) r1 = r1 + d * (J.h * ratjir - I.h * ratijr) + mu * (J.h * (1.0 - ratjir) - I.h * (1.0 - ratijr));
+            }
+        }
+        // the low-order momentum sums; without them (entropy viscosity alone) the residual's
+        r2 = r2 + xx2;
+        r3 = r3 + xx3;
+        e1 = e1 + xe;
+        if (off) {
+            const double a = WRITE_LO ? ratjir : ratji0, b = WRITE_LO ? ratijr : ratij0;
+            r2 = r2 + d * (J.qx * a - I.qx * b) + mu * (J.qx * (1.0 - a) - I.qx * (1.0 - b));
+            r3 = r3 + d * (J.qy * a - I.qy * b) + mu * (J.qy * (1.0 - a) - I.qy * (1.0 - b));
+            e1 = e1 + d * (J.h * ratji0 - I.h * ratij0) + mu * (J.h * (1.0 - ratji0) - I.h * (1.0 - ratij0));
+        }
+        r2 = r2 - topo * c.x;
+        r3 = r3 - topo * c.y;
+        if (!WET && split) {
+            e2 = e2 + xx2;
+            e3 = e3 + xx3;
+            if (off) {
+                e2 = e2 + d * (J.qx * ratji0 - I.qx * ratij0) + mu * (J.qx * (1.0 - ratji0) - I.qx * (1.0 - ratij0));
+                e3 = e3 + d * (J.qy * ratji0 - I.qy * ratij0) + mu * (J.qy * (1.0 - ratji0) - I.qy * (1.0 - ratij0));
+            }
+            e2 = e2 - topo * c.x;
+            e3 = e3 - topo * c.y;
+        }
+        const double Ej = n.E;
+        if (q == 0) {
+            emax = Ej;
+            emin = Ej;
+        } else {
+            emax = (Ej > emax) ? Ej : emax;
+            emin = (Ej < emin) ? Ej : emin;
+        }
+    }
+    if (!split) {
+        e2 = r2;
+        e3 = r3;
+    }
+    s = LoSums{r1, r2, r3, fix, e1, e2, e3, emax, emin};
+}
+
+// =============================================================================================
+// FCT / entropy-viscosity stage, pass 1 on tiles: k_fct_lo's results (viscosities dmu, low-order solution,
+// entropy residual).
+// =============================================================================================
+template <bool ALPHA, bool WRITE_LO, bool HAS_SRC, bool D0>
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, double* __restrict__ ulo_h,
+          double2* __restrict__ ulo_q, double2* __restrict__ dmu, double* __restrict__ res,
+          const double* __restrict__ d0, const double* __restrict__ alpha, int roundoff, int* __restrict__ flags_out,
+          int remap) {
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    LoNode* nodes = (LoNode*)smem;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const Consts K = T[inst].K;
+    const double dt = T[inst].dt;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const double wet_h = fmaxF(K.htiny, 0.0);
+    bool wet = true;
+    auto stage = [&](int k, const Node& A, int row) {
+        LoNode n;
+        n.h = A.h;
+        n.z = A.z;
+        n.qx = A.qx;
+        n.qy = A.qy;
+        n.ovh = ovh_of(A.h, K.htiny);
+        n.sq = D0 ? 0.0 : sqrt_rn(K.g * fabs(A.h));
+        n.q = own_ratio(A.h, A.z);
+        // entropy (update.f90:924-935)
+        double E = K.g * (A.h * A.h);
+        E = E + (A.qx * n.ovh) * A.qx;
+        E = E + (A.qy * n.ovh) * A.qy;
+        n.E = 0.5 * E;
+        n.alpha = ALPHA ? alpha[row] : 0.0;
+        nodes[k] = n;
+        wet = wet && A.h > wet_h;
+    };
+    Node I{};
+    if (len > 0) {
+        I = U[i];
+        stage(tid, I, i);
+    }
+    for (int k = tid; k < S.nhalo; k += R) {
+        const int j = M.halo[(int64_t)s0 * kHaloStride + k];
+        stage(R + k, U[j], j);
+    }
+    const bool all_wet = __syncthreads_and(wet ? 1 : 0) != 0;
+    if (len == 0) return;
+    const Rcp r16 = uniform_rcp(K.g16);
+    const int64_t pb = M.sl[s0 + w].sbase + (tid & 63);
+    int err = 0;
+    LoSums s;
+    if (all_wet) lo_rows<true, ALPHA, WRITE_LO, D0>(nodes, M, pb, len, I, K, r16, d0, dmu, roundoff, s, err);
+    else lo_rows<false, ALPHA, WRITE_LO, D0>(nodes, M, pb, len, I, K, r16, d0, dmu, roundoff, s, err);
+    const double mi = M.m[i];
+    const double ovh_i = nodes[tid].ovh;
+    const double v1i = I.qx * ovh_i, v2i = I.qy * ovh_i;
+    double e1 = s.e1, e2 = s.e2, e3 = s.e3;
+    add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, e2, e3);
+    if (WRITE_LO) {
+        double r1 = s.r1, r2 = s.r2, r3 = s.r3;
+        add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, r2, r3);
+        r1 = r1 / mi;
+        r2 = r2 / mi;
+        r3 = r3 / mi;
+        double hL;
+        if (roundoff) hL = I.h * (1.0 + dt * s.fix / mi) + dt * r1;
+        else hL = fmaxF(I.h + dt * r1, 0.0);
+        st_entry1(ulo_h + i, hL);
+        st_entry(ulo_q + i, make_double2(I.qx + dt * r2, I.qy + dt * r3));
+        if (K.check_h && hL < 0.0) err |= FLAG_NEG_H;
+    }
+    // entropy_residual (update.f90:838-868)
+    e1 = e1 / mi;
+    e2 = e2 / mi;
+    e3 = e3 / mi;
+    const double ht = I.h + dt * e1;
+    const double qxt = I.qx + dt * e2;
+    const double qyt = I.qy + dt * e3;
+    const double ovt = ovh_of(ht, K.htiny);
+    const double vn1 = qxt * ovt, vn2 = qyt * ovt;
+    const double E = nodes[tid].E;
+    double En = K.g * (ht * ht);
+    En = En + vn1 * qxt;
+    En = En + vn2 * qyt;
+    En = 0.5 * En;
+    double Ep0 = K.g * I.h;
+    Ep0 = Ep0 - 0.5 * (v1i * v1i);
+    Ep0 = Ep0 - 0.5 * (v2i * v2i);
+    double r = mi * (En - E) / dt;
+    r = r - mi * e1 * Ep0;
+    r = r - mi * e2 * v1i;
+    r = r - mi * e3 * v2i;
+    const double rescale = fabs(s.emax - s.emin) / 2.0 + K.ent_cst;
+    res[i] = fabs(r) / rescale;
+    raise_flag(flags_out, inst, err);
+}
+
+// =============================================================================================
+// FCT stage, pass 2 on tiles: k_fct_rminus's R-.
+// =============================================================================================
+// What the limiter passes stage per node.
+struct alignas(16) FluxNode {
+    double h, z, q, res;   // q: own_ratio
+};
+struct alignas(16) ApplyNode {
+    double h, z, q, res, qx, qy, Rm, pad;
+};
+
+// Entries a lane holds in registers: their viscosities and columns are loaded before the staging barrier, all
+// at once; longer rows read the rest in a loop.
+constexpr int kHeld = 8;
+
+struct HeldRow {
+    double2 lo[kHeld];
+    int l[kHeld];
+};
+__device__ __forceinline__ void hold_row(HeldRow& H, const Mesh& M, const double2* __restrict__ dmu, int64_t pb, int len) {
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q)
+        if (q < len) {
+            H.lo[q] = ld_entry(dmu + pb + 64 * q);
+            H.l[q] = M.lcol[pb + 64 * q];
+        }
+}
+
+// Antidiffusive flux of an off-diagonal entry (fct_flux of swe_rows.h, the depth ratios from the staged nodes).
+template <class N>
+__device__ __forceinline__ double tile_flux(const N& I, const N& J, const double2 lo, double& dA, double& muA,
+                                            double& ratij, double& ratji) {
+    const double rij = fmaxF(I.res, J.res);
+    dA = fminF(lo.x, 1.0 * rij) - lo.x;
+    muA = fminF(lo.y, 1.0 * rij) - lo.y;
+    double Hji;
+    depth_ratios(I.h, I.z, I.q, J.h, J.z, J.q, Hji, ratij, ratji);
+    ratij = (I.h <= 0.0) ? 0.0 : ratij;
+    ratji = (J.h <= 0.0) ? 0.0 : ratji;
+    return dA * (J.h * ratji - I.h * ratij) + muA * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
+}
+
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_rminus(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const double* __restrict__ ulo_h,
+              const double2* __restrict__ dmu, const double* __restrict__ res, double* __restrict__ Rm, int remap) {
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    FluxNode* nodes = (FluxNode*)smem;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const double dt = T[inst].dt;
+    const double htiny = T[inst].K.htiny;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    HeldRow H;
+    hold_row(H, M, dmu, pb, len);
+    auto stage = [&](int k, int row) {
+        const Node A = U[row];
+        nodes[k] = FluxNode{A.h, A.z, own_ratio(A.h, A.z), res[row]};
+    };
+    if (len > 0) stage(tid, i);
+    for (int k = tid; k < S.nhalo; k += R) stage(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    __syncthreads();
+    if (len == 0) return;
+    const FluxNode I = nodes[tid];
+    double P = -1.0e-15;
+    auto entry = [&](const double2 lo, int l) {
+        if (l == tid) return;    // f_ii is a zero, never < 0
+        double dA, muA, rij_, rji_;
+        const double f = tile_flux(I, nodes[l], lo, dA, muA, rij_, rji_);
+        if (f < 0.0) P = P + f;
+    };
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q)
+        if (q < len) entry(H.lo[q], H.l[q]);
+    for (int q = kHeld; q < len; ++q) entry(ld_entry(dmu + pb + 64 * q), M.lcol[pb + 64 * q]);
+    const double scaled = (M.m[i] / dt) * ulo_h[i];
+    const double Q = 0.0 - scaled;
+    double Ri = fminF(Q / P, 1.0);
+    if (scaled <= htiny) Ri = 0.0;
+    Rm[i] = Ri;
+}
+
+// =============================================================================================
+// FCT stage, pass 3 on tiles: k_fct_apply's limited update and RK combination, with the wall and inflow
+// values of bdy.
+// =============================================================================================
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_apply(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const Node* __restrict__ Uo,
+             const double* __restrict__ ulo_h, const double2* __restrict__ ulo_q, Node* __restrict__ out,
+             const double2* __restrict__ dmu, const double* __restrict__ res, const double* __restrict__ Rm, int stage,
+             int bdy, int* __restrict__ flags_out, int remap) {
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    ApplyNode* nodes = (ApplyNode*)smem;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const double dt = T[inst].dt;
+    const int check_h = T[inst].K.check_h;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    HeldRow H;
+    hold_row(H, M, dmu, pb, len);
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
+        nodes[k] = ApplyNode{A.h, A.z, own_ratio(A.h, A.z), res[row], A.qx, A.qy, Rm[row], 0.0};
+    };
+    if (len > 0) put(tid, i);
+    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    __syncthreads();
+    if (len == 0) return;
+    const ApplyNode I = nodes[tid];
+    double x1 = 0.0, x2 = 0.0, x3 = 0.0;
+    auto entry = [&](const double2 lo, int l) {
+        if (l == tid) return;    // contributes d*(0) + mu*(0)
+        const ApplyNode& J = nodes[l];
+        double dA, muA, ratij, ratji;
+        const double f = tile_flux(I, J, lo, dA, muA, ratij, ratji);
+        const double lim = (f >= 0.0) ? J.Rm : I.Rm;
+        const double d = dA * lim;
+        const double mu = muA * lim;
+        const double a = 1.0 - ratji, b = 1.0 - ratij;
+        x1 = x1 + d * (J.h * ratji - I.h * ratij) + mu * (J.h * a - I.h * b);
+        x2 = x2 + d * (J.qx * ratji - I.qx * ratij) + mu * (J.qx * a - I.qx * b);
+        x3 = x3 + d * (J.qy * ratji - I.qy * ratij) + mu * (J.qy * a - I.qy * b);
+    };
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q)
+        if (q < len) entry(H.lo[q], H.l[q]);
+    for (int q = kHeld; q < len; ++q) entry(ld_entry(dmu + pb + 64 * q), M.lcol[pb + 64 * q]);
+    const double mi = M.m[i];
+    const double hL = ld_entry1(ulo_h + i);   // low-order solution of k_tile_lo
+    const double2 qL = ld_entry(ulo_q + i);
+    Node o;
+    o.h = hL + dt * (x1 / mi);
+    o.qx = qL.x + dt * (x2 / mi);
+    o.qy = qL.y + dt * (x3 / mi);
+    const int err = (check_h && o.h < 0.0) ? FLAG_NEG_H : 0;
+    if (stage != 0) {
+        const Node P = Uo[i];
+        o.h = rk_combine(stage, P.h, o.h);
+        o.qx = rk_combine(stage, P.qx, o.qx);
+        o.qy = rk_combine(stage, P.qy, o.qy);
+    }
+    o.z = I.z;
+    if (bdy) {
+        const int mask = M.dirm[i];
+        if (mask) bdy_row(o, mask, T[inst], stage);
+    }
+    out[i] = o;
+    raise_flag(flags_out, inst, err);
+}
+
+// =============================================================================================
+// COMPUTE_DT on tiles: k_compute_dt's d_ij (kept in d0 for the first stage) and per-instance maxima; with
+// advance, the workgroup that ends last does the step's bookkeeping (k_finalize_dt) as well.
+// =============================================================================================
+struct alignas(16) DtNode {
+    double h, qx, qy, ovh, sq, pad;
+};
+
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_dt(Mesh M, InstDev* __restrict__ T, const Node* __restrict__ U, double* __restrict__ d0,
+          unsigned long long* __restrict__ vmax, int* __restrict__ flags, unsigned* __restrict__ done, int all,
+          int advance, int ninst, int remap) {
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    DtNode* nodes = (DtNode*)smem;
+    __shared__ unsigned long long red[kMaxTileSlices];
+    __shared__ int last;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // (per wave: a check raised meanwhile may end some waves' part; every barrier is met by all of them)
+    const bool live = inst >= 0 && (all ? T[inst].state != INST_FREE : takes_steps(T[inst], flags[inst]));
+    const int i = s0 * 64 + tid;
+    const int len = (live && w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    Consts K{};
+    double2 c_next{};
+    int l_next = 0;
+    if (live) {
+        K = T[inst].K;
+        if (len > 0) {
+            c_next = ld_entry(M.c + pb);
+            l_next = M.lcol[pb];
+        }
+        auto put = [&](int k, int row) {
+            const Node A = U[row];
+            nodes[k] = DtNode{A.h, A.qx, A.qy, ovh_of(A.h, K.htiny), sqrt_rn(K.g * fabs(A.h)), 0.0};
+        };
+        if (len > 0) put(tid, i);
+        for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    }
+    __syncthreads();
+    double v = 0.0;
+    int err = 0;
+    if (len > 0) {
+        const Rcp r16 = uniform_rcp(K.g16);
+        const DtNode A = nodes[tid];
+        const Node I{A.h, A.qx, A.qy, 0.0};
+        double s = 0.0;
+        for (int q = 0; q < len; ++q) {
+            const int64_t p = pb + 64 * (int64_t)q;
+            const double2 c = c_next;
+            const int l = l_next;
+            if (q + 1 < len) {
+                c_next = ld_entry(M.c + p + 64);
+                l_next = M.lcol[p + 64];
+            }
+            if (l == tid) continue;    // the reference's row sum adds a 0.0 there
+            const DtNode& B = nodes[l];
+            const Node J{B.h, B.qx, B.qy, 0.0};
+            const double d = dij_from_c(c, I, J, A.ovh, B.ovh, A.sq, B.sq, K, r16, err);
+            if (d0) st_entry1(d0 + p, d);
+            s = s + d;
+        }
+        v = fabs(-s) / M.m[i];
+    }
+    if (err) {
+        atomicOr(flags + inst, err);
+        __builtin_amdgcn_s_waitcnt(0);    // done before this workgroup's arrival below
+    }
+    // v >= 0 orders like its bit pattern
+    unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(b, off, 64);
+        b = (o > b) ? o : b;
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = b;
+    __syncthreads();
+    if (tid == 0) {
+        unsigned long long mx = 0ull;
+        for (int k = 0; k < R / 64; ++k) mx = (red[k] > mx) ? red[k] : mx;
+        // most workgroups find a greater maximum already there and leave the word alone
+        if (mx > __hip_atomic_load(vmax + inst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(vmax + inst, mx);
+    }
+    if (!advance) return;
+    // The workgroup's flags and maximum are in place before its arrival counts (each thread waits for its own
+    // atomics), so the workgroup that arrives last sees all of them; it reads them with atomics, which bypass
+    // what its XCD may have cached.
+    // Arrivals count in kDoneGroups words first and then, once per word, in one: a single word serialises them
+    // (1568 workgroups: 31 us for the pass, 22 us with half as many).
+    if (tid == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        const unsigned n = gridDim.x, g = blockIdx.x % kDoneGroups;
+        const unsigned groups = n < kDoneGroups ? n : kDoneGroups, members = (n - g + kDoneGroups - 1) / kDoneGroups;
+        unsigned* mine = done + kDoneStride * (1 + g);
+        int end = 0;
+        if (atomicAdd(mine, 1u) == members - 1) {
+            atomicExch(mine, 0u);
+            if (atomicAdd(done, 1u) == groups - 1) {
+                atomicExch(done, 0u);
+                end = 1;
+            }
+        }
+        last = end;
+    }
+    __syncthreads();
+    if (!last) return;
+    for (int k = tid; k < ninst; k += R) {
+        const unsigned long long mx = atomicExch(vmax + k, 0ull);
+        const int f = __hip_atomic_load(flags + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        finalize_one(T, mx, f, k, 1);
+    }
+}
+
+template <bool ALPHA, bool WRITE_LO, bool HAS_SRC, bool D0>
+void go_tile_lo(Pool& P, const Node* U, const double* d0) {
+    const Mesh M = mesh_view(P);
+    hipLaunchKernelGGL((k_tile_lo<ALPHA, WRITE_LO, HAS_SRC, D0>), dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                       sizeof(LoNode) * (size_t)P.tile_nodes, P.stream, M, (const InstDev*)P.tab, U, P.ulo_h, P.ulo_q,
+                       P.dmu, P.res, d0, (const double*)P.alpha, P.mode.roundoff, P.flags, P.tune.k[KID_FCT_LO].remap);
+}
+
+template <bool ALPHA, bool WRITE_LO>
+void go_tile_lo(Pool& P, const Node* U, const double* d0) {
+    if (P.any_src) {
+        if (d0) go_tile_lo<ALPHA, WRITE_LO, true, true>(P, U, d0);
+        else go_tile_lo<ALPHA, WRITE_LO, true, false>(P, U, d0);
+    } else {
+        if (d0) go_tile_lo<ALPHA, WRITE_LO, false, true>(P, U, d0);
+        else go_tile_lo<ALPHA, WRITE_LO, false, false>(P, U, d0);
+    }
+}
+
+}  // namespace
+
+void launch_tile_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo) {
+    if (write_lo) {
+        if (alpha) go_tile_lo<true, true>(P, U, d0);
+        else go_tile_lo<false, true>(P, U, d0);
+    } else {
+        if (alpha) go_tile_lo<true, false>(P, U, d0);
+        else go_tile_lo<false, false>(P, U, d0);
+    }
+}
+
+void launch_tile_rminus(Pool& P, const Node* U) {
+    hipLaunchKernelGGL(k_tile_rminus, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                       sizeof(FluxNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U,
+                       (const double*)P.ulo_h, (const double2*)P.dmu, (const double*)P.res, P.Rm,
+                       P.tune.k[KID_RMINUS].remap);
+}
+
+void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy) {
+    hipLaunchKernelGGL(k_tile_apply, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                       sizeof(ApplyNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U, Uo,
+                       (const double*)P.ulo_h, (const double2*)P.ulo_q, out, (const double2*)P.dmu,
+                       (const double*)P.res, (const double*)P.Rm, stage, bdy ? 1 : 0, P.flags,
+                       P.tune.k[KID_APPLY].remap);
+}
+
+void launch_tile_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
+    hipLaunchKernelGGL(k_tile_dt, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                       sizeof(DtNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), P.tab, U, d0, P.vmax, P.flags,
+                       P.done, all, advance ? 1 : 0, P.ninst(), P.tune.k[KID_DT].remap);
+}
+
+}  // namespace swe
