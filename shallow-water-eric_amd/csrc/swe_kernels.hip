@@ -375,14 +375,6 @@ k_stage_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
 // the RK combination.  One kernel per stage; its workgroup size and slice order (dispatch or
 // XCD-aware) are the tuned ones of the first-order stage, whose place it takes in the step.
 // =============================================================================================
-// pTilde (update.f90:515-518) at node n: paper_constant = lambdaSGN*g/(3*SQRT(lumped)),
-// x = (h*eta)/h**2; the literal integer powers are products from the left, as flang expands them.
-__device__ __forceinline__ double sgn_ptilde(double h, double he, double m, const Consts& K) {
-    const double pc = K.lambda_sgn * K.g / (3.0 * sqrt_rn(m));
-    const double x = he / (h * h);
-    return pc * (h * h * h) * (2.0 + 4.0 * (x * x * x) - 6.0 * (x * x * x * x));
-}
-
 template <int BS, int SMB, bool ALPHA>
 __global__ void __launch_bounds__(BS)
 k_stage_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const NodeX* __restrict__ UX,
@@ -1498,12 +1490,17 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
                                                   M, T, U, P.alpha, L.remap))
         timed_end(P, KID_ALPHA);
     }
-    if (md.sgn) {
+    if (md.sgn && !(ext_of(P, U) && ext_of(P, Uo) && ext_of(P, out)))
+        return fail(SWE_EINVAL, "SGN stage on a buffer without h*eta, h*w");
+    if ((md.viscosity_type == SWE_GALERKIN || md.viscosity_type == SWE_VISCOUS) && tile_stage_applies(P)) {
+        timed_begin(P, KID_STAGE_LO);
+        launch_tile_stage(P, U, Uo, out, d0, alpha, stage, bdy);
+        timed_end(P, KID_STAGE_LO);
+    } else if (md.sgn) {
         // the SGN model (first-order and galerkin schemes only)
         const NodeX* UX = ext_of(P, U);
         const NodeX* UoX = ext_of(P, Uo);
         NodeX* outX = ext_of(P, out);
-        if (!UX || !UoX || !outX) return fail(SWE_EINVAL, "SGN stage on a buffer without h*eta, h*w");
         const LaunchCfg& L = P.tune.k[KID_STAGE_LO];
         const int smb = (md.viscosity_type == SWE_GALERKIN) ? SMB_GALERKIN
                         : (md.viscous_type == 1)             ? SMB_1
@@ -1576,18 +1573,20 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
         if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, false);
         else if (alpha) launch_fct_lo<true, false>(P, U, d0);
         else launch_fct_lo<false, false>(P, U, d0);
-        const LaunchCfg& L = P.tune.k[KID_EV];
         timed_begin(P, KID_EV);
-        constexpr int BS = 256;
-        const dim3 g(blocks_of((int64_t)M.nact * 64, BS));
-        if (P.any_src)
-            hipLaunchKernelGGL((k_ev_update<BS, true>), g, dim3(BS), 0, P.stream, M, T, U, Uo, out,
-                               (const double2*)P.dmu, (const double*)P.res, md.roundoff, stage,
-                               P.flags, L.remap);
-        else
-            hipLaunchKernelGGL((k_ev_update<BS, false>), g, dim3(BS), 0, P.stream, M, T, U, Uo, out,
-                               (const double2*)P.dmu, (const double*)P.res, md.roundoff, stage,
-                               P.flags, L.remap);
+        if (tiles_apply(P)) {
+            launch_tile_ev(P, U, Uo, out, stage, bdy);
+        } else {
+            const LaunchCfg& L = P.tune.k[KID_EV];
+            constexpr int BS = 256;
+            const dim3 g(blocks_of((int64_t)M.nact * 64, BS));
+            if (P.any_src)
+                hipLaunchKernelGGL((k_ev_update<BS, true>), g, dim3(BS), 0, P.stream, M, T, U, Uo, out,
+                                   (const double2*)P.dmu, (const double*)P.res, md.roundoff, stage, P.flags, L.remap);
+            else
+                hipLaunchKernelGGL((k_ev_update<BS, false>), g, dim3(BS), 0, P.stream, M, T, U, Uo, out,
+                                   (const double2*)P.dmu, (const double*)P.res, md.roundoff, stage, P.flags, L.remap);
+        }
         timed_end(P, KID_EV);
     }
     const hipError_t e = hipGetLastError();
@@ -1595,7 +1594,10 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
     return SWE_OK;
 }
 
-bool bdy_fused(const Pool& P) { return P.mode.viscosity_type == SWE_FCT && tiles_apply(P); }
+bool bdy_fused(const Pool& P) {
+    const bool two_pass = P.mode.viscosity_type == SWE_FCT || P.mode.viscosity_type == SWE_ENTROPY_VISC;
+    return two_pass ? tiles_apply(P) : tile_stage_applies(P);
+}
 
 void launch_bdy(Pool& P, Node* u, int stage) {
     const int64_t n = P.nbc();

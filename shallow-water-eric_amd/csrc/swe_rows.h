@@ -259,6 +259,14 @@ __device__ __forceinline__ double fct_flux(const Node& I, const Node& J, double 
     return (dH - dLp) * (J.h * ratji - I.h * ratij) + (muH - muLp) * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
 }
 
+// pTilde (update.f90:515-518) at node n: paper_constant = lambdaSGN*g/(3*SQRT(lumped)),
+// x = (h*eta)/h**2; the literal integer powers are products from the left, as flang expands them.
+__device__ __forceinline__ double sgn_ptilde(double h, double he, double m, const Consts& K) {
+    const double pc = K.lambda_sgn * K.g / (3.0 * sqrt_rn(m));
+    const double x = he / (h * h);
+    return pc * (h * h * h) * (2.0 + 4.0 * (x * x * x) - 6.0 * (x * x * x * x));
+}
+
 // bdy (SOURCES/main.f90:176-188) of one row whose Dirichlet components are the bits of mask (1 h, 2 qx, 4 qy):
 // the wall and inflow programs, whose values follow from the instance's record.  (Given values come from
 // the boundary list: k_bdy.)

@@ -11,6 +11,8 @@
 // on the same operands, so the results are the same bits.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "swe_engine.h"
 #include "swe_kernels.h"
 #include "swe_rows.h"
@@ -31,10 +33,10 @@ __device__ __forceinline__ double own_ratio(double h, double z) { return fmaxF(0
 // The depth ratios of an entry before the dry-node rule: qij = MAX(0, h_i + z_i - zmax)/h_i, qji likewise
 // for j, zmax = MAX(z_i, z_j); qi, qj are own_ratio of the two nodes.
 __device__ __forceinline__ void depth_ratios(double hi, double zi, double qi, double hj, double zj, double qj,
-                                             double& Hji, double& qij, double& qji) {
+                                             double& Hij, double& Hji, double& qij, double& qji) {
     const bool up = zi > zj;
     const double zmax = up ? zi : zj;
-    const double Hij = fmaxF(0.0, hi + zi - zmax);
+    Hij = fmaxF(0.0, hi + zi - zmax);
     Hji = fmaxF(0.0, hj + zj - zmax);
     const double quo = (up ? Hji : Hij) / (up ? hj : hi);
     qij = up ? qi : quo;
@@ -85,8 +87,8 @@ __device__ __forceinline__ void lo_rows(const LoNode* __restrict__ nodes, const 
         const Node J{n.h, n.qx, n.qy, n.z};
         const double ovh_j = n.ovh;
         const double v1j = J.qx * ovh_j, v2j = J.qy * ovh_j;
-        double Hji, qij, qji;
-        depth_ratios(I.h, I.z, qi, J.h, J.z, n.q, Hji, qij, qji);
+        double Hij, Hji, qij, qji;
+        depth_ratios(I.h, I.z, qi, J.h, J.z, n.q, Hij, Hji, qij, qji);
         const double ratij0 = (!WET && I.h <= 0.0) ? 0.0 : qij;
         const double ratji0 = (!WET && J.h <= 0.0) ? 0.0 : qji;
         const double ratijr = (!WET && I.h <= thr_lo) ? 0.0 : qij;
@@ -303,8 +305,8 @@ __device__ __forceinline__ double tile_flux(const N& I, const N& J, const double
     const double rij = fmaxF(I.res, J.res);
     dA = fminF(lo.x, 1.0 * rij) - lo.x;
     muA = fminF(lo.y, 1.0 * rij) - lo.y;
-    double Hji;
-    depth_ratios(I.h, I.z, I.q, J.h, J.z, J.q, Hji, ratij, ratji);
+    double Hij, Hji;
+    depth_ratios(I.h, I.z, I.q, J.h, J.z, J.q, Hij, Hji, ratij, ratji);
     ratij = (I.h <= 0.0) ? 0.0 : ratij;
     ratji = (J.h <= 0.0) ? 0.0 : ratji;
     return dA * (J.h * ratji - I.h * ratij) + muA * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
@@ -428,6 +430,373 @@ k_tile_apply(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
         if (mask) bdy_row(o, mask, T[inst], stage);
     }
     out[i] = o;
+    raise_flag(flags_out, inst, err);
+}
+
+// =============================================================================================
+// First-order stage on tiles: k_stage_lo's update, with the wall and inflow values of bdy.
+// =============================================================================================
+struct alignas(16) StageNode {
+    double h, z, qx, qy, ovh, sq, q, alpha;
+};
+
+// Low-order sums of an entry with the neighbour's components uj over the own ui (k_stage_lo's and
+// k_stage_sgn's; v2fi, v2fj are the second velocities of the flux).
+template <int SMB, int NC>
+__device__ __forceinline__ void stage_entry(double (&r)[NC], double& fix, const double (&ui)[NC], const double (&uj)[NC],
+                                            double zi, double zj, const double2 c, double v1i, double v2fi, double v1j,
+                                            double v2fj, double Hij, double Hji, double ratij, double ratji, double d,
+                                            double mu, bool off, const Consts& K) {
+    if constexpr (SMB == SMB_1) {
+        // smb_1 (update.f90:378-409)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const double xx = -(c.x * (v1j * uj[k] * ratji + v1i * ui[k] * ratij)) -
+                              c.y * (v2fj * uj[k] * ratji + v2fi * ui[k] * ratij);
+            r[k] = r[k] + xx;
+            if (off) r[k] = r[k] + d * (uj[k] * ratji - ui[k] * ratij);
+        }
+        if (off) {
+            const double t = 0.5 * K.g * (Hji * Hji - Hij * Hij);
+            r[1] = r[1] - t * c.x;
+            r[2] = r[2] - t * c.y;
+        }
+    } else {
+        constexpr int k0 = (SMB == SMB_ROUNDOFF) ? 1 : 0;
+        if constexpr (SMB == SMB_ROUNDOFF) {
+            // smb_2_roundoff (update.f90:566-611): mass equation with fix_roundoff
+            const double xm = -(c.x * (v1j)) - c.y * (v2fj);
+            if (!off) {
+                fix = fix + xm;
+            } else {
+                fix = fix - mu + (d - mu) * (-ratij);
+                r[0] = r[0] + (xm + mu) * uj[0] + posF((d - mu) * Hji);
+            }
+        }
+        const double aj = 1.0 - ratji, ai = 1.0 - ratij;
+#pragma unroll
+        for (int k = k0; k < NC; ++k) {
+            // smb_2 (update.f90:656-663)
+            const double xx = -(c.x * (v1j * uj[k])) - c.y * (v2fj * uj[k]);
+            r[k] = r[k] + xx;
+            if (SMB != SMB_GALERKIN && off)
+                r[k] = r[k] + d * (uj[k] * ratji - ui[k] * ratij) + mu * (uj[k] * aj - ui[k] * ai);
+        }
+        const double topo = K.g * ui[0] * (uj[0] + zj - ui[0] - zi);
+        r[1] = r[1] - topo * c.x;
+        r[2] = r[2] - topo * c.y;
+    }
+}
+
+// The Euler update of the depth and the RK combination with the walls and inflow of bdy.
+template <int SMB>
+__device__ __forceinline__ double stage_depth(double h, double dt, double fix, double mi, double r1) {
+    if constexpr (SMB == SMB_1) return h + dt * r1;
+    else if constexpr (SMB == SMB_ROUNDOFF) return h * (1.0 + dt * fix / mi) + dt * r1;
+    else return fmaxF(h + dt * r1, 0.0);
+}
+__device__ __forceinline__ void stage_out(Node o, const Mesh& M, const InstDev& D, const Node* __restrict__ Uo,
+                                          Node* __restrict__ out, int i, int stage, int bdy) {
+    if (stage != 0) {
+        const Node P = Uo[i];
+        o.h = rk_combine(stage, P.h, o.h);
+        o.qx = rk_combine(stage, P.qx, o.qx);
+        o.qy = rk_combine(stage, P.qy, o.qy);
+    }
+    if (bdy) {
+        const int mask = M.dirm[i];
+        if (mask) bdy_row(o, mask, D, stage);
+    }
+    out[i] = o;
+}
+
+template <int SMB, bool ALPHA, bool HAS_SRC, bool D0>
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_stage(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const Node* __restrict__ Uo,
+             Node* __restrict__ out, const double* __restrict__ d0, const double* __restrict__ alpha, int stage, int bdy,
+             int* __restrict__ flags_out, int remap) {
+    constexpr bool VISC = SMB != SMB_GALERKIN;
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    StageNode* nodes = (StageNode*)smem;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const Consts K = T[inst].K;
+    const double dt = T[inst].dt;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    double2 c_next{};
+    int l_next = 0;
+    double d_next = 0.0;
+    if (len > 0) {
+        c_next = ld_entry(M.c + pb);
+        l_next = M.lcol[pb];
+        if constexpr (VISC && D0) d_next = ld_entry1(d0 + pb);
+    }
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
+        nodes[k] = StageNode{A.h, A.z, A.qx, A.qy, ovh_of(A.h, K.htiny),
+                             (VISC && !D0) ? sqrt_rn(K.g * fabs(A.h)) : 0.0, own_ratio(A.h, A.z),
+                             ALPHA ? alpha[row] : 0.0};
+    };
+    if (len > 0) put(tid, i);
+    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    __syncthreads();
+    if (len == 0) return;
+    const Rcp r16 = uniform_rcp(K.g16);
+    const StageNode A = nodes[tid];
+    const Node I{A.h, A.qx, A.qy, A.z};
+    const double v1i = I.qx * A.ovh, v2i = I.qy * A.ovh;
+    const double thr = (SMB == SMB_ROUNDOFF || SMB == SMB_1) ? K.htiny : 0.0;
+    const double ui[3] = {I.h, I.qx, I.qy};
+    double r[3] = {0.0, 0.0, 0.0}, fix = 0.0;
+    int err = 0;
+    for (int q = 0; q < len; ++q) {
+        const int64_t p = pb + 64 * (int64_t)q;
+        const double2 c = c_next;
+        const int l = l_next;
+        const double d0p = d_next;
+        if (q + 1 < len) {
+            c_next = ld_entry(M.c + p + 64);
+            l_next = M.lcol[p + 64];
+            if constexpr (VISC && D0) d_next = ld_entry1(d0 + p + 64);
+        }
+        const StageNode& B = nodes[l];
+        const Node J{B.h, B.qx, B.qy, B.z};
+        const double v1j = J.qx * B.ovh, v2j = J.qy * B.ovh;
+        double Hij, Hji, ratij, ratji;
+        depth_ratios(I.h, I.z, A.q, J.h, J.z, B.q, Hij, Hji, ratij, ratji);
+        ratij = (I.h <= thr) ? 0.0 : ratij;
+        ratji = (J.h <= thr) ? 0.0 : ratji;
+        const bool off = (l != tid);
+        double d = 0.0, mu = 0.0;
+        if (VISC && off) {
+            d = D0 ? d0p : dij_from_c(c, I, J, A.ovh, B.ovh, A.sq, B.sq, K, r16, err);
+            mu = mu_of(c.x, c.y, v1i, v2i, v1j, v2j);
+            d = fmaxF(d, mu);
+            if constexpr (ALPHA) {
+                const double a = fmaxF(A.alpha, B.alpha);
+                d = d * a;
+                mu = mu * a;
+            }
+        }
+        const double uj[3] = {J.h, J.qx, J.qy};
+        stage_entry<SMB, 3>(r, fix, ui, uj, I.z, J.z, c, v1i, v2i, v1j, v2j, Hij, Hji, ratij, ratji, d, mu, off, K);
+    }
+    const double mi = M.m[i];
+    add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, r[1], r[2]);
+    for (int k = 0; k < 3; ++k) r[k] = r[k] / mi;
+    const Node o{stage_depth<SMB>(I.h, dt, fix, mi, r[0]), I.qx + dt * r[1], I.qy + dt * r[2], I.z};
+    stage_out(o, M, T[inst], Uo, out, i, stage, bdy);
+    raise_flag(flags_out, inst, err);
+}
+
+// =============================================================================================
+// SGN stage on tiles: k_stage_sgn's update.  pTilde (two divisions and a square root) is one of the staged
+// terms, once per node.
+// =============================================================================================
+struct alignas(16) SgnNode {
+    double h, z, qx, qy, ovh, sq, q, alpha, he, hw, pt, pad;
+};
+
+template <int SMB, bool ALPHA, bool D0>
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const NodeX* __restrict__ UX,
+           const Node* __restrict__ Uo, const NodeX* __restrict__ UoX, Node* __restrict__ out, NodeX* __restrict__ outX,
+           const double* __restrict__ d0, const double* __restrict__ alpha, int stage, int bdy,
+           int* __restrict__ flags_out, int remap) {
+    constexpr bool VISC = SMB != SMB_GALERKIN;
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    SgnNode* nodes = (SgnNode*)smem;
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const Consts K = T[inst].K;
+    const double dt = T[inst].dt;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    double2 c_next{};
+    int l_next = 0;
+    double d_next = 0.0;
+    if (len > 0) {
+        c_next = M.c[pb];
+        l_next = M.lcol[pb];
+        if constexpr (VISC && D0) d_next = ld_entry1(d0 + pb);
+    }
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
+        const NodeX X = UX[row];
+        nodes[k] = SgnNode{A.h, A.z, A.qx, A.qy, ovh_of(A.h, K.htiny),
+                           (VISC && !D0) ? sqrt_rn(K.g * fabs(A.h)) : 0.0, own_ratio(A.h, A.z),
+                           ALPHA ? alpha[row] : 0.0, X.he, X.hw, sgn_ptilde(A.h, X.he, M.m[row], K), 0.0};
+    };
+    if (len > 0) put(tid, i);
+    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    __syncthreads();
+    if (len == 0) return;
+    const Rcp r16 = uniform_rcp(K.g16);
+    const SgnNode& A = nodes[tid];
+    const Node I{A.h, A.qx, A.qy, A.z};
+    const double ovh_i = A.ovh, sql = A.sq, qi = A.q, ai = A.alpha;
+    const double v1i = I.qx * ovh_i, v2i = I.qy * ovh_i;
+    const double v2fi = I.qy * ovh_i * 0.0;   // velocity(2,i) of the model's flux
+    const double thr = (SMB == SMB_ROUNDOFF || SMB == SMB_1) ? K.htiny : 0.0;
+    const double ui[5] = {I.h, I.qx, I.qy, A.he, A.hw};
+    double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, fix = 0.0;
+    int err = 0;
+    for (int q = 0; q < len; ++q) {
+        const int64_t p = pb + 64 * (int64_t)q;
+        const double2 c = c_next;
+        const int l = l_next;
+        const double d0p = d_next;
+        if (q + 1 < len) {
+            c_next = M.c[p + 64];
+            l_next = M.lcol[p + 64];
+            if constexpr (VISC && D0) d_next = ld_entry1(d0 + p + 64);
+        }
+        const SgnNode& B = nodes[l];
+        const Node J{B.h, B.qx, B.qy, B.z};
+        const double v1j = J.qx * B.ovh, v2j = J.qy * B.ovh;
+        const double v2fj = J.qy * B.ovh * 0.0;
+        double Hij, Hji, ratij, ratji;
+        depth_ratios(I.h, I.z, qi, J.h, J.z, B.q, Hij, Hji, ratij, ratji);
+        ratij = (I.h <= thr) ? 0.0 : ratij;
+        ratji = (J.h <= thr) ? 0.0 : ratji;
+        const bool off = (l != tid);
+        double d = 0.0, mu = 0.0;
+        if (VISC && off) {
+            d = D0 ? d0p : dij_from_c(c, I, J, ovh_i, B.ovh, sql, B.sq, K, r16, err);
+            mu = mu_of(c.x, c.y, v1i, v2i, v1j, v2j);
+            d = fmaxF(d, mu);
+            if constexpr (ALPHA) {
+                const double a = fmaxF(ai, B.alpha);
+                d = d * a;
+                mu = mu * a;
+            }
+        }
+        const double uj[5] = {J.h, J.qx, J.qy, B.he, B.hw};
+        stage_entry<SMB, 5>(r, fix, ui, uj, I.z, J.z, c, v1i, v2fi, v1j, v2fj, Hij, Hji, ratij, ratji, d, mu, off, K);
+    }
+    // mSGN_RHS: the momenta lose pTilde(j)*c_ij over the row in CSR order, then the h*eta and h*w sources
+    for (int q = 0; q < len; ++q) {
+        const double2 c = M.c[pb + 64 * (int64_t)q];
+        const double pt = nodes[M.lcol[pb + 64 * (int64_t)q]].pt;
+        r[1] = r[1] - pt * c.x;
+        r[2] = r[2] - pt * c.y;
+    }
+    const double mi = M.m[i];
+    {
+        const double pc = K.lambda_sgn * K.g / (3.0 * sqrt_rn(mi));
+        const double x = ui[3] / (I.h * I.h);
+        const double psi = 12.0 * (x - 1.0);
+        const double t = ui[3] / I.h;
+        const double s = 3.0 * pc * (t * t) * psi;
+        r[3] = r[3] + mi * ui[4];
+        r[4] = r[4] - mi * s;
+    }
+    for (int k = 0; k < 5; ++k) r[k] = r[k] / mi;
+    const Node o{stage_depth<SMB>(I.h, dt, fix, mi, r[0]), I.qx + dt * r[1], I.qy + dt * r[2], I.z};
+    NodeX x{ui[3] + dt * r[3], ui[4] + dt * r[4]};
+    if (stage != 0) {
+        const NodeX PX = UoX[i];
+        x.he = rk_combine(stage, PX.he, x.he);
+        x.hw = rk_combine(stage, PX.hw, x.hw);
+    }
+    outX[i] = x;
+    stage_out(o, M, T[inst], Uo, out, i, stage, bdy);
+    raise_flag(flags_out, inst, err);
+}
+
+// =============================================================================================
+// Entropy-viscosity-only stage, pass 2 on tiles: k_ev_update's update.
+// =============================================================================================
+template <bool HAS_SRC>
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const Node* __restrict__ Uo,
+          Node* __restrict__ out, const double2* __restrict__ dmu, const double* __restrict__ res, int roundoff,
+          int stage, int bdy, int* __restrict__ flags_out, int remap) {
+    const int R = (int)blockDim.x;
+    extern __shared__ double smem[];
+    StageNode* nodes = (StageNode*)smem;     // alpha holds the residual, sq is unused
+    const int s0 = block_tile(M, remap);
+    const SliceInfo S = M.sl[s0];
+    const int inst = S.inst;
+    if (inst < 0 || !T[inst].go) return;
+    const Consts K = T[inst].K;
+    const double dt = T[inst].dt;
+    const int tid = (int)threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = s0 * 64 + tid;
+    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    double2 c_next{}, lo_next{};
+    int l_next = 0;
+    if (len > 0) {
+        c_next = ld_entry(M.c + pb);
+        lo_next = ld_entry(dmu + pb);
+        l_next = M.lcol[pb];
+    }
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
+        nodes[k] = StageNode{A.h, A.z, A.qx, A.qy, ovh_of(A.h, K.htiny), 0.0, own_ratio(A.h, A.z), res[row]};
+    };
+    if (len > 0) put(tid, i);
+    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    __syncthreads();
+    if (len == 0) return;
+    const StageNode A = nodes[tid];
+    const Node I{A.h, A.qx, A.qy, A.z};
+    const double v1i = I.qx * A.ovh, v2i = I.qy * A.ovh;
+    const double thr = roundoff ? K.htiny : 0.0;
+    const double ui[3] = {I.h, I.qx, I.qy};
+    double r[3] = {0.0, 0.0, 0.0}, fix = 0.0;
+    for (int q = 0; q < len; ++q) {
+        const int64_t p = pb + 64 * (int64_t)q;
+        const double2 c = c_next, lo = lo_next;
+        const int l = l_next;
+        if (q + 1 < len) {
+            c_next = ld_entry(M.c + p + 64);
+            lo_next = ld_entry(dmu + p + 64);
+            l_next = M.lcol[p + 64];
+        }
+        const StageNode& B = nodes[l];
+        const Node J{B.h, B.qx, B.qy, B.z};
+        const double v1j = J.qx * B.ovh, v2j = J.qy * B.ovh;
+        double Hij, Hji, ratij, ratji;
+        depth_ratios(I.h, I.z, A.q, J.h, J.z, B.q, Hij, Hji, ratij, ratji);
+        ratij = (I.h <= thr) ? 0.0 : ratij;
+        ratji = (J.h <= thr) ? 0.0 : ratji;
+        const bool off = (l != tid);
+        double d = 0.0, mu = 0.0;
+        if (off) {
+            const double rij = fmaxF(A.alpha, B.alpha);
+            d = fminF(lo.x, 1.0 * rij);
+            mu = fminF(lo.y, 1.0 * rij);
+        }
+        const double uj[3] = {J.h, J.qx, J.qy};
+        if (roundoff)
+            stage_entry<SMB_ROUNDOFF, 3>(r, fix, ui, uj, I.z, J.z, c, v1i, v2i, v1j, v2j, Hij, Hji, ratij, ratji, d, mu,
+                                         off, K);
+        else
+            stage_entry<SMB_2, 3>(r, fix, ui, uj, I.z, J.z, c, v1i, v2i, v1j, v2j, Hij, Hji, ratij, ratji, d, mu, off, K);
+    }
+    const double mi = M.m[i];
+    add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, r[1], r[2]);
+    for (int k = 0; k < 3; ++k) r[k] = r[k] / mi;
+    const double h = roundoff ? stage_depth<SMB_ROUNDOFF>(I.h, dt, fix, mi, r[0]) : stage_depth<SMB_2>(I.h, dt, fix, mi, r[0]);
+    const Node o{h, I.qx + dt * r[1], I.qy + dt * r[2], I.z};
+    const int err = (K.check_h && h < 0.0) ? FLAG_NEG_H : 0;
+    stage_out(o, M, T[inst], Uo, out, i, stage, bdy);
     raise_flag(flags_out, inst, err);
 }
 
@@ -567,6 +936,52 @@ void go_tile_lo(Pool& P, const Node* U, const double* d0) {
     }
 }
 
+template <int SMB, bool ALPHA>
+void go_tile_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage, bool bdy) {
+    auto go = [&](auto src, auto has_d0) {
+        constexpr bool S = decltype(src)::value, D = decltype(has_d0)::value;
+        hipLaunchKernelGGL((k_tile_stage<SMB, ALPHA, S, D>), dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                           sizeof(StageNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U,
+                           Uo, out, d0, (const double*)P.alpha, stage, bdy ? 1 : 0, P.flags,
+                           P.tune.k[KID_STAGE_LO].remap);
+    };
+    using T_ = std::true_type;
+    using F_ = std::false_type;
+    constexpr bool visc = SMB != SMB_GALERKIN;
+    if (P.any_src) {
+        if (visc && d0) go(T_{}, std::bool_constant<visc>{});
+        else go(T_{}, F_{});
+    } else {
+        if (visc && d0) go(F_{}, std::bool_constant<visc>{});
+        else go(F_{}, F_{});
+    }
+}
+
+template <int SMB, bool ALPHA>
+void go_tile_sgn(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage, bool bdy) {
+    auto go = [&](auto has_d0) {
+        constexpr bool D = decltype(has_d0)::value;
+        hipLaunchKernelGGL((k_tile_sgn<SMB, ALPHA, D>), dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                           sizeof(SgnNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U,
+                           (const NodeX*)ext_of(P, U), Uo, (const NodeX*)ext_of(P, Uo), out, ext_of(P, out), d0,
+                           (const double*)P.alpha, stage, bdy ? 1 : 0, P.flags, P.tune.k[KID_STAGE_LO].remap);
+    };
+    constexpr bool visc = SMB != SMB_GALERKIN;
+    if (visc && d0) go(std::bool_constant<visc>{});
+    else go(std::false_type{});
+}
+
+template <int SMB>
+void go_tile_first(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy) {
+    if (P.mode.sgn) {
+        if (alpha) go_tile_sgn<SMB, SMB != SMB_GALERKIN>(P, U, Uo, out, d0, stage, bdy);
+        else go_tile_sgn<SMB, false>(P, U, Uo, out, d0, stage, bdy);
+    } else {
+        if (alpha) go_tile_stage<SMB, SMB != SMB_GALERKIN>(P, U, Uo, out, d0, stage, bdy);
+        else go_tile_stage<SMB, false>(P, U, Uo, out, d0, stage, bdy);
+    }
+}
+
 }  // namespace
 
 void launch_tile_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo) {
@@ -598,6 +1013,32 @@ void launch_tile_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
     hipLaunchKernelGGL(k_tile_dt, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
                        sizeof(DtNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), P.tab, U, d0, P.vmax, P.flags,
                        P.done, all, advance ? 1 : 0, P.ninst(), P.tune.k[KID_DT].remap);
+}
+
+static_assert(sizeof(LoNode) * kTileNodes <= 65536, "a tile's records fit a workgroup's LDS");
+
+// The SGN records are longer than the others: pools with a longer halo keep the gather kernel.
+bool tile_stage_applies(const Pool& P) {
+    return tiles_apply(P) && (!P.mode.sgn || sizeof(SgnNode) * (size_t)P.tile_nodes <= 65536);
+}
+
+void launch_tile_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy) {
+    const Mode& md = P.mode;
+    if (md.viscosity_type == SWE_GALERKIN) go_tile_first<SMB_GALERKIN>(P, U, Uo, out, d0, false, stage, bdy);
+    else if (md.viscous_type == 1) go_tile_first<SMB_1>(P, U, Uo, out, d0, alpha, stage, bdy);
+    else if (md.roundoff) go_tile_first<SMB_ROUNDOFF>(P, U, Uo, out, d0, alpha, stage, bdy);
+    else go_tile_first<SMB_2>(P, U, Uo, out, d0, alpha, stage, bdy);
+}
+
+void launch_tile_ev(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy) {
+    auto go = [&](auto src) {
+        hipLaunchKernelGGL((k_tile_ev<decltype(src)::value>), dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                           sizeof(StageNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U,
+                           Uo, out, (const double2*)P.dmu, (const double*)P.res, P.mode.roundoff, stage, bdy ? 1 : 0,
+                           P.flags, P.tune.k[KID_EV].remap);
+    };
+    if (P.any_src) go(std::true_type{});
+    else go(std::false_type{});
 }
 
 }  // namespace swe
