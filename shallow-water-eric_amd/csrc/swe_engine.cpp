@@ -851,6 +851,7 @@ int pool_update_active(Pool* P) {
     std::vector<std::pair<int64_t, int64_t>> runs;
     P->any_src = false;
     P->any_bc_values = false;
+    P->one = -1;
     bool tiles = true;
     int max_halo = 0;
     for (int k = 0; k < P->inst_cap; ++k)
@@ -859,6 +860,7 @@ int pool_update_active(Pool* P) {
             tiles &= P->inst[(size_t)k].max_halo >= 0;
             max_halo = std::max(max_halo, P->inst[(size_t)k].max_halo);
             runs.emplace_back(P->inst[(size_t)k].slice0, P->inst[(size_t)k].nslices);
+            P->one = (runs.size() == 1) ? k : -1;
             Consts K;
             if (make_consts(P->inst[(size_t)k].prm, K) == SWE_OK && K.src != SRC_NONE) P->any_src = true;
         }
@@ -1007,11 +1009,12 @@ int64_t tuning_hash(const Tuning& t) {
 
 // The captured step stays valid while the launch extents, the scheme and the schedules stay.
 int ensure_graph(Pool* P) {
-    const int64_t key[6] = {(int64_t)P->nact * 2048 + (P->ntile > 0 ? P->tile_nodes : 0) * 2 + (P->any_bc_values ? 1 : 0), (int64_t)P->ninst(), P->nbc(), (int64_t)P->wmax,
+    const int64_t key[7] = {(int64_t)P->nact * 2048 + (P->ntile > 0 ? P->tile_nodes : 0) * 2 + (P->any_bc_values ? 1 : 0), (int64_t)P->ninst(), P->nbc(), (int64_t)P->wmax,
                             (int64_t)(P->mode.viscosity_type * 128 + P->mode.viscous_type * 16 + P->mode.alpha * 4 +
                                       P->mode.roundoff * 2 + (P->any_src ? 1 : 0)),
-                            tuning_hash(P->tune)};
-    if (P->gexec && std::equal(key, key + 6, P->graph_key)) return SWE_OK;
+                            tuning_hash(P->tune),
+                            (P->one < 0) ? -1 : (int64_t)P->one * (1ll << 32) + P->inst[(size_t)P->one].slice0};
+    if (P->gexec && std::equal(key, key + 7, P->graph_key)) return SWE_OK;
     if (P->gexec) {
         (void)hipGraphExecDestroy(P->gexec);
         P->gexec = nullptr;
@@ -1031,7 +1034,7 @@ int ensure_graph(Pool* P) {
         P->gexec = nullptr;
         return fail(SWE_EHIP, "hipGraphInstantiate: %s", hipGetErrorString(ei));
     }
-    std::copy(key, key + 6, P->graph_key);
+    std::copy(key, key + 7, P->graph_key);
     return SWE_OK;
 }
 

@@ -161,6 +161,7 @@ struct Pool {
     int* tact = nullptr;                     // first slices of their tiles, when every listed instance
     int ntile = 0;                           // can be tiled (else 0: the gather kernels run)
     int tile_nodes = 0;                      // their largest rows + halo: the LDS records of a workgroup
+    int one = -1;                            // the only listed instance, or -1
     std::vector<char> listed;                // per instance: its slices are in the list
     bool any_bc_values = false;              // a listed instance's boundary program takes given values (k_bdy)
     bool any_src = false;                    // a listed instance has a source term (type_test)
@@ -198,7 +199,7 @@ struct Pool {
     unsigned* bar = nullptr;          // the persistent step's barrier word and abort word
     bool use_graph = false;
     hipGraphExec_t gexec = nullptr;
-    int64_t graph_key[6] = {-1, -1, -1, -1, -1, -1};
+    int64_t graph_key[7] = {-1, -1, -1, -1, -1, -1, -1};
     bool timing = false;
     std::string timed_name;
     TimedKernel tk;

@@ -1439,8 +1439,9 @@ bool block_supported(int kid, int block) {
 }
 
 Mesh mesh_view(const Pool& P) {
-    return Mesh{P.sl,   P.len,  P.col,   P.dcol, P.c,    P.m,   P.elist, P.dpos,
-                P.dirm, P.lcol, P.halo, P.tact, P.ntile, P.act, P.nact, P.wmax};
+    const InstHost* one = (P.one >= 0) ? &P.inst[(size_t)P.one] : nullptr;
+    return Mesh{P.sl,     P.len,  P.col,  P.dcol, P.c,     P.m,   P.elist, P.dpos, P.dirm, P.lcol, P.halo, P.tact,
+                P.ntile,  P.one,  one ? (int)one->slice0 : 0,    one ? (int)one->nslices : 0, P.act, P.nact, P.wmax};
 }
 
 bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {

@@ -123,6 +123,8 @@ struct Mesh {
     const int* __restrict__ halo;       // halo lists of the tiles (global rows)
     const int* __restrict__ tact;       // first slices of the tiles a launch covers, ascending
     int ntile;                          // number of them
+    int one, one_slice0, one_nsl;       // the instance, first slice and slices of a launch over one instance;
+                                        // one = -1: the lists tell
     const int* __restrict__ act;        // the slices a launch covers, ascending (one wave each)
     int nact;                           // number of them
     int wmax;                           // longest row of the resident instances

@@ -21,9 +21,60 @@ namespace swe {
 
 namespace {
 
-// First slice of this workgroup's tile.
-__device__ __forceinline__ int block_tile(const Mesh& M, int remap) {
-    return __builtin_amdgcn_readfirstlane(M.tact[remap ? xcd_block() : (int)blockIdx.x]);
+// What every kernel reads first.  On a small mesh a kernel's time is the chain of dependent loads (about 0.7 us
+// each, nothing being cached across a launch), so all that can be is loaded without waiting for anything
+// else: a launch over one instance knows its slices and instance from its arguments, the row's data, the
+// halo's rows and the instance's record are loaded side by side, and whether the instance steps at all
+// decides afterwards (by emptying the rows) what happens to them.
+struct TileHead {
+    int s0, nsl;          // first slice and slices of the tile
+    int inst;             // its instance
+    int tid, w, i;        // thread, wave, global row (of the tile's last slice for waves past it)
+    bool own;             // the wave has a slice of the tile
+    int len, nhalo;       // entries of the row (0 past the tile), rows of the halo
+    int64_t pb;           // first slot of the row
+    int64_t hbase;        // start of the halo list
+    int hrow;             // this thread's first row of the halo (if it has one)
+};
+__device__ __forceinline__ TileHead tile_head(const Mesh& M, int remap) {
+    TileHead h;
+    const int b = remap ? xcd_block() : (int)blockIdx.x;
+    const int ts = (int)(blockDim.x >> 6);
+    h.tid = (int)threadIdx.x;
+    h.w = __builtin_amdgcn_readfirstlane(h.tid >> 6);
+    SliceInfo S;
+    if (M.one >= 0) {
+        h.s0 = M.one_slice0 + b * ts;
+        const int left = M.one_nsl - b * ts;
+        h.nsl = (left < ts) ? left : ts;
+        h.inst = M.one;
+        S = M.sl[h.s0];
+    } else {
+        h.s0 = __builtin_amdgcn_readfirstlane(M.tact[b]);
+        S = M.sl[h.s0];
+        h.nsl = S.tile_slices;
+        h.inst = S.inst;
+    }
+    h.nhalo = S.nhalo;
+    h.own = h.w < h.nsl;
+    const int sw = h.own ? h.s0 + h.w : h.s0 + h.nsl - 1;
+    h.i = sw * 64 + (h.tid & 63);
+    h.len = M.len[h.i];
+    h.hbase = (int64_t)h.s0 * kHaloStride;
+    h.hrow = M.halo[h.hbase + (h.tid < kHaloStride ? h.tid : kHaloStride - 1)];
+    h.pb = M.sl[sw].sbase + (h.tid & 63);
+    if (!h.own) h.len = 0;
+    return h;
+}
+// put(k, row) for the nodes of the tile: k = 0..rows-1 its rows (padding rows of its slices too), then its halo.
+template <class F>
+__device__ __forceinline__ void stage_nodes(const TileHead& h, const Mesh& M, bool go, F&& put) {
+    const int R = (int)blockDim.x;
+    if (h.own) put(h.tid, h.i);
+    if (go) {
+        if (h.tid < h.nhalo) put(R + h.tid, h.tid < kHaloStride ? h.hrow : M.halo[h.hbase + h.tid]);
+        for (int k = h.tid + R; k < h.nhalo; k += R) put(R + k, M.halo[h.hbase + k]);
+    }
 }
 
 // MAX(0, h + zb - zb)/h, the depth ratio of a node against its own bed (smb_2: U_i's ratio where its bed is
@@ -176,22 +227,18 @@ k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, dou
           double2* __restrict__ ulo_q, double2* __restrict__ dmu, double* __restrict__ res,
           const double* __restrict__ d0, const double* __restrict__ alpha, int roundoff, int* __restrict__ flags_out,
           int remap) {
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     LoNode* nodes = (LoNode*)smem;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const Consts K = T[inst].K;
     const double dt = T[inst].dt;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
+    const int len = go ? h.len : 0;
     const double wet_h = fmaxF(K.htiny, 0.0);
     bool wet = true;
-    auto stage = [&](int k, const Node& A, int row) {
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
         LoNode n;
         n.h = A.h;
         n.z = A.z;
@@ -207,25 +254,18 @@ k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, dou
         n.E = 0.5 * E;
         n.alpha = ALPHA ? alpha[row] : 0.0;
         nodes[k] = n;
-        wet = wet && A.h > wet_h;
+        // (padding rows of the tile's slices, which nothing refers to, do not count)
+        wet = wet && (A.h > wet_h || (k == tid && len == 0));
     };
-    Node I{};
-    if (len > 0) {
-        I = U[i];
-        stage(tid, I, i);
-    }
-    for (int k = tid; k < S.nhalo; k += R) {
-        const int j = M.halo[(int64_t)s0 * kHaloStride + k];
-        stage(R + k, U[j], j);
-    }
+    stage_nodes(h, M, go, put);
     const bool all_wet = __syncthreads_and(wet ? 1 : 0) != 0;
     if (len == 0) return;
     const Rcp r16 = uniform_rcp(K.g16);
-    const int64_t pb = M.sl[s0 + w].sbase + (tid & 63);
+    const Node I{nodes[tid].h, nodes[tid].qx, nodes[tid].qy, nodes[tid].z};
     int err = 0;
     LoSums s;
-    if (all_wet) lo_rows<true, ALPHA, WRITE_LO, D0>(nodes, M, pb, len, I, K, r16, d0, dmu, roundoff, s, err);
-    else lo_rows<false, ALPHA, WRITE_LO, D0>(nodes, M, pb, len, I, K, r16, d0, dmu, roundoff, s, err);
+    if (all_wet) lo_rows<true, ALPHA, WRITE_LO, D0>(nodes, M, h.pb, len, I, K, r16, d0, dmu, roundoff, s, err);
+    else lo_rows<false, ALPHA, WRITE_LO, D0>(nodes, M, h.pb, len, I, K, r16, d0, dmu, roundoff, s, err);
     const double mi = M.m[i];
     const double ovh_i = nodes[tid].ovh;
     const double v1i = I.qx * ovh_i, v2i = I.qy * ovh_i;
@@ -315,28 +355,22 @@ __device__ __forceinline__ double tile_flux(const N& I, const N& J, const double
 __global__ void __launch_bounds__(64 * kMaxTileSlices)
 k_tile_rminus(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const double* __restrict__ ulo_h,
               const double2* __restrict__ dmu, const double* __restrict__ res, double* __restrict__ Rm, int remap) {
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     FluxNode* nodes = (FluxNode*)smem;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const double dt = T[inst].dt;
     const double htiny = T[inst].K.htiny;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    const int len = go ? h.len : 0;
+    const int64_t pb = h.pb;
     HeldRow H;
     hold_row(H, M, dmu, pb, len);
     auto stage = [&](int k, int row) {
         const Node A = U[row];
         nodes[k] = FluxNode{A.h, A.z, own_ratio(A.h, A.z), res[row]};
     };
-    if (len > 0) stage(tid, i);
-    for (int k = tid; k < S.nhalo; k += R) stage(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    stage_nodes(h, M, go, stage);
     __syncthreads();
     if (len == 0) return;
     const FluxNode I = nodes[tid];
@@ -367,28 +401,22 @@ k_tile_apply(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
              const double* __restrict__ ulo_h, const double2* __restrict__ ulo_q, Node* __restrict__ out,
              const double2* __restrict__ dmu, const double* __restrict__ res, const double* __restrict__ Rm, int stage,
              int bdy, int* __restrict__ flags_out, int remap) {
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     ApplyNode* nodes = (ApplyNode*)smem;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const double dt = T[inst].dt;
     const int check_h = T[inst].K.check_h;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    const int len = go ? h.len : 0;
+    const int64_t pb = h.pb;
     HeldRow H;
     hold_row(H, M, dmu, pb, len);
     auto put = [&](int k, int row) {
         const Node A = U[row];
         nodes[k] = ApplyNode{A.h, A.z, own_ratio(A.h, A.z), res[row], A.qx, A.qy, Rm[row], 0.0};
     };
-    if (len > 0) put(tid, i);
-    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    stage_nodes(h, M, go, put);
     __syncthreads();
     if (len == 0) return;
     const ApplyNode I = nodes[tid];
@@ -516,20 +544,15 @@ k_tile_stage(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
              Node* __restrict__ out, const double* __restrict__ d0, const double* __restrict__ alpha, int stage, int bdy,
              int* __restrict__ flags_out, int remap) {
     constexpr bool VISC = SMB != SMB_GALERKIN;
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     StageNode* nodes = (StageNode*)smem;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const Consts K = T[inst].K;
     const double dt = T[inst].dt;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    const int len = go ? h.len : 0;
+    const int64_t pb = h.pb;
     double2 c_next{};
     int l_next = 0;
     double d_next = 0.0;
@@ -544,8 +567,7 @@ k_tile_stage(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
                              (VISC && !D0) ? sqrt_rn(K.g * fabs(A.h)) : 0.0, own_ratio(A.h, A.z),
                              ALPHA ? alpha[row] : 0.0};
     };
-    if (len > 0) put(tid, i);
-    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    stage_nodes(h, M, go, put);
     __syncthreads();
     if (len == 0) return;
     const Rcp r16 = uniform_rcp(K.g16);
@@ -611,20 +633,15 @@ k_tile_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
            const double* __restrict__ d0, const double* __restrict__ alpha, int stage, int bdy,
            int* __restrict__ flags_out, int remap) {
     constexpr bool VISC = SMB != SMB_GALERKIN;
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     SgnNode* nodes = (SgnNode*)smem;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const Consts K = T[inst].K;
     const double dt = T[inst].dt;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    const int len = go ? h.len : 0;
+    const int64_t pb = h.pb;
     double2 c_next{};
     int l_next = 0;
     double d_next = 0.0;
@@ -640,8 +657,7 @@ k_tile_sgn(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, co
                            (VISC && !D0) ? sqrt_rn(K.g * fabs(A.h)) : 0.0, own_ratio(A.h, A.z),
                            ALPHA ? alpha[row] : 0.0, X.he, X.hw, sgn_ptilde(A.h, X.he, M.m[row], K), 0.0};
     };
-    if (len > 0) put(tid, i);
-    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    stage_nodes(h, M, go, put);
     __syncthreads();
     if (len == 0) return;
     const Rcp r16 = uniform_rcp(K.g16);
@@ -725,20 +741,15 @@ __global__ void __launch_bounds__(64 * kMaxTileSlices)
 k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, const Node* __restrict__ Uo,
           Node* __restrict__ out, const double2* __restrict__ dmu, const double* __restrict__ res, int roundoff,
           int stage, int bdy, int* __restrict__ flags_out, int remap) {
-    const int R = (int)blockDim.x;
     extern __shared__ double smem[];
     StageNode* nodes = (StageNode*)smem;     // alpha holds the residual, sq is unused
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    if (inst < 0 || !T[inst].go) return;
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
+    const bool go = T[inst].go != 0;
     const Consts K = T[inst].K;
     const double dt = T[inst].dt;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = s0 * 64 + tid;
-    const int len = (w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
+    const int len = go ? h.len : 0;
+    const int64_t pb = h.pb;
     double2 c_next{}, lo_next{};
     int l_next = 0;
     if (len > 0) {
@@ -750,8 +761,7 @@ k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, con
         const Node A = U[row];
         nodes[k] = StageNode{A.h, A.z, A.qx, A.qy, ovh_of(A.h, K.htiny), 0.0, own_ratio(A.h, A.z), res[row]};
     };
-    if (len > 0) put(tid, i);
-    for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    stage_nodes(h, M, go, put);
     __syncthreads();
     if (len == 0) return;
     const StageNode A = nodes[tid];
@@ -793,9 +803,9 @@ k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, con
     const double mi = M.m[i];
     add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, r[1], r[2]);
     for (int k = 0; k < 3; ++k) r[k] = r[k] / mi;
-    const double h = roundoff ? stage_depth<SMB_ROUNDOFF>(I.h, dt, fix, mi, r[0]) : stage_depth<SMB_2>(I.h, dt, fix, mi, r[0]);
-    const Node o{h, I.qx + dt * r[1], I.qy + dt * r[2], I.z};
-    const int err = (K.check_h && h < 0.0) ? FLAG_NEG_H : 0;
+    const Node o{roundoff ? stage_depth<SMB_ROUNDOFF>(I.h, dt, fix, mi, r[0]) : stage_depth<SMB_2>(I.h, dt, fix, mi, r[0]),
+                 I.qx + dt * r[1], I.qy + dt * r[2], I.z};
+    const int err = (K.check_h && o.h < 0.0) ? FLAG_NEG_H : 0;
     stage_out(o, M, T[inst], Uo, out, i, stage, bdy);
     raise_flag(flags_out, inst, err);
 }
@@ -817,32 +827,24 @@ k_tile_dt(Mesh M, InstDev* __restrict__ T, const Node* __restrict__ U, double* _
     DtNode* nodes = (DtNode*)smem;
     __shared__ unsigned long long red[kMaxTileSlices];
     __shared__ int last;
-    const int s0 = block_tile(M, remap);
-    const SliceInfo S = M.sl[s0];
-    const int inst = S.inst;
-    const int tid = (int)threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid, i = h.i;
     // (per wave: a check raised meanwhile may end some waves' part; every barrier is met by all of them)
-    const bool live = inst >= 0 && (all ? T[inst].state != INST_FREE : takes_steps(T[inst], flags[inst]));
-    const int i = s0 * 64 + tid;
-    const int len = (live && w < S.tile_slices) ? M.len[i] : 0;
-    const int64_t pb = M.sl[(w < S.tile_slices) ? s0 + w : s0].sbase + (tid & 63);
-    Consts K{};
+    const bool live = all ? T[inst].state != INST_FREE : takes_steps(T[inst], flags[inst]);
+    const int len = live ? h.len : 0;
+    const int64_t pb = h.pb;
+    const Consts K = T[inst].K;
     double2 c_next{};
     int l_next = 0;
-    if (live) {
-        K = T[inst].K;
-        if (len > 0) {
-            c_next = ld_entry(M.c + pb);
-            l_next = M.lcol[pb];
-        }
-        auto put = [&](int k, int row) {
-            const Node A = U[row];
-            nodes[k] = DtNode{A.h, A.qx, A.qy, ovh_of(A.h, K.htiny), sqrt_rn(K.g * fabs(A.h)), 0.0};
-        };
-        if (len > 0) put(tid, i);
-        for (int k = tid; k < S.nhalo; k += R) put(R + k, M.halo[(int64_t)s0 * kHaloStride + k]);
+    if (len > 0) {
+        c_next = ld_entry(M.c + pb);
+        l_next = M.lcol[pb];
     }
+    auto put = [&](int k, int row) {
+        const Node A = U[row];
+        nodes[k] = DtNode{A.h, A.qx, A.qy, ovh_of(A.h, K.htiny), sqrt_rn(K.g * fabs(A.h)), 0.0};
+    };
+    stage_nodes(h, M, live, put);
     __syncthreads();
     double v = 0.0;
     int err = 0;
