@@ -112,15 +112,14 @@ int swe_assembly_destroy(swe_assembly *a);
 
 /* Create a solver over one mesh: copies the mesh arrays to the device.  Replaces the module
  * state built by construct_matrices (SOURCES/update.f90:18-132) and construct_mesh.
- * The environment variable SWE_SORT_WINDOW (default 64) sets the window of rows inside which
- * the internal numbering sorts rows by length; SWE_REORDER (default 1) renumbers rows internally by
- * reverse Cuthill-McKee when the caller's numbering scatters neighbours (mean |i-j| above
- * 2*sqrt(np)), 0 never, 2 always.  These are layout choices; results do not depend on them. */
+ * The environment variable SWE_SORT_WINDOW (default: the rows of a tile, 64 to 256) sets the
+ * window of rows inside which the internal numbering sorts rows by length; SWE_REORDER=0 keeps the
+ * caller's numbering as the base order instead of a locality order of the mesh graph.  These are layout choices; results do not depend on them. */
 int swe_create(const swe_mesh_desc *mesh, const swe_params *prm, swe_handle **out);
 /* swe_create over a mesh assembled by swe_assemble_device, without taking the matrices to the
  * host: the solver's layout is built on the GPU from the assembly (rows sorted by length inside
- * 64-row windows of a base order: the caller's numbering, or under SWE_REORDER -- see swe_create --
- * the nodes sorted along a Hilbert curve of their coordinates), bath and the Dirichlet
+ * the tiles of a base order: the nodes sorted along a Hilbert curve of their coordinates,
+ * or the caller's numbering under SWE_REORDER=0), bath and the Dirichlet
  * lists (1-based, as in swe_mesh_desc) are copied from the host.  The solver does not keep the
  * assembly; results are bitwise those of swe_create on the same arrays.  This replaces, together
  * with swe_assemble_device, construct_matrices (SOURCES/update.f90:18-132, called at

@@ -229,7 +229,7 @@ int swe_create_from_assembly(const swe_assembly* a, const double* bath, int n_h_
     if ((rc = mode_of(*prm, md))) return rc;
     if ((rc = check_sgn_lists(md, n_ux_dir, n_uy_dir))) return rc;
     DeviceLayout DL;
-    if ((rc = build_layout_device(a, DL))) return rc;
+    if ((rc = build_layout_device(a, tile_slices_for(assembly_rows(a)), DL))) return rc;
     if (DL.nnz > INT_MAX) {
         free_device_layout(DL);
         return fail(SWE_EINVAL, "%lld entries do not fit the solver's 32-bit CSR", (long long)DL.nnz);
@@ -721,7 +721,7 @@ int swe_batch_add_assembled(swe_batch* b, const swe_assembly* a, const double* b
     if (!b || !a || !bath || !prm || !un || !id) return fail(SWE_EINVAL, "null argument");
     if (max_steps < 0) return fail(SWE_EINVAL, "max_steps < 0");
     DeviceLayout DL;
-    int rc = build_layout_device(a, DL);
+    int rc = build_layout_device(a, b->P->tile_slices, DL);
     if (rc) return rc;
     if (DL.nnz > INT_MAX) {
         free_device_layout(DL);

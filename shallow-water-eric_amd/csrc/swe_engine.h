@@ -79,7 +79,7 @@ int validate_mesh(const swe_mesh_desc& d);
 int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostLayout& L);
 // Slices per tile for a pool of `rows` rows.
 int tile_slices_for(int64_t rows);
-// Rows sorted by length inside windows of this many rows: SWE_SORT_WINDOW, else 64.
+// Rows sorted by length inside windows of this many rows: SWE_SORT_WINDOW, else 0 (a tile's rows).
 int sort_window_default();
 // SWE_REORDER: 0 keeps the caller's numbering as the base order; otherwise (default) rows are renumbered
 // for locality, so that tiles are compact.
@@ -130,7 +130,7 @@ struct Pool {
     hipEvent_t released = nullptr;    // recorded on `stream` when ranges are given back
     bool mode_set = false;
     Mode mode{};
-    int sort_window = 64;
+    int sort_window = 0;
     // capacities and allocators
     int64_t rows_cap = 0, slots_cap = 0, elist_cap = 0, bc_cap = 0;
     int inst_cap = 0;
@@ -253,7 +253,7 @@ int pool_tune(Pool* P, int steps, int trials);
 
 // ---- layout of a mesh assembled on the device (swe_setup_device.hip) --------------------------
 // The same internal numbering and sliced layout build_layout makes on the host (rows sorted by
-// length inside 64-row windows of the caller's numbering), computed on the GPU from an assembly.
+// length inside the rows of each tile), computed on the GPU from an assembly.
 struct DeviceLayout {
     int np = 0, nsl = 0, wmax = 0;
     int64_t nnz = 0, nslot = 0, ne = 0;
@@ -264,7 +264,8 @@ struct DeviceLayout {
     int64_t* eoff = nullptr;   // compact-list offset of each slice (nsl + 1)
     hipStream_t stream = nullptr;   // the assembly's stream: the buffers are allocated and freed on it
 };
-int build_layout_device(const swe_assembly* a, DeviceLayout& DL);
+int64_t assembly_rows(const swe_assembly* a);      // its nodes, rounded up to slices
+int build_layout_device(const swe_assembly* a, int tile_slices, DeviceLayout& DL);
 void free_device_layout(DeviceLayout& DL);
 // Admit an assembled mesh with its device layout; bath(np) and the 1-based Dirichlet lists are host
 // arrays; csr2slot (may be null) receives the slot of each CSR entry, relative to the instance.

@@ -331,8 +331,7 @@ extern "C" int swe_assembly_destroy(swe_assembly* a) {
 
 // =============================================================================================
 // The sliced layout of an assembled mesh, built on the GPU (the same internal numbering and slots
-// as build_layout on the host: rows stably sorted by length inside each 64-row window of the
-// caller's numbering, one 64-row slice per window).
+// as build_layout on the host: rows stably sorted by length inside each tile's rows of the base order).
 // =============================================================================================
 namespace {
 
@@ -344,23 +343,20 @@ __global__ void k_lay_len(int np, const int64_t* __restrict__ ia0, int* __restri
     if (l > swe::kMaxRow || l < 1) atomicOr(bad, 1);
 }
 
-// One wave per window of the base order (base[p], or p when base is null): each lane's rank among
-// the window's valid rows by (length, position in the base order).
-__global__ void k_lay_sort(int np, int nwin, const int* __restrict__ lenc, const int* __restrict__ base,
-                           int* __restrict__ perm) {
-    const int w = (int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
-    const int pos = w * 64 + lane;
-    const bool valid = w < nwin && pos < np;
-    const int i = valid ? (base ? base[pos] : pos) : 0;
-    const int li = valid ? lenc[i] : 0x7fffffff;
+// One workgroup per tile, one thread per row of it in the base order (base[p], or p when base is null): each
+// row's rank among the tile's by (length, position in the base order).
+__global__ void __launch_bounds__(64 * swe::kMaxTileSlices)
+k_lay_sort(int np, const int* __restrict__ lenc, const int* __restrict__ base, int* __restrict__ perm) {
+    __shared__ int key[64 * swe::kMaxTileSlices];
+    const int n = (int)blockDim.x, k = (int)threadIdx.x;
+    const int w0 = (int)blockIdx.x * n, pos = w0 + k;
+    const int i = (pos < np) ? (base ? base[pos] : pos) : 0;
+    const int mine = (pos < np) ? lenc[i] * n + k : 0x7fffffff;
+    key[k] = mine;
+    __syncthreads();
     int rank = 0;
-    for (int m = 0; m < 64; ++m) {
-        const int lm = __shfl(li, m, 64);
-        const bool vm = w < nwin && (w * 64 + m) < np;
-        rank += (vm && (lm < li || (lm == li && m < lane))) ? 1 : 0;
-    }
-    if (valid) perm[w * 64 + rank] = i;
+    for (int m = 0; m < n; ++m) rank += (key[m] < mine) ? 1 : 0;
+    if (pos < np) perm[w0 + rank] = i;
 }
 
 // ---- locality order: nodes sorted along a Hilbert curve of their coordinates ------------------
@@ -699,7 +695,9 @@ void free_device_layout(DeviceLayout& DL) {
     DL = DeviceLayout{};
 }
 
-int build_layout_device(const swe_assembly* a, DeviceLayout& DL) {
+int64_t assembly_rows(const swe_assembly* a) { return ((int64_t)a->np + 63) / 64 * 64; }
+
+int build_layout_device(const swe_assembly* a, int tile_slices, DeviceLayout& DL) {
     if (!a) return fail(SWE_EINVAL, "null assembly");
     DL = DeviceLayout{};
     const int np = a->np;
@@ -729,8 +727,8 @@ int build_layout_device(const swe_assembly* a, DeviceLayout& DL) {
     int hflag[2] = {0, 0};
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_lay_len, dim3(grid_of(np, 256)), dim3(256), 0, s, np, (const int64_t*)a->ia0, lenc, flag);
-        hipLaunchKernelGGL(k_lay_sort, dim3(grid_of(nsl, 4)), dim3(256), 0, s, np, nsl, (const int*)lenc,
-                           (const int*)base, DL.perm);
+        hipLaunchKernelGGL(k_lay_sort, dim3(grid_of(nsl, tile_slices)), dim3(64 * tile_slices), 0, s, np,
+                           (const int*)lenc, (const int*)base, DL.perm);
         hipLaunchKernelGGL(k_lay_iperm, dim3(grid_of(np_pad, 256)), dim3(256), 0, s, np, np_pad, (const int*)DL.perm,
                            (const int*)lenc, DL.iperm, DL.len);
         hipLaunchKernelGGL(k_lay_slices, dim3(grid_of(nsl, 256)), dim3(256), 0, s, nsl, np, (const int*)DL.len, slots,
