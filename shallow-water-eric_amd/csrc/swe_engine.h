@@ -284,7 +284,7 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
 // ---- launch wrappers (swe_kernels.hip) --------------------------------------------------------
 Mesh mesh_view(const Pool& P);
 // COMPUTE_DT's pass; true when it did the step's bookkeeping too (advance, on tiles), which otherwise is
-// launch_finalize_dt's.
+// launch_finalize_dt's.  With advance on tiles it also leaves the alpha factors at U in P.alpha.
 bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance);
 void launch_finalize_dt(Pool& P, int advance);
 // The tile form of k_fct_lo (swe_tiles.hip), where tiles_apply.
@@ -295,8 +295,18 @@ bool tile_stage_applies(const Pool& P);
 void launch_tile_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy);
 void launch_tile_ev(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
 void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
-// The dt pass on tiles; advance: the last workgroup also does finalize_one for every instance.
-void launch_tile_dt(Pool& P, const Node* U, double* d0, int all, bool advance);
+// The dt pass on tiles; alpha (may be null) receives the alpha limiter's factors at U; advance: the last
+// workgroup also does finalize_one for every instance.
+void launch_tile_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance);
+// The same passes with four lanes per row (swe_quads.hip), where tiles_apply and quads_apply.  k_quad_lo and
+// k_quad_stage compute the alpha factors themselves unless d0 says that the dt pass has.
+bool quads_apply(const Pool& P);
+void launch_quad_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo);
+void launch_quad_rminus(Pool& P, const Node* U);
+void launch_quad_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
+void launch_quad_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy);
+void launch_quad_ev(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
+void launch_quad_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance);
 int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage,
                        bool bdy = false);
 // Whether launch_euler_stage can write the wall and inflow values itself (given values need launch_bdy).

@@ -1444,12 +1444,18 @@ Mesh mesh_view(const Pool& P) {
                 P.ntile,  P.one,  one ? (int)one->slice0 : 0,    one ? (int)one->nslices : 0, P.act, P.nact, P.wmax};
 }
 
+namespace {
+bool alpha_used(const Mode& md) { return md.alpha != 0 && md.viscosity_type != SWE_GALERKIN; }
+}  // namespace
+
 bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return false;
     if (tiles_apply(P)) {
         timed_begin(P, KID_DT);
-        launch_tile_dt(P, U, d0, all, advance);
+        double* const al = (advance && alpha_used(P.mode)) ? P.alpha : nullptr;
+        if (quads_apply(P)) launch_quad_dt(P, U, d0, al, all, advance);
+        else launch_tile_dt(P, U, d0, al, all, advance);
         timed_end(P, KID_DT);
         return advance;
     }
@@ -1483,8 +1489,10 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return SWE_OK;
     const InstDev* T = P.tab;
-    const bool alpha = md.alpha != 0 && md.viscosity_type != SWE_GALERKIN;
-    if (alpha) {
+    const bool alpha = alpha_used(md);
+    const bool quads = tiles_apply(P) && quads_apply(P) && !md.sgn;
+    // on tiles the dt pass that gave d0 gave alpha too, and four lanes per row compute it where they stage
+    if (alpha && !quads && !(d0 && tiles_apply(P))) {
         const LaunchCfg& L = P.tune.k[KID_ALPHA];
         timed_begin(P, KID_ALPHA);
         SWE_BS_SWITCH(L.block, hipLaunchKernelGGL((k_alpha<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0, P.stream,
@@ -1495,7 +1503,8 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
         return fail(SWE_EINVAL, "SGN stage on a buffer without h*eta, h*w");
     if ((md.viscosity_type == SWE_GALERKIN || md.viscosity_type == SWE_VISCOUS) && tile_stage_applies(P)) {
         timed_begin(P, KID_STAGE_LO);
-        launch_tile_stage(P, U, Uo, out, d0, alpha, stage, bdy);
+        if (quads) launch_quad_stage(P, U, Uo, out, d0, alpha, stage, bdy);
+        else launch_tile_stage(P, U, Uo, out, d0, alpha, stage, bdy);
         timed_end(P, KID_STAGE_LO);
     } else if (md.sgn) {
         // the SGN model (first-order and galerkin schemes only)
@@ -1544,16 +1553,19 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
         timed_end(P, KID_STAGE_LO);
     } else if (md.viscosity_type == SWE_FCT) {
         timed_begin(P, KID_FCT_LO);
-        if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, true);
+        if (quads) launch_quad_lo(P, U, d0, alpha, true);
+        else if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, true);
         else if (alpha) launch_fct_lo<true, true>(P, U, d0);
         else launch_fct_lo<false, true>(P, U, d0);
         timed_end(P, KID_FCT_LO);
         if (tiles_apply(P)) {
             timed_begin(P, KID_RMINUS);
-            launch_tile_rminus(P, U);
+            if (quads) launch_quad_rminus(P, U);
+            else launch_tile_rminus(P, U);
             timed_end(P, KID_RMINUS);
             timed_begin(P, KID_APPLY);
-            launch_tile_apply(P, U, Uo, out, stage, bdy);
+            if (quads) launch_quad_apply(P, U, Uo, out, stage, bdy);
+            else launch_tile_apply(P, U, Uo, out, stage, bdy);
             timed_end(P, KID_APPLY);
         } else {
             const LaunchCfg& L = P.tune.k[KID_RMINUS];
@@ -1571,11 +1583,14 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
             timed_end(P, KID_APPLY);
         }
     } else {  // entropy_visc
-        if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, false);
+        if (quads) launch_quad_lo(P, U, d0, alpha, false);
+        else if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, false);
         else if (alpha) launch_fct_lo<true, false>(P, U, d0);
         else launch_fct_lo<false, false>(P, U, d0);
         timed_begin(P, KID_EV);
-        if (tiles_apply(P)) {
+        if (quads) {
+            launch_quad_ev(P, U, Uo, out, stage, bdy);
+        } else if (tiles_apply(P)) {
             launch_tile_ev(P, U, Uo, out, stage, bdy);
         } else {
             const LaunchCfg& L = P.tune.k[KID_EV];

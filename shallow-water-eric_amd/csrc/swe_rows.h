@@ -161,10 +161,21 @@ __device__ __forceinline__ void first_order_dmu(const double2 c, double v1i, dou
     }
 }
 
+// alpha_i from its row sums num = sum(h_j - h_i), denom = sum|h_j - h_i|.
+__device__ __forceinline__ double alpha_value(double num, double denom, double hi, double htiny) {
+    double a = 1.0;
+    if (!(hi <= htiny)) {
+        if (!(denom <= fabs(num))) a = fabs(num) / (denom);
+        a = a * a;
+        a = a * a;
+        a = a * a;
+    }
+    return a;
+}
+
 // alpha_limit, first loop (update.f90:758-781) for row i: alpha_i = (|sum(h_j-h_i)| /
 // sum|h_j-h_i|)**8, 1 if h_i <= htiny or the denominator does not exceed the numerator.  All index
-// loads, then all gathers, then the sums in entry order.  (Evaluating it inside the dt pass for
-// stage 1 was measured slower than this separate sweep: the gathers after the LDS phase stall.)
+// loads, then all gathers, then the sums in entry order.
 __device__ __forceinline__ double alpha_of(const Mesh& M, const Node* __restrict__ U, int i, double hi, double htiny) {
     double a = 1.0;
     if (!(hi <= htiny)) {
@@ -192,11 +203,7 @@ __device__ __forceinline__ double alpha_of(const Mesh& M, const Node* __restrict
             num = num + hj - hi;
             denom = denom + fabs(hj - hi);
         }
-        if (denom <= fabs(num)) a = 1.0;
-        else a = fabs(num) / (denom);
-        a = a * a;
-        a = a * a;
-        a = a * a;
+        a = alpha_value(num, denom, hi, htiny);
     }
     return a;
 }

@@ -15,7 +15,7 @@
 
 #include "swe_engine.h"
 #include "swe_kernels.h"
-#include "swe_rows.h"
+#include "swe_tile.h"
 
 namespace swe {
 
@@ -76,36 +76,6 @@ __device__ __forceinline__ void stage_nodes(const TileHead& h, const Mesh& M, bo
         for (int k = h.tid + R; k < h.nhalo; k += R) put(R + k, M.halo[h.hbase + k]);
     }
 }
-
-// MAX(0, h + zb - zb)/h, the depth ratio of a node against its own bed (smb_2: U_i's ratio where its bed is
-// the higher one).
-__device__ __forceinline__ double own_ratio(double h, double z) { return fmaxF(0.0, h + z - z) / h; }
-
-// The depth ratios of an entry before the dry-node rule: qij = MAX(0, h_i + z_i - zmax)/h_i, qji likewise
-// for j, zmax = MAX(z_i, z_j); qi, qj are own_ratio of the two nodes.
-__device__ __forceinline__ void depth_ratios(double hi, double zi, double qi, double hj, double zj, double qj,
-                                             double& Hij, double& Hji, double& qij, double& qji) {
-    const bool up = zi > zj;
-    const double zmax = up ? zi : zj;
-    Hij = fmaxF(0.0, hi + zi - zmax);
-    Hji = fmaxF(0.0, hj + zj - zmax);
-    const double quo = (up ? Hji : Hij) / (up ? hj : hi);
-    qij = up ? qi : quo;
-    qji = up ? quo : qj;
-}
-
-// Sums of one row over its entries, for lo_finish.
-struct LoSums {
-    double r1, r2, r3, fix, e1, e2, e3, emax, emin;
-};
-
-// What k_tile_lo stages per node: 80 bytes, read in 16-byte pieces.
-struct alignas(16) LoNode {
-    double h, z, qx, qy;
-    double ovh, sq;       // one_over_h, SQRT(g*ABS(h))
-    double q, E;          // own_ratio, entropy
-    double alpha, pad;
-};
 
 // The row loop of k_tile_lo (the sums of fct_lo_body in swe_kernels.hip).  WET: every node of the tile and its
 // halo is deeper than the dry-node thresholds of both sums, so the ratios need no selection and the two
@@ -239,20 +209,7 @@ k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, dou
     bool wet = true;
     auto put = [&](int k, int row) {
         const Node A = U[row];
-        LoNode n;
-        n.h = A.h;
-        n.z = A.z;
-        n.qx = A.qx;
-        n.qy = A.qy;
-        n.ovh = ovh_of(A.h, K.htiny);
-        n.sq = D0 ? 0.0 : sqrt_rn(K.g * fabs(A.h));
-        n.q = own_ratio(A.h, A.z);
-        // entropy (update.f90:924-935)
-        double E = K.g * (A.h * A.h);
-        E = E + (A.qx * n.ovh) * A.qx;
-        E = E + (A.qy * n.ovh) * A.qy;
-        n.E = 0.5 * E;
-        n.alpha = ALPHA ? alpha[row] : 0.0;
+        const LoNode n = lo_node<D0>(A, ALPHA ? alpha[row] : 0.0, K);
         nodes[k] = n;
         // (padding rows of the tile's slices, which nothing refers to, do not count)
         wet = wet && (A.h > wet_h || (k == tid && len == 0));
@@ -266,61 +223,13 @@ k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, dou
     LoSums s;
     if (all_wet) lo_rows<true, ALPHA, WRITE_LO, D0>(nodes, M, h.pb, len, I, K, r16, d0, dmu, roundoff, s, err);
     else lo_rows<false, ALPHA, WRITE_LO, D0>(nodes, M, h.pb, len, I, K, r16, d0, dmu, roundoff, s, err);
-    const double mi = M.m[i];
-    const double ovh_i = nodes[tid].ovh;
-    const double v1i = I.qx * ovh_i, v2i = I.qy * ovh_i;
-    double e1 = s.e1, e2 = s.e2, e3 = s.e3;
-    add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, e2, e3);
-    if (WRITE_LO) {
-        double r1 = s.r1, r2 = s.r2, r3 = s.r3;
-        add_sources<HAS_SRC>(K.src, I, mi, v1i, v2i, dt, K, r2, r3);
-        r1 = r1 / mi;
-        r2 = r2 / mi;
-        r3 = r3 / mi;
-        double hL;
-        if (roundoff) hL = I.h * (1.0 + dt * s.fix / mi) + dt * r1;
-        else hL = fmaxF(I.h + dt * r1, 0.0);
-        st_entry1(ulo_h + i, hL);
-        st_entry(ulo_q + i, make_double2(I.qx + dt * r2, I.qy + dt * r3));
-        if (K.check_h && hL < 0.0) err |= FLAG_NEG_H;
-    }
-    // entropy_residual (update.f90:838-868)
-    e1 = e1 / mi;
-    e2 = e2 / mi;
-    e3 = e3 / mi;
-    const double ht = I.h + dt * e1;
-    const double qxt = I.qx + dt * e2;
-    const double qyt = I.qy + dt * e3;
-    const double ovt = ovh_of(ht, K.htiny);
-    const double vn1 = qxt * ovt, vn2 = qyt * ovt;
-    const double E = nodes[tid].E;
-    double En = K.g * (ht * ht);
-    En = En + vn1 * qxt;
-    En = En + vn2 * qyt;
-    En = 0.5 * En;
-    double Ep0 = K.g * I.h;
-    Ep0 = Ep0 - 0.5 * (v1i * v1i);
-    Ep0 = Ep0 - 0.5 * (v2i * v2i);
-    double r = mi * (En - E) / dt;
-    r = r - mi * e1 * Ep0;
-    r = r - mi * e2 * v1i;
-    r = r - mi * e3 * v2i;
-    const double rescale = fabs(s.emax - s.emin) / 2.0 + K.ent_cst;
-    res[i] = fabs(r) / rescale;
+    lo_finish<WRITE_LO, HAS_SRC>(I, nodes[tid].ovh, nodes[tid].E, s, M.m[i], dt, K, roundoff, i, ulo_h, ulo_q, res, err);
     raise_flag(flags_out, inst, err);
 }
 
 // =============================================================================================
 // FCT stage, pass 2 on tiles: k_fct_rminus's R-.
 // =============================================================================================
-// What the limiter passes stage per node.
-struct alignas(16) FluxNode {
-    double h, z, q, res;   // q: own_ratio
-};
-struct alignas(16) ApplyNode {
-    double h, z, q, res, qx, qy, Rm, pad;
-};
-
 // Entries a lane holds in registers: their viscosities and columns are loaded before the staging barrier, all
 // at once; longer rows read the rest in a loop.
 constexpr int kHeld = 8;
@@ -336,20 +245,6 @@ __device__ __forceinline__ void hold_row(HeldRow& H, const Mesh& M, const double
             H.lo[q] = ld_entry(dmu + pb + 64 * q);
             H.l[q] = M.lcol[pb + 64 * q];
         }
-}
-
-// Antidiffusive flux of an off-diagonal entry (fct_flux of swe_rows.h, the depth ratios from the staged nodes).
-template <class N>
-__device__ __forceinline__ double tile_flux(const N& I, const N& J, const double2 lo, double& dA, double& muA,
-                                            double& ratij, double& ratji) {
-    const double rij = fmaxF(I.res, J.res);
-    dA = fminF(lo.x, 1.0 * rij) - lo.x;
-    muA = fminF(lo.y, 1.0 * rij) - lo.y;
-    double Hij, Hji;
-    depth_ratios(I.h, I.z, I.q, J.h, J.z, J.q, Hij, Hji, ratij, ratji);
-    ratij = (I.h <= 0.0) ? 0.0 : ratij;
-    ratji = (J.h <= 0.0) ? 0.0 : ratji;
-    return dA * (J.h * ratji - I.h * ratij) + muA * (J.h * (1.0 - ratji) - I.h * (1.0 - ratij));
 }
 
 __global__ void __launch_bounds__(64 * kMaxTileSlices)
@@ -464,10 +359,6 @@ k_tile_apply(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, 
 // =============================================================================================
 // First-order stage on tiles: k_stage_lo's update, with the wall and inflow values of bdy.
 // =============================================================================================
-struct alignas(16) StageNode {
-    double h, z, qx, qy, ovh, sq, q, alpha;
-};
-
 // Low-order sums of an entry with the neighbour's components uj over the own ui (k_stage_lo's and
 // k_stage_sgn's; v2fi, v2fj are the second velocities of the flux).
 template <int SMB, int NC>
@@ -514,28 +405,6 @@ __device__ __forceinline__ void stage_entry(double (&r)[NC], double& fix, const 
         r[1] = r[1] - topo * c.x;
         r[2] = r[2] - topo * c.y;
     }
-}
-
-// The Euler update of the depth and the RK combination with the walls and inflow of bdy.
-template <int SMB>
-__device__ __forceinline__ double stage_depth(double h, double dt, double fix, double mi, double r1) {
-    if constexpr (SMB == SMB_1) return h + dt * r1;
-    else if constexpr (SMB == SMB_ROUNDOFF) return h * (1.0 + dt * fix / mi) + dt * r1;
-    else return fmaxF(h + dt * r1, 0.0);
-}
-__device__ __forceinline__ void stage_out(Node o, const Mesh& M, const InstDev& D, const Node* __restrict__ Uo,
-                                          Node* __restrict__ out, int i, int stage, int bdy) {
-    if (stage != 0) {
-        const Node P = Uo[i];
-        o.h = rk_combine(stage, P.h, o.h);
-        o.qx = rk_combine(stage, P.qx, o.qx);
-        o.qy = rk_combine(stage, P.qy, o.qy);
-    }
-    if (bdy) {
-        const int mask = M.dirm[i];
-        if (mask) bdy_row(o, mask, D, stage);
-    }
-    out[i] = o;
 }
 
 template <int SMB, bool ALPHA, bool HAS_SRC, bool D0>
@@ -811,18 +680,14 @@ k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, con
 }
 
 // =============================================================================================
-// COMPUTE_DT on tiles: k_compute_dt's d_ij (kept in d0 for the first stage) and per-instance maxima; with
+// COMPUTE_DT on tiles: k_compute_dt's d_ij (kept in d0 for the first stage) and per-instance maxima, and where
+// asked for the first stage's alpha (its neighbours' depths are staged here anyway); with
 // advance, the workgroup that ends last does the step's bookkeeping (k_finalize_dt) as well.
 // =============================================================================================
-struct alignas(16) DtNode {
-    double h, qx, qy, ovh, sq, pad;
-};
-
 __global__ void __launch_bounds__(64 * kMaxTileSlices)
 k_tile_dt(Mesh M, InstDev* __restrict__ T, const Node* __restrict__ U, double* __restrict__ d0,
-          unsigned long long* __restrict__ vmax, int* __restrict__ flags, unsigned* __restrict__ done, int all,
-          int advance, int ninst, int remap) {
-    const int R = (int)blockDim.x;
+          double* __restrict__ alpha, unsigned long long* __restrict__ vmax, int* __restrict__ flags,
+          unsigned* __restrict__ done, int all, int advance, int ninst, int remap) {
     extern __shared__ double smem[];
     DtNode* nodes = (DtNode*)smem;
     __shared__ unsigned long long red[kMaxTileSlices];
@@ -852,7 +717,7 @@ k_tile_dt(Mesh M, InstDev* __restrict__ T, const Node* __restrict__ U, double* _
         const Rcp r16 = uniform_rcp(K.g16);
         const DtNode A = nodes[tid];
         const Node I{A.h, A.qx, A.qy, 0.0};
-        double s = 0.0;
+        double s = 0.0, num = 0.0, den = 0.0;
         for (int q = 0; q < len; ++q) {
             const int64_t p = pb + 64 * (int64_t)q;
             const double2 c = c_next;
@@ -861,62 +726,19 @@ k_tile_dt(Mesh M, InstDev* __restrict__ T, const Node* __restrict__ U, double* _
                 c_next = ld_entry(M.c + p + 64);
                 l_next = M.lcol[p + 64];
             }
-            if (l == tid) continue;    // the reference's row sum adds a 0.0 there
             const DtNode& B = nodes[l];
+            num = num + B.h - A.h;
+            den = den + fabs(B.h - A.h);
+            if (l == tid) continue;    // the reference's row sum adds a 0.0 there
             const Node J{B.h, B.qx, B.qy, 0.0};
             const double d = dij_from_c(c, I, J, A.ovh, B.ovh, A.sq, B.sq, K, r16, err);
             if (d0) st_entry1(d0 + p, d);
             s = s + d;
         }
         v = fabs(-s) / M.m[i];
+        if (alpha) alpha[i] = alpha_value(num, den, A.h, K.htiny);
     }
-    if (err) {
-        atomicOr(flags + inst, err);
-        __builtin_amdgcn_s_waitcnt(0);    // done before this workgroup's arrival below
-    }
-    // v >= 0 orders like its bit pattern
-    unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long o = __shfl_xor(b, off, 64);
-        b = (o > b) ? o : b;
-    }
-    if ((tid & 63) == 0) red[tid >> 6] = b;
-    __syncthreads();
-    if (tid == 0) {
-        unsigned long long mx = 0ull;
-        for (int k = 0; k < R / 64; ++k) mx = (red[k] > mx) ? red[k] : mx;
-        // most workgroups find a greater maximum already there and leave the word alone
-        if (mx > __hip_atomic_load(vmax + inst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(vmax + inst, mx);
-    }
-    if (!advance) return;
-    // The workgroup's flags and maximum are in place before its arrival counts (each thread waits for its own
-    // atomics), so the workgroup that arrives last sees all of them; it reads them with atomics, which bypass
-    // what its XCD may have cached.
-    // Arrivals count in kDoneGroups words first and then, once per word, in one: a single word serialises them
-    // (1568 workgroups: 31 us for the pass, 22 us with half as many).
-    if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);
-        const unsigned n = gridDim.x, g = blockIdx.x % kDoneGroups;
-        const unsigned groups = n < kDoneGroups ? n : kDoneGroups, members = (n - g + kDoneGroups - 1) / kDoneGroups;
-        unsigned* mine = done + kDoneStride * (1 + g);
-        int end = 0;
-        if (atomicAdd(mine, 1u) == members - 1) {
-            atomicExch(mine, 0u);
-            if (atomicAdd(done, 1u) == groups - 1) {
-                atomicExch(done, 0u);
-                end = 1;
-            }
-        }
-        last = end;
-    }
-    __syncthreads();
-    if (!last) return;
-    for (int k = tid; k < ninst; k += R) {
-        const unsigned long long mx = atomicExch(vmax + k, 0ull);
-        const int f = __hip_atomic_load(flags + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        finalize_one(T, mx, f, k, 1);
-    }
+    dt_finish(T, v, err, inst, vmax, flags, done, red, &last, advance, ninst);
 }
 
 template <bool ALPHA, bool WRITE_LO, bool HAS_SRC, bool D0>
@@ -1011,10 +833,10 @@ void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int st
                        P.tune.k[KID_APPLY].remap);
 }
 
-void launch_tile_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
+void launch_tile_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance) {
     hipLaunchKernelGGL(k_tile_dt, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
-                       sizeof(DtNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), P.tab, U, d0, P.vmax, P.flags,
-                       P.done, all, advance ? 1 : 0, P.ninst(), P.tune.k[KID_DT].remap);
+                       sizeof(DtNode) * (size_t)P.tile_nodes, P.stream, mesh_view(P), P.tab, U, d0, alpha, P.vmax,
+                       P.flags, P.done, all, advance ? 1 : 0, P.ninst(), P.tune.k[KID_DT].remap);
 }
 
 static_assert(sizeof(LoNode) * kTileNodes <= 65536, "a tile's records fit a workgroup's LDS");
