@@ -489,25 +489,14 @@ constexpr size_t kBcBytes = sizeof(BcEntry) + 3 * sizeof(double);   // entry, va
 
 void free_pool(Pool* P) {
     if (!P) return;
-    void* bufs[] = {P->sl,  P->len,     P->dpos,  P->perm, P->m,     P->z,     P->col,   P->dcol,  P->c,
-                    P->elist,   P->S[0],  P->S[1], P->S[2],  P->scratch, P->ulo_h, P->ulo_q, P->d0,    P->dmu,
-                    P->ework,   P->alpha, P->res,  P->Rm,    P->nwork, P->stage3, P->tab, P->vmax,
-                    P->flags, P->bc,    P->bcv,  P->X[0], P->X[1], P->X[2], P->X[3], P->stage5, P->xscratch,
-                    P->bar,     P->lcol,  P->halo,   P->tact,   P->dirm,  P->done};
+    void* bufs[] = {P->block, P->X[0], P->X[1], P->X[2], P->X[3], P->stage5, P->xscratch};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (P->act) (void)hipFree(P->act);
-    for (int k = 0; k < 2; ++k) {
-        if (P->act_host[k]) (void)hipHostFree(P->act_host[k]);
-        if (P->act_ev[k]) (void)hipEventDestroy(P->act_ev[k]);
-    }
-    for (auto& sn : P->snaps) {
-        if (sn.tab) (void)hipHostFree(sn.tab);
-        if (sn.flags) (void)hipHostFree(sn.flags);
+    if (P->host_block) (void)hipHostFree(P->host_block);
+    for (hipEvent_t e : P->act_ev)
+        if (e) (void)hipEventDestroy(e);
+    for (auto& sn : P->snaps)
         if (sn.ev) (void)hipEventDestroy(sn.ev);
-    }
-    if (P->tab_host) (void)hipHostFree(P->tab_host);
-    if (P->flags_host) (void)hipHostFree(P->flags_host);
     if (P->gexec) (void)hipGraphExecDestroy(P->gexec);
     for (hipEvent_t e : P->tk.ev) (void)hipEventDestroy(e);
     if (P->released) (void)hipEventDestroy(P->released);
@@ -565,69 +554,73 @@ int pool_create(const PoolCaps& caps, Pool** out) {
     }
     const size_t R = (size_t)P->rows_cap, S = (size_t)caps.slots;
     int rc;
-#define ALLOC(ptr, n)                      \
-    do {                                   \
-        if ((rc = dalloc(&(ptr), (n)))) {  \
-            free_pool(P);                  \
-            return rc;                     \
-        }                                  \
-    } while (0)
-    ALLOC(P->sl, (size_t)slices);
-    ALLOC(P->len, R);
-    ALLOC(P->dpos, R);
-    ALLOC(P->dirm, R);
-    ALLOC(P->perm, R);
-    ALLOC(P->m, R);
-    ALLOC(P->z, R);
-    ALLOC(P->col, S);
-    ALLOC(P->dcol, S);
-    ALLOC(P->c, S);
-    ALLOC(P->elist, (size_t)std::max<int64_t>(caps.elist, 1));
-    for (int k = 0; k < 3; ++k) ALLOC(P->S[k], R);
-    ALLOC(P->scratch, R);
-    ALLOC(P->ulo_h, R);
-    ALLOC(P->ulo_q, R);
-    ALLOC(P->d0, S);
-    ALLOC(P->dmu, S);
-    ALLOC(P->ework, S);
-    ALLOC(P->alpha, R);
-    ALLOC(P->res, R);
-    ALLOC(P->Rm, R);
-    ALLOC(P->nwork, R);
-    ALLOC(P->stage3, 3 * R);
-    ALLOC(P->tab, (size_t)caps.instances);
-    ALLOC(P->vmax, (size_t)caps.instances);
-    ALLOC(P->flags, (size_t)caps.instances);
-    ALLOC(P->bc, (size_t)std::max<int64_t>(caps.bc, 1));
     P->bcv_stride = std::max<int64_t>(caps.bc, 1);
-    ALLOC(P->bcv, 3 * (size_t)P->bcv_stride);
-    ALLOC(P->act, (size_t)slices);
-    ALLOC(P->tact, (size_t)slices);
-    ALLOC(P->lcol, S);
-    ALLOC(P->halo, (size_t)slices * kHaloStride);
-    ALLOC(P->bar, 2);
-    ALLOC(P->done, (kDoneGroups + 1) * kDoneStride);
-#undef ALLOC
+    Carver dev, host;
+    dev.add(&P->sl, (size_t)slices);
+    dev.add(&P->len, R);
+    dev.add(&P->dpos, R);
+    dev.add(&P->dirm, R);
+    dev.add(&P->perm, R);
+    dev.add(&P->m, R);
+    dev.add(&P->z, R);
+    dev.add(&P->col, S);
+    dev.add(&P->dcol, S);
+    dev.add(&P->c, S);
+    dev.add(&P->elist, (size_t)std::max<int64_t>(caps.elist, 1));
+    for (int k = 0; k < 3; ++k) dev.add(&P->S[k], R);
+    dev.add(&P->scratch, R);
+    dev.add(&P->ulo_h, R);
+    dev.add(&P->ulo_q, R);
+    dev.add(&P->d0, S);
+    dev.add(&P->dmu, S);
+    dev.add(&P->ework, S);
+    dev.add(&P->alpha, R);
+    dev.add(&P->res, R);
+    dev.add(&P->Rm, R);
+    dev.add(&P->nwork, R);
+    dev.add(&P->stage3, 3 * R);
+    dev.add(&P->tab, (size_t)caps.instances);
+    dev.add(&P->vmax, (size_t)caps.instances);
+    dev.add(&P->flags, (size_t)caps.instances);
+    dev.add(&P->bc, (size_t)std::max<int64_t>(caps.bc, 1));
+    dev.add(&P->bcv, 3 * (size_t)P->bcv_stride);
+    dev.add(&P->act, (size_t)slices);
+    dev.add(&P->tact, (size_t)slices);
+    dev.add(&P->lcol, S);
+    dev.add(&P->halo, (size_t)slices * kHaloStride);
+    dev.add(&P->bar, 2);
+    dev.add(&P->done, (kDoneGroups + 1) * kDoneStride);
+    for (int k = 0; k < 2; ++k) host.add(&P->act_host[k], 2 * (size_t)slices);
+    for (auto& sn : P->snaps) {
+        host.add(&sn.tab, (size_t)caps.instances);
+        host.add(&sn.flags, (size_t)caps.instances);
+    }
+    host.add(&P->tab_host, (size_t)caps.instances);
+    host.add(&P->flags_host, (size_t)caps.instances);
+    char* block = nullptr;
+    if ((rc = dalloc(&block, dev.bytes()))) {
+        free_pool(P);
+        return rc;
+    }
+    P->block = block;
+    dev.place(block);
     P->listed.assign((size_t)caps.instances, 0);
+    e = hipHostMalloc(&P->host_block, host.bytes(), hipHostMallocDefault);
+    if (e != hipSuccess) {
+        P->host_block = nullptr;
+        free_pool(P);
+        return fail(SWE_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", host.bytes(), hipGetErrorString(e));
+    }
+    host.place(P->host_block);
     for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        e = hipHostMalloc((void**)&P->act_host[k], 2 * sizeof(int) * (size_t)slices, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&P->act_ev[k], hipEventDisableTiming);
+        e = hipEventCreateWithFlags(&P->act_ev[k], hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventRecord(P->act_ev[k], P->stream);
     }
+    for (auto& sn : P->snaps)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&sn.ev, hipEventDisableTiming);
     if (e != hipSuccess) {
         free_pool(P);
         return fail(SWE_EHIP, "pool lists: %s", hipGetErrorString(e));
-    }
-    for (auto& sn : P->snaps) {
-        if (e == hipSuccess) e = hipHostMalloc((void**)&sn.tab, sizeof(InstDev) * (size_t)caps.instances, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostMalloc((void**)&sn.flags, sizeof(int) * (size_t)caps.instances, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&sn.ev, hipEventDisableTiming);
-    }
-    if (e == hipSuccess) e = hipHostMalloc((void**)&P->tab_host, sizeof(InstDev) * (size_t)caps.instances, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&P->flags_host, sizeof(int) * (size_t)caps.instances, hipHostMallocDefault);
-    if (e != hipSuccess) {
-        free_pool(P);
-        return fail(SWE_ENOMEM, "hipHostMalloc failed: %s", hipGetErrorString(e));
     }
     // empty tables: every slice free, every instance free; len = 0 marks rows without work
     std::vector<SliceInfo> sl0((size_t)slices);

@@ -5,11 +5,11 @@
 //
 // Same contract as the host assembly in swe_setup.cpp, bit for bit: every entry is accumulated in
 // ascending element order (Gauss points in order inside an element) with the shared element
-// geometry of swe_p1.h, and lumped(i) is the sequential row sum.  One lane per row:
+// geometry of swe_p1.h, and lumped(i) is the sequential row sum:
 //   1. node -> element lists: counts (integer atomics), exclusive scan, fill, then each list
 //      sorted ascending in its lane, so the lists do not depend on the order the atomics ran in;
-//   2. row pattern: the sorted unique nodes of the row's elements, counted, scanned into ia;
-//   3. row fill: ja, then mass and c_ij accumulated element by element, lumped, diag.
+//   2. row pattern: the sorted unique nodes of the row's elements, counted, scanned into ia, written to ja;
+//   3. values: mass and c_ij accumulated element by element, eight lanes per row, then lumped.
 // A node may belong to at most kMaxElems elements (rows of at most 3*kMaxElems candidates);
 // larger fans are reported as SWE_EINVAL and can be assembled on the host.
 #include <hip/hip_runtime.h>
@@ -33,134 +33,157 @@ using swe_p1::ElemGeom;
 using swe_p1::P1Rule;
 using swe_p1::element_geometry;
 
-__global__ void k_count_elems(const int* __restrict__ jj, int64_t n3, int64_t* __restrict__ cnt) {
+constexpr int kFlagMany = 1, kFlagRange = 2;   // a node in more than kMaxElems elements; an entry of jj out of range
+
+__global__ void k_count_elems(const int* __restrict__ jj, int64_t n3, int np, int64_t* __restrict__ cnt,
+                              unsigned long long* __restrict__ flag) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n3) atomicAdd((unsigned long long*)&cnt[jj[q] - 1], 1ull);
+    if (q >= n3) return;
+    const int j = jj[q];
+    if (j < 1 || j > np) atomicOr(flag, (unsigned long long)kFlagRange);
+    else atomicAdd((unsigned long long*)&cnt[j - 1], 1ull);
 }
 
-__global__ void k_fill_elems(const int* __restrict__ jj, int me, const int64_t* __restrict__ start,
+__global__ void k_fill_elems(const int* __restrict__ jj, int me, int np, const int64_t* __restrict__ start,
                              int* __restrict__ fill, int* __restrict__ elem) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= 3 * (int64_t)me) return;
     const int n = jj[q] - 1;
+    if (n < 0 || n >= np) return;
     const int k = atomicAdd(&fill[n], 1);
     elem[start[n] + k] = (int)(q / 3);
 }
 
-// Sort each node's element list ascending; flags a node in more than kMaxElems elements.
-__global__ void k_sort_elems(int np, const int64_t* __restrict__ start, int* __restrict__ elem,
-                             int* __restrict__ too_many) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+// A lane's array of N ints in LDS (word t of lane l at t*64 + l: no bank conflicts).  As a private array it would
+// lie in scratch memory, each access a trip through the caches.
+struct LaneInts {
+    int* base;
+    __device__ int& operator[](int t) const { return base[64 * t]; }
+};
+
+// Sorted unique nodes (0-based) of the n elements el; returns their number.
+__device__ int row_pattern(LaneInts el, int n, const int* __restrict__ jj, LaneInts row) {
+    int w = 0;
+    for (int s = 0; s < n; ++s) {
+        const int m = el[s];
+        for (int a = 0; a < 3; ++a) {
+            const int v = jj[3 * (int64_t)m + a] - 1;
+            // insert v keeping row[0..w) sorted and unique
+            int c = w - 1, x = -1;
+            while (c >= 0 && (x = row[c]) > v) --c;
+            if (c >= 0 && x == v) continue;
+            for (int t = w; t > c + 1; --t) row[t] = row[t - 1];
+            row[c + 1] = v;
+            ++w;
+        }
+    }
+    return w;
+}
+
+// One wave per 64 rows.  FILL false: sorts each row's element list ascending (elem) and counts its pattern (cnt);
+// flags a node in more than kMaxElems elements.  FILL true: writes the pattern (ja) and the diagonal's position.
+template <bool FILL>
+__global__ void __launch_bounds__(64)
+k_row_pattern(int np, const int64_t* __restrict__ start, int* __restrict__ elem, const int* __restrict__ jj,
+              int64_t* __restrict__ cnt, unsigned long long* __restrict__ flag, const int64_t* __restrict__ ia0,
+              int* __restrict__ ja, int* __restrict__ diag) {
+    __shared__ int lds[64 * (kMaxElems + kMaxPattern)];
+    const LaneInts el{lds + threadIdx.x}, row{lds + 64 * kMaxElems + threadIdx.x};
+    const int i = (int)(blockIdx.x * 64 + threadIdx.x);
     if (i >= np) return;
     const int64_t b = start[i];
     const int n = (int)(start[i + 1] - b);
     if (n > kMaxElems) {
-        atomicOr(too_many, 1);
+        if (!FILL) {
+            atomicOr(flag, (unsigned long long)kFlagMany);
+            cnt[i] = 0;
+        }
         return;
     }
-    for (int a = 1; a < n; ++a) {
+    for (int a = 0; a < n; ++a) {
         const int v = elem[b + a];
-        int c = a - 1;
-        while (c >= 0 && elem[b + c] > v) {
-            elem[b + c + 1] = elem[b + c];
+        int c = a - 1, x;
+        while (!FILL && c >= 0 && (x = el[c]) > v) {
+            el[c + 1] = x;
             --c;
         }
-        elem[b + c + 1] = v;
+        el[FILL ? a : c + 1] = v;
     }
-}
-
-// Sorted unique nodes (0-based) of the elements of row i; returns their number.
-__device__ int row_pattern(int i, const int64_t* __restrict__ start, const int* __restrict__ elem,
-                           const int* __restrict__ jj, int* row) {
-    int n = 0;
-    for (int64_t s = start[i]; s < start[i + 1]; ++s) {
-        const int m = elem[s];
-        for (int a = 0; a < 3; ++a) {
-            const int v = jj[3 * (int64_t)m + a] - 1;
-            // insert v keeping row[0..n) sorted and unique
-            int c = n - 1;
-            bool dup = false;
-            while (c >= 0 && row[c] >= v) {
-                if (row[c] == v) {
-                    dup = true;
-                    break;
-                }
-                --c;
-            }
-            if (dup) continue;
-            for (int t = n; t > c + 1; --t) row[t] = row[t - 1];
-            row[c + 1] = v;
-            ++n;
+    const int w = row_pattern(el, n, jj, row);
+    if (!FILL) {
+        for (int a = 0; a < n; ++a) elem[b + a] = el[a];
+        cnt[i] = w;
+    } else {
+        const int64_t p0 = ia0[i];
+        for (int q = 0; q < w; ++q) {
+            const int j = row[q];
+            ja[p0 + q] = j + 1;
+            if (j == i) diag[i] = (int)(p0 + q) + 1;
         }
     }
-    return n;
 }
 
-__global__ void k_row_count(int np, const int64_t* __restrict__ start, const int* __restrict__ elem,
-                            const int* __restrict__ jj, int64_t* __restrict__ cnt) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+// mass, c_ij and lumped of the rows: eight lanes per row, lane e taking the entries e, e+8, ...; an entry walks
+// the row's elements in ascending order and adds what those that contain its column give, as the host does
+// (qs_00_M visits l, then nj, then ni; x(d) = SUM_l dw(d,nj,l) * ww(ni,l) * rj(l)), so the sums are the same
+// additions.  (One lane per row, finding the pattern and adding into
+// the entries in memory: 631 us at 300k nodes; the pattern and these values now 119 + 144.)
+__global__ void __launch_bounds__(256)
+k_row_values(int np, const int64_t* __restrict__ start, const int* __restrict__ elem, const int* __restrict__ jj,
+             const double* __restrict__ rr, const int64_t* __restrict__ ia0, const int* __restrict__ ja,
+             double* __restrict__ mass, double* __restrict__ lumped, double* __restrict__ cx, double* __restrict__ cy) {
+    const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 3), e = (int)(threadIdx.x & 7);
     if (i >= np) return;
-    int row[kMaxPattern];
-    cnt[i] = row_pattern(i, start, elem, jj, row);
-}
-
-__device__ __forceinline__ int slot_of(const int* row, int n, int j) {
-    int lo = 0, hi = n;   // first position with row[pos] >= j
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (row[mid] < j) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
-__global__ void k_row_fill(int np, const int64_t* __restrict__ start, const int* __restrict__ elem,
-                           const int* __restrict__ jj, const double* __restrict__ rr, const int64_t* __restrict__ ia0,
-                           int* __restrict__ ja, int* __restrict__ diag, double* __restrict__ mass,
-                           double* __restrict__ lumped, double* __restrict__ cx, double* __restrict__ cy) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= np) return;
-    int row[kMaxPattern];
-    const int n = row_pattern(i, start, elem, jj, row);
-    const int64_t p0 = ia0[i];
-    for (int q = 0; q < n; ++q) {
-        ja[p0 + q] = row[q] + 1;
-        mass[p0 + q] = 0.0;
-        cx[p0 + q] = 0.0;
-        cy[p0 + q] = 0.0;
-    }
     const P1Rule R;
-    for (int64_t s = start[i]; s < start[i + 1]; ++s) {
-        const int m = elem[s];
-        const int nd[3] = {jj[3 * (int64_t)m] - 1, jj[3 * (int64_t)m + 1] - 1, jj[3 * (int64_t)m + 2] - 1};
-        const int ni = (nd[0] == i) ? 0 : (nd[1] == i) ? 1 : 2;
-        ElemGeom G;
-        element_geometry(R, rr, nd, G);
-        // mass: qs_00_M visits l, then nj, then ni; for this row ni is fixed
-        for (int l = 0; l < 3; ++l) {
-            const double al = 1.0 * G.rj[l];
-            for (int nj = 0; nj < 3; ++nj) {
-                const int64_t p = p0 + slot_of(row, n, nd[nj]);
-                mass[p] = mass[p] + R.ww[nj][l] * al * R.ww[ni][l];
-            }
-        }
-        // c_ij: x(d) = SUM_l dw(d,nj,l) * ww(ni,l) * rj(l)
-        for (int nj = 0; nj < 3; ++nj) {
-            double x[2];
-            for (int d = 0; d < 2; ++d) {
-                double sacc = 0.0;
-                for (int l = 0; l < 3; ++l) sacc = sacc + G.dw[d][nj][l] * R.ww[ni][l] * G.rj[l];
-                x[d] = sacc;
-            }
-            const int64_t p = p0 + slot_of(row, n, nd[nj]);
-            cx[p] = cx[p] + x[0];
-            cy[p] = cy[p] + x[1];
-        }
-    }
+    const int64_t p0 = ia0[i], s0 = start[i], s1 = start[i + 1];
+    const int n = (int)(ia0[i + 1] - p0);
     double sl = 0.0;
-    for (int q = 0; q < n; ++q) sl = sl + mass[p0 + q];
-    lumped[i] = sl;
-    diag[i] = (int)(p0 + slot_of(row, n, i)) + 1;
+    for (int q0 = 0; q0 < n; q0 += 8) {
+        const bool has = q0 + e < n;
+        double am = 0.0, ax = 0.0, ay = 0.0;
+        if (has) {
+            const int64_t p = p0 + q0 + e;
+            const int j = ja[p] - 1;
+            for (int64_t s = s0; s < s1; ++s) {
+                const int64_t m = elem[s];
+                const int nd[3] = {jj[3 * m] - 1, jj[3 * m + 1] - 1, jj[3 * m + 2] - 1};
+                if (nd[0] != j && nd[1] != j && nd[2] != j) continue;
+                const int ni = (nd[0] == i) ? 0 : (nd[1] == i) ? 1 : 2;
+                ElemGeom G;
+                element_geometry(R, rr, nd, G);
+                double wi[3];
+#pragma unroll
+                for (int l = 0; l < 3; ++l) wi[l] = (ni == 0) ? R.ww[0][l] : (ni == 1) ? R.ww[1][l] : R.ww[2][l];
+#pragma unroll
+                for (int l = 0; l < 3; ++l) {
+                    const double al = 1.0 * G.rj[l];
+#pragma unroll
+                    for (int nj = 0; nj < 3; ++nj)
+                        if (nd[nj] == j) am = am + R.ww[nj][l] * al * wi[l];
+                }
+#pragma unroll
+                for (int nj = 0; nj < 3; ++nj)
+                    if (nd[nj] == j) {
+                        double x[2];
+#pragma unroll
+                        for (int d = 0; d < 2; ++d) {
+                            double sacc = 0.0;
+#pragma unroll
+                            for (int l = 0; l < 3; ++l) sacc = sacc + G.dw[d][nj][l] * wi[l] * G.rj[l];
+                            x[d] = sacc;
+                        }
+                        ax = ax + x[0];
+                        ay = ay + x[1];
+                    }
+            }
+            mass[p] = am;
+            cx[p] = ax;
+            cy[p] = ay;
+        }
+        const int left = (n - q0 < 8) ? n - q0 : 8;
+        for (int k = 0; k < left; ++k) sl = sl + __shfl(am, k, 8);
+    }
+    if (e == 0) lumped[i] = sl;
 }
 
 unsigned grid_of(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -171,6 +194,7 @@ struct swe_assembly {
     int np = 0;
     int64_t nnz = 0;
     hipStream_t stream = nullptr;
+    void *nodes = nullptr, *entries = nullptr;   // the allocations that hold the arrays per node and per entry
     int64_t* ia0 = nullptr;   // 0-based row starts, np+1
     int* ja = nullptr;
     int* diag = nullptr;
@@ -182,10 +206,12 @@ namespace {
 
 // Device memory of the set-up is stream-ordered (hipMallocAsync / hipFreeAsync on the set-up's own
 // stream): unlike hipFree, releasing it does not wait for the work queued on other streams, so a
-// batch can admit meshes while its steps run.
-template <class T>
-hipError_t dalloc(T** p, size_t n, hipStream_t s) {
-    return hipMallocAsync((void**)p, sizeof(T) * (n ? n : 1), s);
+// batch can admit meshes while its steps run.  Each stage takes one block for all its arrays.
+hipError_t block_alloc(swe::Carver& c, void** block, hipStream_t s) {
+    const hipError_t e = hipMallocAsync(block, c.bytes() ? c.bytes() : 1, s);
+    if (e == hipSuccess) c.place(*block);
+    else *block = nullptr;
+    return e;
 }
 
 void dfree(void* p, hipStream_t s) {
@@ -194,8 +220,8 @@ void dfree(void* p, hipStream_t s) {
 
 void release(swe_assembly* a) {
     if (!a) return;
-    void* bufs[] = {a->ia0, a->ja, a->diag, a->mass, a->lumped, a->cx, a->cy, a->rr};
-    for (void* b : bufs) dfree(b, a->stream);
+    dfree(a->nodes, a->stream);
+    dfree(a->entries, a->stream);
     if (a->stream) {
         (void)hipStreamSynchronize(a->stream);
         (void)hipStreamDestroy(a->stream);
@@ -203,16 +229,14 @@ void release(swe_assembly* a) {
     delete a;
 }
 
-// Exclusive prefix sum on stream s (ordered with the stream's other work; nothing waits here).
-hipError_t exclusive_scan(const int64_t* in, int64_t* out, int n, hipStream_t s) {
+// Scratch of an exclusive prefix sum of n values, and the sum itself on stream s (nothing waits here).
+size_t scan_bytes(int n) {
     size_t bytes = 0;
-    hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, in, out, n, s);
-    if (e != hipSuccess) return e;
-    void* tmp = nullptr;
-    if ((e = hipMallocAsync(&tmp, bytes ? bytes : 1, s)) != hipSuccess) return e;
-    e = hipcub::DeviceScan::ExclusiveSum(tmp, bytes, in, out, n, s);
-    dfree(tmp, s);
-    return e;
+    (void)hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (const int64_t*)nullptr, (int64_t*)nullptr, n, nullptr);
+    return bytes;
+}
+hipError_t exclusive_scan(const int64_t* in, int64_t* out, int n, char* tmp, size_t bytes, hipStream_t s) {
+    return hipcub::DeviceScan::ExclusiveSum(tmp, bytes, in, out, n, s);
 }
 
 }  // namespace
@@ -224,70 +248,77 @@ extern "C" int swe_assemble_device(int np, int me, const int* jj, const double* 
     *out = nullptr;
     *nnz = 0;
     const int64_t n3 = 3 * (int64_t)me;
-    for (int64_t q = 0; q < n3; ++q)
-        if (jj[q] < 1 || jj[q] > np) return swe::fail(SWE_EINVAL, "jj(%lld)=%d out of range", (long long)q + 1, jj[q]);
     swe_assembly* a = new swe_assembly();
     a->np = np;
-    int *djj = nullptr, *elem = nullptr, *fill = nullptr, *flag = nullptr;
-    double* drr = nullptr;
+    int *djj = nullptr, *elem = nullptr, *fill = nullptr;
+    unsigned long long* flag = nullptr;
     int64_t *cnt = nullptr, *start = nullptr;
-    int too_many = 0;
-    hipError_t e = hipStreamCreate(&a->stream);
+    char* tmp = nullptr;
+    void* work = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&a->stream, hipStreamNonBlocking);
     hipStream_t s = a->stream;
-    if (e == hipSuccess) e = dalloc(&djj, (size_t)n3, s);
-    if (e == hipSuccess) e = dalloc(&drr, 2 * (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&elem, (size_t)n3, s);
-    if (e == hipSuccess) e = dalloc(&fill, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&flag, 1, s);
-    if (e == hipSuccess) e = dalloc(&cnt, (size_t)np + 1, s);
-    if (e == hipSuccess) e = dalloc(&start, (size_t)np + 1, s);
-    if (e == hipSuccess) e = dalloc(&a->ia0, (size_t)np + 1, s);
+    const size_t nscan = scan_bytes(np + 1);
+    swe::Carver keep, temp;
+    keep.add(&a->rr, 2 * (size_t)np);
+    keep.add(&a->ia0, (size_t)np + 1);
+    keep.add(&a->diag, (size_t)np);
+    keep.add(&a->lumped, (size_t)np);
+    temp.add(&flag, 1);          // flag, cnt and fill start at zero: one clearing
+    temp.add(&cnt, (size_t)np + 1);
+    temp.add(&fill, (size_t)np);
+    const size_t zeroed = temp.bytes();
+    temp.add(&djj, (size_t)n3);
+    temp.add(&elem, (size_t)n3);
+    temp.add(&start, (size_t)np + 1);
+    temp.add(&tmp, nscan);
+    if (e == hipSuccess) e = block_alloc(keep, &a->nodes, s);
+    if (e == hipSuccess) e = block_alloc(temp, &work, s);
     if (e == hipSuccess) e = hipMemcpyAsync(djj, jj, sizeof(int) * (size_t)n3, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(drr, rr, sizeof(double) * 2 * (size_t)np, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemsetAsync(cnt, 0, sizeof(int64_t) * ((size_t)np + 1), s);
-    if (e == hipSuccess) e = hipMemsetAsync(fill, 0, sizeof(int) * (size_t)np, s);
-    if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(int), s);
+    if (e == hipSuccess) e = hipMemcpyAsync(a->rr, rr, sizeof(double) * 2 * (size_t)np, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipMemsetAsync(work, 0, zeroed, s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_count_elems, dim3(grid_of(n3, 256)), dim3(256), 0, s, djj, n3, cnt);
-        e = exclusive_scan(cnt, start, np + 1, s);
+        hipLaunchKernelGGL(k_count_elems, dim3(grid_of(n3, 256)), dim3(256), 0, s, djj, n3, np, cnt, flag);
+        e = exclusive_scan(cnt, start, np + 1, tmp, nscan, s);
     }
+    unsigned long long bad = 0;
+    int64_t total = 0;
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_fill_elems, dim3(grid_of(n3, 256)), dim3(256), 0, s, djj, me, start, fill, elem);
-        hipLaunchKernelGGL(k_sort_elems, dim3(grid_of(np, 256)), dim3(256), 0, s, np, start, elem, flag);
-        e = hipMemcpyAsync(&too_many, flag, sizeof(int), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        hipLaunchKernelGGL(k_fill_elems, dim3(grid_of(n3, 256)), dim3(256), 0, s, djj, me, np, start, fill, elem);
+        // (cnt's last word stays the zero it was: no entry of jj counts there)
+        hipLaunchKernelGGL(k_row_pattern<false>, dim3(grid_of(np, 64)), dim3(64), 0, s, np, start, elem, djj, cnt, flag,
+                           (const int64_t*)nullptr, (int*)nullptr, (int*)nullptr);
+        e = exclusive_scan(cnt, a->ia0, np + 1, tmp, nscan, s);
     }
+    if (e == hipSuccess) e = hipMemcpyAsync(&bad, flag, sizeof bad, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&total, a->ia0 + np, sizeof total, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     int rc = SWE_OK;
-    if (e == hipSuccess && too_many) {
+    if (e == hipSuccess && (bad & kFlagRange)) {
+        for (int64_t q = 0; q < n3 && rc == SWE_OK; ++q)
+            if (jj[q] < 1 || jj[q] > np) rc = swe::fail(SWE_EINVAL, "jj(%lld)=%d out of range", (long long)q + 1, jj[q]);
+    } else if (e == hipSuccess && bad) {
         rc = swe::fail(SWE_EINVAL, "a node belongs to more than %d elements; use swe_assemble", kMaxElems);
+    } else if (e == hipSuccess && total >= (int64_t)INT32_MAX) {
+        rc = swe::fail(SWE_EINVAL, "nnz = %lld does not fit the 32-bit row pointers", (long long)total);
     } else if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_row_count, dim3(grid_of(np, 128)), dim3(128), 0, s, np, start, elem, djj, cnt);
-        e = hipMemsetAsync(cnt + np, 0, sizeof(int64_t), s);
-        if (e == hipSuccess) e = exclusive_scan(cnt, a->ia0, np + 1, s);
-        int64_t total = 0;
-        if (e == hipSuccess) e = hipMemcpyAsync(&total, a->ia0 + np, sizeof(int64_t), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e == hipSuccess && total >= (int64_t)INT32_MAX) {
-            rc = swe::fail(SWE_EINVAL, "nnz = %lld does not fit the 32-bit row pointers", (long long)total);
-        } else if (e == hipSuccess) {
-            a->nnz = total;
-            e = dalloc(&a->ja, (size_t)total, s);
-            if (e == hipSuccess) e = dalloc(&a->diag, (size_t)np, s);
-            if (e == hipSuccess) e = dalloc(&a->mass, (size_t)total, s);
-            if (e == hipSuccess) e = dalloc(&a->lumped, (size_t)np, s);
-            if (e == hipSuccess) e = dalloc(&a->cx, (size_t)total, s);
-            if (e == hipSuccess) e = dalloc(&a->cy, (size_t)total, s);
-            if (e == hipSuccess) {
-                hipLaunchKernelGGL(k_row_fill, dim3(grid_of(np, 128)), dim3(128), 0, s, np, start, elem, djj, drr,
-                                   a->ia0, a->ja, a->diag, a->mass, a->lumped, a->cx, a->cy);
-                e = hipGetLastError();
-            }
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
+        a->nnz = total;
+        swe::Carver entries;
+        entries.add(&a->ja, (size_t)total);
+        entries.add(&a->mass, (size_t)total);
+        entries.add(&a->cx, (size_t)total);
+        entries.add(&a->cy, (size_t)total);
+        e = block_alloc(entries, &a->entries, s);
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(k_row_pattern<true>, dim3(grid_of(np, 64)), dim3(64), 0, s, np, start, elem, djj,
+                               (int64_t*)nullptr, flag, (const int64_t*)a->ia0, a->ja, a->diag);
+            hipLaunchKernelGGL(k_row_values, dim3(grid_of(8 * (int64_t)np, 256)), dim3(256), 0, s, np, start, elem, djj,
+                               (const double*)a->rr, (const int64_t*)a->ia0, (const int*)a->ja, a->mass, a->lumped, a->cx,
+                               a->cy);
+            e = hipGetLastError();
         }
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
     }
-    a->rr = drr;
-    void* tmp[] = {djj, elem, fill, flag, cnt, start};
-    for (void* b : tmp) dfree(b, s);
+    dfree(work, s);
     if (e != hipSuccess) rc = swe::fail(SWE_EHIP, "device assembly: %s", hipGetErrorString(e));
     if (rc != SWE_OK) {
         release(a);
@@ -373,7 +404,7 @@ double double_of_ord(unsigned long long o) {
 }
 
 // box = {min x, max x, min y, max y} as orderable images (initialised to ~0, 0, ~0, 0).
-__global__ void k_bbox(int np, const double* __restrict__ rr, unsigned long long* __restrict__ box) {
+__global__ void __launch_bounds__(256) k_bbox(int np, const double* __restrict__ rr, unsigned long long* __restrict__ box) {
     unsigned long long v[4] = {~0ull, 0ull, ~0ull, 0ull};
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < np; i += (int64_t)gridDim.x * blockDim.x) {
         const unsigned long long x = ord_of(rr[2 * i]), y = ord_of(rr[2 * i + 1]);
@@ -387,12 +418,17 @@ __global__ void k_bbox(int np, const double* __restrict__ rr, unsigned long long
             const unsigned long long o = __shfl_xor(v[q], off, 64);
             v[q] = (q & 1) ? ((o > v[q]) ? o : v[q]) : ((o < v[q]) ? o : v[q]);
         }
-    if ((threadIdx.x & 63) == 0) {
-        atomicMin(box + 0, v[0]);
-        atomicMax(box + 1, v[1]);
-        atomicMin(box + 2, v[2]);
-        atomicMax(box + 3, v[3]);
-    }
+    // one atomic per workgroup and bound: they serialise on one cache line
+    __shared__ unsigned long long red[4][4];
+    const int w = (int)(threadIdx.x >> 6), q = (int)threadIdx.x;
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 4; ++k) red[k][w] = v[k];
+    __syncthreads();
+    if (q >= 4) return;
+    unsigned long long r = red[q][0];
+    for (int k = 1; k < 4; ++k) r = (q & 1) ? ((red[q][k] > r) ? red[q][k] : r) : ((red[q][k] < r) ? red[q][k] : r);
+    if (q & 1) atomicMax(box + q, r);
+    else atomicMin(box + q, r);
 }
 
 constexpr int kCurveBits = 20;   // per coordinate: 2^20 cells along each side of the bounding box
@@ -443,6 +479,7 @@ __global__ void k_lay_iperm(int np, int np_pad, const int* __restrict__ perm, co
 __global__ void k_lay_slices(int nsl, int np, const int* __restrict__ lenr, int64_t* __restrict__ slots,
                              int64_t* __restrict__ ecnt, int* __restrict__ wmax) {
     const int s = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (s == nsl) slots[s] = ecnt[s] = 0;
     if (s >= nsl) return;
     int w = 0;
     int64_t e = 0;
@@ -455,6 +492,16 @@ __global__ void k_lay_slices(int nsl, int np, const int* __restrict__ lenr, int6
     slots[s] = 64 * (int64_t)w;
     ecnt[s] = e;
     atomicMax(wmax, w);
+}
+
+// What the host reads of a layout: its slots, its list entries, the row-length check and the longest row.
+__global__ void k_lay_sums(int nsl, const int64_t* __restrict__ sptr, const int64_t* __restrict__ eoff,
+                           const int* __restrict__ flag, int64_t* __restrict__ sums) {
+    if (threadIdx.x != 0) return;
+    sums[0] = sptr[nsl];
+    sums[1] = eoff[nsl];
+    sums[2] = flag[0];
+    sums[3] = flag[1];
 }
 
 struct LayOut {
@@ -640,48 +687,50 @@ hipError_t read_u64(const unsigned long long* d, unsigned long long* h, int n, h
     return (e == hipSuccess) ? hipStreamSynchronize(s) : e;
 }
 
+// Scratch of the locality order.
+struct OrderWork {
+    unsigned long long *box = nullptr, *keys = nullptr, *keys2 = nullptr;
+    int *idx = nullptr, *order = nullptr;
+    char* tmp = nullptr;
+    size_t bytes = 0;
+    bool used = false;
+    void add(swe::Carver& c, int np) {
+        used = swe::reorder_enabled() && np >= 2;
+        if (!used) return;
+        (void)hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, nullptr);
+        c.add(&box, 4);
+        c.add(&keys, (size_t)np);
+        c.add(&keys2, (size_t)np);
+        c.add(&idx, (size_t)np);
+        c.add(&order, (size_t)np);
+        c.add(&tmp, bytes);
+    }
+};
+
 // The base order of the layout: the nodes along a Hilbert curve of their coordinates, the device
 // counterpart of the host layout's locality order, or the caller's numbering (*base null) under
 // SWE_REORDER=0.  Only the processing order changes; results do not depend on it.
-hipError_t locality_order(const swe_assembly* a, hipStream_t s, int** base) {
+hipError_t locality_order(const swe_assembly* a, hipStream_t s, OrderWork& w, const int** base) {
     *base = nullptr;
     const int np = a->np;
-    if (!swe::reorder_enabled() || np < 2) return hipSuccess;
-    unsigned long long* box = nullptr;
-    unsigned long long *keys = nullptr, *keys2 = nullptr;
-    int *idx = nullptr, *order = nullptr;
-    void* tmp = nullptr;
+    if (!w.used) return hipSuccess;
     unsigned long long h[4] = {~0ull, 0ull, ~0ull, 0ull};
-    const unsigned bl = (unsigned)((np + 255) / 256);
-    hipError_t e = dalloc(&box, 4, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(box, h, sizeof h, hipMemcpyHostToDevice, s);
+    const unsigned bl = grid_of(np, 256);
+    hipError_t e = hipMemcpyAsync(w.box, h, sizeof h, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_bbox, dim3(bl < 1024u ? bl : 1024u), dim3(256), 0, s, np, (const double*)a->rr, box);
+        hipLaunchKernelGGL(k_bbox, dim3(bl < 256u ? bl : 256u), dim3(256), 0, s, np, (const double*)a->rr, w.box);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = read_u64(box, h, 4, s);
+    if (e == hipSuccess) e = read_u64(w.box, h, 4, s);
+    if (e != hipSuccess) return e;
     const double x0 = double_of_ord(h[0]), x1 = double_of_ord(h[1]);
     const double y0 = double_of_ord(h[2]), y1 = double_of_ord(h[3]);
     const double top = (double)((1 << kCurveBits) - 1);
     const double sx = (x1 > x0) ? top / (x1 - x0) : 0.0, sy = (y1 > y0) ? top / (y1 - y0) : 0.0;
-    if (e == hipSuccess) e = dalloc(&keys, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&keys2, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&idx, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&order, (size_t)np, s);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_curve_key, dim3(bl), dim3(256), 0, s, np, (const double*)a->rr, x0, sx, y0, sy, keys, idx);
-        e = hipGetLastError();
-    }
-    size_t bytes = 0;
-    if (e == hipSuccess)
-        e = hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
-    if (e == hipSuccess) e = hipMallocAsync(&tmp, bytes ? bytes : 1, s);
-    if (e == hipSuccess)   // a radix sort is stable: equal keys keep the caller's order
-        e = hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, keys2, idx, order, np, 0, 2 * kCurveBits, s);
-    void* bufs[] = {box, keys, keys2, idx, tmp};
-    for (void* b : bufs) dfree(b, s);
-    if (e == hipSuccess) *base = order;
-    else dfree(order, s);
+    hipLaunchKernelGGL(k_curve_key, dim3(bl), dim3(256), 0, s, np, (const double*)a->rr, x0, sx, y0, sy, w.keys, w.idx);
+    // a radix sort is stable: equal keys keep the caller's order
+    e = hipcub::DeviceRadixSort::SortPairs(w.tmp, w.bytes, w.keys, w.keys2, w.idx, w.order, np, 0, 2 * kCurveBits, s);
+    if (e == hipSuccess) *base = w.order;
     return e;
 }
 
@@ -690,8 +739,7 @@ hipError_t locality_order(const swe_assembly* a, hipStream_t s, int** base) {
 namespace swe {
 
 void free_device_layout(DeviceLayout& DL) {
-    void* bufs[] = {DL.perm, DL.iperm, DL.len, DL.sptr, DL.eoff};
-    for (void* b : bufs) dfree(b, DL.stream);
+    dfree(DL.block, DL.stream);
     DL = DeviceLayout{};
 }
 
@@ -710,48 +758,61 @@ int build_layout_device(const swe_assembly* a, int tile_slices, DeviceLayout& DL
     int* lenc = nullptr;
     int* flag = nullptr;
     int64_t *slots = nullptr, *ecnt = nullptr;
-    hipError_t e = dalloc(&DL.perm, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&DL.iperm, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&DL.len, (size_t)np_pad, s);
-    if (e == hipSuccess) e = dalloc(&DL.sptr, (size_t)nsl + 1, s);
-    if (e == hipSuccess) e = dalloc(&DL.eoff, (size_t)nsl + 1, s);
-    if (e == hipSuccess) e = dalloc(&lenc, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&flag, 2, s);
-    if (e == hipSuccess) e = dalloc(&slots, (size_t)nsl + 1, s);
-    if (e == hipSuccess) e = dalloc(&ecnt, (size_t)nsl + 1, s);
-    if (e == hipSuccess) e = hipMemsetAsync(flag, 0, 2 * sizeof(int), s);
-    if (e == hipSuccess) e = hipMemsetAsync(slots + nsl, 0, sizeof(int64_t), s);
-    if (e == hipSuccess) e = hipMemsetAsync(ecnt + nsl, 0, sizeof(int64_t), s);
-    int* base = nullptr;
-    if (e == hipSuccess) e = locality_order(a, s, &base);
-    int hflag[2] = {0, 0};
+    int64_t* sums = nullptr;
+    char* tmp = nullptr;
+    void* work = nullptr;
+    const size_t nscan = scan_bytes(nsl + 1);
+    Carver keep, temp;
+    keep.add(&DL.perm, (size_t)np);
+    keep.add(&DL.iperm, (size_t)np);
+    keep.add(&DL.len, (size_t)np_pad);
+    keep.add(&DL.sptr, (size_t)nsl + 1);
+    keep.add(&DL.eoff, (size_t)nsl + 1);
+    temp.add(&flag, 2);
+    const size_t zeroed = temp.bytes();
+    temp.add(&sums, 4);
+    temp.add(&lenc, (size_t)np);
+    temp.add(&slots, (size_t)nsl + 1);
+    temp.add(&ecnt, (size_t)nsl + 1);
+    temp.add(&tmp, nscan);
+    OrderWork ow;
+    ow.add(temp, np);
+    hipError_t e = block_alloc(keep, &DL.block, s);
+    if (e == hipSuccess) e = block_alloc(temp, &work, s);
+    if (e == hipSuccess) e = hipMemsetAsync(work, 0, zeroed, s);
+    const int* base = nullptr;
+    if (e == hipSuccess) e = locality_order(a, s, ow, &base);
+    int64_t h[4] = {0, 0, 0, 0};
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_lay_len, dim3(grid_of(np, 256)), dim3(256), 0, s, np, (const int64_t*)a->ia0, lenc, flag);
         hipLaunchKernelGGL(k_lay_sort, dim3(grid_of(nsl, tile_slices)), dim3(64 * tile_slices), 0, s, np,
-                           (const int*)lenc, (const int*)base, DL.perm);
+                           (const int*)lenc, base, DL.perm);
         hipLaunchKernelGGL(k_lay_iperm, dim3(grid_of(np_pad, 256)), dim3(256), 0, s, np, np_pad, (const int*)DL.perm,
                            (const int*)lenc, DL.iperm, DL.len);
-        hipLaunchKernelGGL(k_lay_slices, dim3(grid_of(nsl, 256)), dim3(256), 0, s, nsl, np, (const int*)DL.len, slots,
+        hipLaunchKernelGGL(k_lay_slices, dim3(grid_of(nsl + 1, 256)), dim3(256), 0, s, nsl, np, (const int*)DL.len, slots,
                            ecnt, flag + 1);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = exclusive_scan(slots, DL.sptr, nsl + 1, s);
-    if (e == hipSuccess) e = exclusive_scan(ecnt, DL.eoff, nsl + 1, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(hflag, flag, 2 * sizeof(int), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&DL.nslot, DL.sptr + nsl, sizeof(int64_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&DL.ne, DL.eoff + nsl, sizeof(int64_t), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = exclusive_scan(slots, DL.sptr, nsl + 1, tmp, nscan, s);
+    if (e == hipSuccess) e = exclusive_scan(ecnt, DL.eoff, nsl + 1, tmp, nscan, s);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_lay_sums, dim3(1), dim3(64), 0, s, nsl, (const int64_t*)DL.sptr, (const int64_t*)DL.eoff,
+                           (const int*)flag, sums);
+        e = hipMemcpyAsync(h, sums, sizeof h, hipMemcpyDeviceToHost, s);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    void* tmp[] = {lenc, flag, slots, ecnt, base};
-    for (void* b : tmp) dfree(b, s);
+    dfree(work, s);
     if (e != hipSuccess) {
         free_device_layout(DL);
         return fail(SWE_EHIP, "device layout: %s", hipGetErrorString(e));
     }
-    if (hflag[0]) {
+    if (h[2]) {
         free_device_layout(DL);
         return fail(SWE_EINVAL, "a row has more than %d entries", kMaxRow);
     }
-    DL.wmax = hflag[1];
+    DL.nslot = h[0];
+    DL.ne = h[1];
+    DL.wmax = (int)h[3];
     return SWE_OK;
 }
 
@@ -794,10 +855,13 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
     int* dnodes = nullptr;
     int* dlong = nullptr;
     int longest = 0;
-    hipError_t e = dalloc(&dbath, (size_t)np, s);
-    if (e == hipSuccess) e = dalloc(&dlong, 1, s);
+    void* work = nullptr;
+    Carver temp;
+    temp.add(&dlong, 1);
+    temp.add(&dbath, (size_t)np);
+    temp.add(&dnodes, (size_t)nbc);
+    hipError_t e = block_alloc(temp, &work, s);
     if (e == hipSuccess) e = hipMemcpyAsync(dlong, &longest, sizeof longest, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = dalloc(&dnodes, (size_t)nbc, s);
     if (e == hipSuccess) e = hipMemcpyAsync(dbath, bath, sizeof(double) * (size_t)np, hipMemcpyHostToDevice, s);
     for (int c = 0, q = 0; c < 3 && e == hipSuccess; q += nlist[c], ++c)
         if (nlist[c] > 0)
@@ -828,9 +892,7 @@ int pool_add_assembled(Pool* P, const swe_assembly* a, const DeviceLayout& DL, c
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&longest, dlong, sizeof longest, hipMemcpyDeviceToHost, s);
-    dfree(dbath, s);
-    dfree(dlong, s);
-    dfree(dnodes, s);
+    dfree(work, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         P->a_slices.release(s0, DL.nsl);
