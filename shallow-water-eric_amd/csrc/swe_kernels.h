@@ -79,12 +79,19 @@ __device__ __forceinline__ Rcp uniform_rcp(double b) {
     R.y = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
     return R;
 }
-__device__ __forceinline__ double div_shared(double a, const Rcp& R) {
-    double q = a * R.y;
-    const double e = __builtin_fma(-R.b, q, a);
-    q = __builtin_fma(e, R.y, q);
+// div_fast is the sequence alone, right where div_ok says so: callers with several quotients check them together,
+// one branch instead of one each, and the code between the branches is long enough to hide its own latency.
+__device__ __forceinline__ double div_fast(double a, const Rcp& R) {
+    const double q = a * R.y;
+    return __builtin_fma(__builtin_fma(-R.b, q, a), R.y, q);
+}
+__device__ __forceinline__ bool div_ok(double a, const Rcp& R) {
     const double m = fabs(a);
-    if (__builtin_expect(!(R.ok && ((m >= 0x1p-500 && m <= 0x1p+500) || m == 0.0)), 0)) q = a / R.b;
+    return R.ok & (((m >= 0x1p-500) & (m <= 0x1p+500)) | (m == 0.0));
+}
+__device__ __forceinline__ double div_shared(double a, const Rcp& R) {
+    double q = div_fast(a, R);
+    if (__builtin_expect(!div_ok(a, R), 0)) q = a / R.b;
     return q;
 }
 
@@ -136,10 +143,12 @@ __device__ __forceinline__ double lambda_vacc(double hl, double qxl, double qyl,
     const double h0 = K.x0 * hmin;
     const double w = vl - vr;
     const double t0 = posF(w + 2.0 * sql + 2.0 * sqr);
-    double ht = fminF(h0, div_shared(t0 * t0, r16));
-    const bool pos = hmin >= 0.0 && hmax <= K.lam_h && h0 >= hmax;
-    const bool small = w <= 0.0 || (hmin >= 0x1p-300 && w * w * K.lam_w <= hmin * hmin * (left ? ovhl : ovhr));
-    if (!(pos && small)) {
+    const double tt = t0 * t0;
+    double ht = fminF(h0, div_fast(tt, r16));
+    const bool quick = div_ok(tt, r16) & (hmin >= 0.0) & (hmax <= K.lam_h) & (h0 >= hmax) &
+                       ((w <= 0.0) | ((hmin >= 0x1p-300) & (w * w * K.lam_w <= hmin * hmin * (left ? ovhl : ovhr))));
+    if (__builtin_expect(!quick, 0)) {
+        ht = fminF(h0, div_shared(tt, r16));
         const double fh = phi_f(h0, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
         if (!(0.0 <= fh)) {
             const double fh2 = phi_f(K.x0 * hmax, vl, hl, vr, hr, ovhl, ovhr, sql, sqr, K);
@@ -159,11 +168,10 @@ __device__ __forceinline__ double lambda_vacc(double hl, double qxl, double qyl,
             }
         }
     }
-    // the arguments are products of two factors >= 1
-    const double lbdl = vl - sql * sqrt_normal((1.0 + posF((ht - hl) * ovhl / 2.0)) *
-                                               (1.0 + posF((ht - hl) * ovhl)));
-    const double lbdr = vr + sqr * sqrt_normal((1.0 + posF((ht - hr) * ovhr / 2.0)) *
-                                               (1.0 + posF((ht - hr) * ovhr)));
+    // the arguments are products of two factors >= 1; MAX(x/2, 0) is MAX(x, 0)/2, exactly
+    const double xl = posF((ht - hl) * ovhl), xr = posF((ht - hr) * ovhr);
+    const double lbdl = vl - sql * sqrt_normal((1.0 + 0.5 * xl) * (1.0 + xl));
+    const double lbdr = vr + sqr * sqrt_normal((1.0 + 0.5 * xr) * (1.0 + xr));
     return fmaxF(fabs(lbdl), fabs(lbdr));
 }
 

@@ -142,7 +142,9 @@ __device__ __forceinline__ double dij_from_c(const double2 c, const Node& I, con
                                              const Rcp& r16, int& err) {
     const double norm = sqrt_normal(c.x * c.x + c.y * c.y);
     const Rcp rn = refined_rcp(norm);
-    return dij_of(make_double2(div_shared(c.x, rn), div_shared(c.y, rn)), norm, I, J, ovh_i, ovh_j, sql, sqr, K, r16,
+    double2 n = make_double2(div_fast(c.x, rn), div_fast(c.y, rn));
+    if (__builtin_expect(!(div_ok(c.x, rn) & div_ok(c.y, rn)), 0)) n = make_double2(div_shared(c.x, rn), div_shared(c.y, rn));
+    return dij_of(n, norm, I, J, ovh_i, ovh_j, sql, sqr, K, r16,
                   err);
 }
 

@@ -192,7 +192,7 @@ __device__ __forceinline__ void lo_rows(const LoNode* __restrict__ nodes, const 
 // entropy residual).
 // =============================================================================================
 template <bool ALPHA, bool WRITE_LO, bool HAS_SRC, bool D0>
-__global__ void __launch_bounds__(64 * kMaxTileSlices)
+__global__ void __launch_bounds__(64 * kMaxTileSlices, 4)
 k_tile_lo(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, double* __restrict__ ulo_h,
           double2* __restrict__ ulo_q, double2* __restrict__ dmu, double* __restrict__ res,
           const double* __restrict__ d0, const double* __restrict__ alpha, int roundoff, int* __restrict__ flags_out,
