@@ -975,7 +975,8 @@ int record_dt(Pool* P) {
 }
 
 int record_stages(Pool* P) {
-    const bool lam = P->mode.viscosity_type != SWE_GALERKIN;
+    // (what the dt pass left serves the form that ran it: a schedule set between the parts of a step may change it)
+    const bool lam = P->mode.viscosity_type != SWE_GALERKIN && P->dt_tiles == tiles_apply(*P);
     Node* A = P->S[0];
     Node* B = P->S[1];
     Node* C = P->S[2];

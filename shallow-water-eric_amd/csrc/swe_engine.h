@@ -221,6 +221,7 @@ struct Pool {
     int step_form = 0;                // swe_step_form: 0 launch sequence (graph), 1 persistent (fct)
     bool coop_ok = false;             // the device takes cooperative launches
     int num_cu = 1;
+    bool dt_tiles = false;            // the last step's dt pass ran on tiles (and gave alpha with d0)
     unsigned* done = nullptr;         // the dt pass's counts of workgroups that are through (0 between launches)
     unsigned* bar = nullptr;          // the persistent step's barrier word and abort word
     bool use_graph = false;

@@ -1451,6 +1451,7 @@ bool alpha_used(const Mode& md) { return md.alpha != 0 && md.viscosity_type != S
 bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return false;
+    if (advance) P.dt_tiles = tiles_apply(P);
     if (tiles_apply(P)) {
         timed_begin(P, KID_DT);
         double* const al = (advance && alpha_used(P.mode)) ? P.alpha : nullptr;

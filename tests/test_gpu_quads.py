@@ -40,3 +40,22 @@ def test_meshes_sharing_a_launch(oracle):
         for k, p, n in zip(ids, ps, steps):
             ref, _, rt, err = oracle_run(oracle, p, n)
             assert err == 0 and b.status(k)[1] == rt and same_bits(b.get_state(k), ref)
+
+
+@pytest.mark.parametrize("n_side", [41, 200])
+@pytest.mark.parametrize("before,after", [(0, 2), (2, 0)])
+def test_schedule_set_between_the_parts_of_a_step(oracle, n_side, before, after):
+    """What the dt pass leaves for the first stage differs between the tile and the gather kernels."""
+    from swe_amd import problems
+    p = problems.bumps(n_side=n_side)
+    ref, rdts, _, err = oracle_run(oracle, p, 2)
+    assert err == 0
+    with p.solver() as s:
+        s.set_state(p.u0)
+        s.time = 0.0
+        for k in range(2):
+            s.schedule = {n: (b, r, before if n == "k_fct_lo" else kd) for n, (b, r, kd) in s.schedule.items()}
+            assert s.step_begin() == rdts[k]
+            s.schedule = {n: (b, r, after if n == "k_fct_lo" else kd) for n, (b, r, kd) in s.schedule.items()}
+            s.step_finish()
+        assert same_bits(s.get_state(), ref)
