@@ -319,6 +319,7 @@ void launch_finalize_dt(Pool& P, int advance);
 inline bool tiles_apply(const Pool& P) { return P.ntile > 0 && P.tune.k[KID_FCT_LO].kind == 2; }
 void launch_tile_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo);
 void launch_tile_rminus(Pool& P, const Node* U);
+void launch_tile_alpha(Pool& P, const Node* U);
 bool tile_stage_applies(const Pool& P);
 void launch_tile_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy);
 void launch_tile_ev(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);

@@ -1496,7 +1496,8 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
     if (alpha && !quads && !(d0 && tiles_apply(P))) {
         const LaunchCfg& L = P.tune.k[KID_ALPHA];
         timed_begin(P, KID_ALPHA);
-        SWE_BS_SWITCH(L.block, hipLaunchKernelGGL((k_alpha<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0, P.stream,
+        if (tiles_apply(P)) launch_tile_alpha(P, U);
+        else SWE_BS_SWITCH(L.block, hipLaunchKernelGGL((k_alpha<BS>), dim3(blocks_of((int64_t)M.nact * 64, BS)), dim3(BS), 0, P.stream,
                                                   M, T, U, P.alpha, L.remap))
         timed_end(P, KID_ALPHA);
     }

@@ -680,6 +680,40 @@ k_tile_ev(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, con
 }
 
 // =============================================================================================
+// alpha_limit's factors on tiles: k_alpha's (the first stage's come from the dt pass).  Bound by latency: the
+// columns are loaded while the depths are staged, and no load depends on another but the halo's.  Measured
+// against k_alpha: 22.0 -> 12.9 us at 1M nodes, 267 -> 187 at 16.8M, 5.0 -> 4.8 at 100k.
+// =============================================================================================
+__global__ void __launch_bounds__(64 * kMaxTileSlices)
+k_tile_alpha(Mesh M, const InstDev* __restrict__ T, const Node* __restrict__ U, double* __restrict__ alpha, int remap) {
+    extern __shared__ double depth[];
+    const TileHead h = tile_head(M, remap);
+    const int inst = h.inst, tid = h.tid;
+    const bool go = T[inst].go != 0;
+    const double htiny = T[inst].K.htiny;
+    const int len = go ? h.len : 0;
+    int l[kHeld];
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q) l[q] = (q < len) ? (int)M.lcol[h.pb + 64 * q] : tid;
+    auto put = [&](int k, int row) { depth[k] = U[row].h; };
+    stage_nodes(h, M, go, put);
+    __syncthreads();
+    if (len == 0) return;
+    const double hi = depth[tid];
+    double num = 0.0, den = 0.0;
+    auto entry = [&](int x) {
+        const double hj = depth[x];
+        num = num + hj - hi;
+        den = den + fabs(hj - hi);
+    };
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q)
+        if (q < len) entry(l[q]);
+    for (int q = kHeld; q < len; ++q) entry(M.lcol[h.pb + 64 * q]);
+    alpha[h.i] = alpha_value(num, den, hi, htiny);
+}
+
+// =============================================================================================
 // COMPUTE_DT on tiles: k_compute_dt's d_ij (kept in d0 for the first stage) and per-instance maxima, and where
 // asked for the first stage's alpha (its neighbours' depths are staged here anyway); with
 // advance, the workgroup that ends last does the step's bookkeeping (k_finalize_dt) as well.
@@ -831,6 +865,12 @@ void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int st
                        (const double*)P.ulo_h, (const double2*)P.ulo_q, out, (const double2*)P.dmu,
                        (const double*)P.res, (const double*)P.Rm, stage, bdy ? 1 : 0, P.flags,
                        P.tune.k[KID_APPLY].remap);
+}
+
+void launch_tile_alpha(Pool& P, const Node* U) {
+    hipLaunchKernelGGL(k_tile_alpha, dim3((unsigned)P.ntile), dim3(64 * P.tile_slices),
+                       sizeof(double) * (size_t)P.tile_nodes, P.stream, mesh_view(P), (const InstDev*)P.tab, U, P.alpha,
+                       P.tune.k[KID_ALPHA].remap);
 }
 
 void launch_tile_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance) {
