@@ -311,11 +311,12 @@ bool reorder_enabled() {
 }
 
 // Tiles are large where the pool has rows enough for several per CU of a 256-CU device (fewer halo rows per
-// row), small where it has not (more workgroups).  Measured per launch at 1, 2 and 4 slices: k_tile_lo 14.0,
-// 14.6, 15.0 us and k_tile_dt 17.1, 17.9, 18.5 us at 5k rows; k_tile_dt 20.4, 19.4, 18.6 us at 100k, the others
-// within 3%; 8 slices were slower than 4 at 1M and 16.8M rows (k_tile_apply 58.2 against 54.0 us, 864 against
-// 830).
-int tile_slices_for(int64_t rows) { return rows <= 32 * 1024 ? 1 : rows <= 128 * 1024 ? 2 : 4; }
+// row), small where it has not (more workgroups).  Measured per launch at 1, 2 and 4 slices, a lane per row:
+// k_tile_lo 14.0, 14.6, 15.0 us and k_tile_dt 17.1, 17.9, 18.5 us at 5k rows; k_tile_dt 20.4, 19.4, 18.6 us at 100k,
+// the others within 3%; 8 slices were slower than 4 at 1M and 16.8M rows (k_tile_apply 58.2 against 54.0 us, 864
+// against 830).  One-slice tiles run with four lanes per row (quads_apply), which pays up to three such
+// workgroups per CU; the figures are there.
+int tile_slices_for(int64_t rows) { return rows <= 48 * 1024 ? 1 : rows <= 128 * 1024 ? 2 : 4; }
 
 // Internal numbering: a base order of the rows (the locality order, or the caller's under SWE_REORDER=0),
 // then inside consecutive windows of `sort_window` rows (0: the rows of a tile)

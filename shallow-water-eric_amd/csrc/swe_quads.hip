@@ -663,11 +663,12 @@ void go_quad_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const doub
 
 static_assert(kQuadSlices <= kMaxTileSlices && kHaloStride <= 3 * 64, "a quad workgroup has a thread per staged row");
 
-// Pools whose tiles are one slice (tile_slices_for: up to 32,768 rows).  Measured per step, a lane per row
-// against four: FCT with alpha 93.6 -> 64.5 us at 5k nodes, 98.9 -> 79.7 at 25k, 102.7 -> 80.8 at 32k; first
-// order 49.1 -> 34.1, 51.5 -> 40.8, 52.7 -> 42.1; entropy viscosity 70.6 -> 51.6, 74.4 -> 63.7, 77.2 -> 65.5.  Above,
-// where every SIMD has a wave anyway, the registers of the terms and the additions made four times cost more
-// than they give: 107.1 -> 113.0 us at 40k, 133.6 -> 202.8 at 100k.
+// Pools whose tiles are one slice (tile_slices_for: up to 49,152 rows, three workgroups per CU).  Measured per
+// step, a lane per row in the tiles used otherwise against four in one-slice tiles: FCT with alpha 93.6 -> 64.5 us at
+// 5k nodes, 102.7 -> 80.8 at 32k, 108.3 -> 103.3 at 47k; first order 49.1 -> 34.1, 52.7 -> 42.1, 54.3 -> 47.8;
+// entropy viscosity 70.6 -> 51.6, 77.2 -> 65.5, 82.9 -> 83.2.  Above, where the SIMDs have waves anyway, the
+// registers of the terms and the additions made four times cost more than they give: at 50k FCT 110.2 -> 112.9 us,
+// first order 55.2 -> 55.5, entropy viscosity 84.2 -> 96.5; at 100k, in two-slice tiles, FCT 133.6 -> 202.8.
 bool quads_apply(const Pool& P) { return P.tile_slices <= kQuadSlices; }
 
 void launch_quad_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo) {

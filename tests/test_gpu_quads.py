@@ -1,4 +1,4 @@
-"""The four-lanes-per-row kernels (csrc/swe_quads.hip, pools of up to 32,768 rows) against the oracle, bit for
+"""The four-lanes-per-row kernels (csrc/swe_quads.hip, pools of up to 49,152 rows) against the oracle, bit for
 bit: a mesh of one partial slice, a partial last slice, the largest mesh they take, and several meshes that
 share each launch, one of which stops first."""
 import pytest
@@ -12,7 +12,7 @@ SCHEMES = [("fct", True), ("fct", False), ("viscous", True), ("viscous", False),
 
 
 @pytest.mark.parametrize("scheme,alpha", SCHEMES)
-@pytest.mark.parametrize("n_side", [5, 17, 181])
+@pytest.mark.parametrize("n_side", [5, 17, 181, 221])
 def test_sizes_against_oracle(oracle, n_side, scheme, alpha):
     from swe_amd import problems
     from swe_amd.solver import SweError
