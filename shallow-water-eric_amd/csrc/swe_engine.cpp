@@ -1005,14 +1005,23 @@ int64_t tuning_hash(const Tuning& t) {
     return h;
 }
 
-// The captured step stays valid while the launch extents, the scheme and the schedules stay.
+// The captured step stays valid while the launch extents, the scheme and the schedules stay.  The number of tiles is
+// an extent of its own: tiles do not cross instances, so other meshes of as many slices can have more or fewer of
+// them (in tiles of two, 5 + 3 slices are 5 tiles and 4 + 4 are 4).
 int ensure_graph(Pool* P) {
-    const int64_t key[7] = {(int64_t)P->nact * 2048 + (P->ntile > 0 ? P->tile_nodes : 0) * 2 + (P->any_bc_values ? 1 : 0), (int64_t)P->ninst(), P->nbc(), (int64_t)P->wmax,
-                            (int64_t)(P->mode.viscosity_type * 128 + P->mode.viscous_type * 16 + P->mode.alpha * 4 +
-                                      P->mode.roundoff * 2 + (P->any_src ? 1 : 0)),
-                            tuning_hash(P->tune),
-                            (P->one < 0) ? -1 : (int64_t)P->one * (1ll << 32) + P->inst[(size_t)P->one].slice0};
-    if (P->gexec && std::equal(key, key + 7, P->graph_key)) return SWE_OK;
+    const std::array<int64_t, kGraphKey> key = {
+        P->nact,
+        P->ntile,
+        P->ntile > 0 ? P->tile_nodes : 0,
+        P->any_bc_values ? 1 : 0,
+        P->ninst(),
+        P->nbc(),
+        P->wmax,
+        P->mode.viscosity_type * 128 + P->mode.viscous_type * 16 + P->mode.alpha * 4 + P->mode.roundoff * 2 +
+            (P->any_src ? 1 : 0),
+        tuning_hash(P->tune),
+        (P->one < 0) ? -1 : (int64_t)P->one * (1ll << 32) + P->inst[(size_t)P->one].slice0};
+    if (P->gexec && key == P->graph_key) return SWE_OK;
     if (P->gexec) {
         (void)hipGraphExecDestroy(P->gexec);
         P->gexec = nullptr;
@@ -1032,7 +1041,7 @@ int ensure_graph(Pool* P) {
         P->gexec = nullptr;
         return fail(SWE_EHIP, "hipGraphInstantiate: %s", hipGetErrorString(ei));
     }
-    std::copy(key, key + 7, P->graph_key);
+    P->graph_key = key;
     return SWE_OK;
 }
 

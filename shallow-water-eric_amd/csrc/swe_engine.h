@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <map>
 #include <string>
 #include <utility>
@@ -47,6 +48,8 @@ struct Tuning {
 // Workgroup sizes a kernel can be launched with.
 bool block_supported(int kid, int block);
 
+// Words of Pool::graph_key.
+constexpr int kGraphKey = 10;
 // Words of Pool::done: one per group of workgroups and one for the groups, a cache line each.
 constexpr unsigned kDoneGroups = 64, kDoneStride = 32;
 
@@ -226,7 +229,7 @@ struct Pool {
     unsigned* bar = nullptr;          // the persistent step's barrier word and abort word
     bool use_graph = false;
     hipGraphExec_t gexec = nullptr;
-    int64_t graph_key[7] = {-1, -1, -1, -1, -1, -1, -1};
+    std::array<int64_t, kGraphKey> graph_key{};   // what the captured step was captured for (ensure_graph)
     bool timing = false;
     std::string timed_name;
     TimedKernel tk;
