@@ -386,7 +386,7 @@ int swe_euler(swe_handle* h, const double* un, double* unext, double dt) {
     const int go = 1;
     if ((rc = pool_set_field(P, kId, offsetof(InstDev, dt), &dt, sizeof dt))) return rc;
     if ((rc = pool_set_field(P, kId, offsetof(InstDev, go), &go, sizeof go))) return rc;
-    if ((rc = launch_euler_stage(*P, P->scratch, P->scratch, P->S[2], nullptr, 0))) return rc;
+    if ((rc = launch_euler_stage(*P, P->scratch, P->scratch, P->S[2], nullptr, false, 0))) return rc;
     if ((rc = pool_download_state(P, kId, P->S[2], unext))) return rc;
     return check_flags(P, kId);
 }
@@ -574,7 +574,8 @@ int swe_step_finish(swe_handle* h, const double* vals) {
             SWE_HIPCHK(hipMemcpyAsync(P->bcv + st * P->bcv_stride + I.bc0, vals + st * n, sizeof(double) * (size_t)n,
                                       hipMemcpyHostToDevice, P->stream));
     }
-    int rc = record_stages(P);
+    // (the caller may have set a schedule or parameters, or run swe_euler, since swe_step_begin)
+    int rc = record_stages(P, false);
     if (rc) return rc;
     SWE_HIPCHK(hipGetLastError());
     return check_flags(P, kId);

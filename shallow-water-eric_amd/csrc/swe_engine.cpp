@@ -975,9 +975,8 @@ int record_dt(Pool* P) {
     return SWE_OK;
 }
 
-int record_stages(Pool* P) {
-    // (what the dt pass left serves the form that ran it: a schedule set between the parts of a step may change it)
-    const bool lam = P->mode.viscosity_type != SWE_GALERKIN && P->dt_tiles == tiles_apply(*P);
+int record_stages(Pool* P, bool same_call) {
+    const bool lam = P->mode.viscosity_type != SWE_GALERKIN;
     Node* A = P->S[0];
     Node* B = P->S[1];
     Node* C = P->S[2];
@@ -985,7 +984,8 @@ int record_stages(Pool* P) {
     const Node* in[3] = {A, B, C};
     Node* out[3] = {B, C, A};
     for (int stage = 0; stage < 3; ++stage) {
-        const int rc = launch_euler_stage(*P, in[stage], A, out[stage], (lam && stage == 0) ? P->d0 : nullptr, stage, true);
+        const bool first = lam && stage == 0;
+        const int rc = launch_euler_stage(*P, in[stage], A, out[stage], first ? P->d0 : nullptr, first && same_call, stage, true);
         if (rc) return rc;
         if (lists) launch_bdy(*P, out[stage], stage);
     }
@@ -996,7 +996,7 @@ namespace {
 
 int record_step(Pool* P) {
     const int rc = record_dt(P);
-    return rc ? rc : record_stages(P);
+    return rc ? rc : record_stages(P, true);
 }
 
 int64_t tuning_hash(const Tuning& t) {

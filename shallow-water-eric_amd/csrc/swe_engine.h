@@ -224,7 +224,6 @@ struct Pool {
     int step_form = 0;                // swe_step_form: 0 launch sequence (graph), 1 persistent (fct)
     bool coop_ok = false;             // the device takes cooperative launches
     int num_cu = 1;
-    bool dt_tiles = false;            // the last step's dt pass ran on tiles (and gave alpha with d0)
     unsigned* done = nullptr;         // the dt pass's counts of workgroups that are through (0 between launches)
     unsigned* bar = nullptr;          // the persistent step's barrier word and abort word
     bool use_graph = false;
@@ -268,7 +267,8 @@ int pool_queue_steps(Pool* P, int nsteps);
 // The parts of one step, launched on the compute stream: the dt pass and its bookkeeping, then the
 // three stages with bdy.
 int record_dt(Pool* P);
-int record_stages(Pool* P);
+// same_call: nothing came between this and record_dt, so what the dt pass left beside d0 still holds.
+int record_stages(Pool* P, bool same_call);
 // Rebuild the launch list from the instances marked listed (ordered on the compute stream).
 int pool_update_active(Pool* P);
 int pool_read_table(Pool* P);         // sync, then tab_host / flags_host hold the table
@@ -331,7 +331,7 @@ void launch_tile_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int st
 // workgroup also does finalize_one for every instance.
 void launch_tile_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance);
 // The same passes with four lanes per row (swe_quads.hip), where tiles_apply and quads_apply.  k_quad_lo and
-// k_quad_stage compute the alpha factors themselves unless d0 says that the dt pass has.
+// k_quad_stage take the alpha factors from P.alpha with d0, and compute them themselves without it.
 bool quads_apply(const Pool& P);
 void launch_quad_lo(Pool& P, const Node* U, const double* d0, bool alpha, bool write_lo);
 void launch_quad_rminus(Pool& P, const Node* U);
@@ -339,7 +339,7 @@ void launch_quad_apply(Pool& P, const Node* U, const Node* Uo, Node* out, int st
 void launch_quad_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool alpha, int stage, bool bdy);
 void launch_quad_ev(Pool& P, const Node* U, const Node* Uo, Node* out, int stage, bool bdy);
 void launch_quad_dt(Pool& P, const Node* U, double* d0, double* alpha, int all, bool advance);
-int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage,
+int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool dt_alpha, int stage,
                        bool bdy = false);
 // Whether launch_euler_stage can write the wall and inflow values itself (given values need launch_bdy).
 bool bdy_fused(const Pool& P);

@@ -1451,7 +1451,6 @@ bool alpha_used(const Mode& md) { return md.alpha != 0 && md.viscosity_type != S
 bool launch_compute_dt(Pool& P, const Node* U, double* d0, int all, bool advance) {
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return false;
-    if (advance) P.dt_tiles = tiles_apply(P);
     if (tiles_apply(P)) {
         timed_begin(P, KID_DT);
         double* const al = (advance && alpha_used(P.mode)) ? P.alpha : nullptr;
@@ -1485,15 +1484,17 @@ void launch_finalize_dt(Pool& P, int advance) {
 // null) holds compute_dij at U.  stage: 0 keeps the Euler output, 1 and 2 apply the RK
 // combinations with Uo.
 // bdy: the kernels that can (bdy_fused) also write the wall and inflow values of `stage`.
-int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, int stage, bool bdy) {
+// dt_alpha: a dt pass of the same call, in the same form, gave d0, so on tiles P.alpha holds the factors at U.
+int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const double* d0, bool dt_alpha, int stage,
+                       bool bdy) {
     const Mode& md = P.mode;
     const Mesh M = mesh_view(P);
     if (M.nact == 0) return SWE_OK;
     const InstDev* T = P.tab;
     const bool alpha = alpha_used(md);
     const bool quads = tiles_apply(P) && quads_apply(P) && !md.sgn;
-    // on tiles the dt pass that gave d0 gave alpha too, and four lanes per row compute it where they stage
-    if (alpha && !quads && !(d0 && tiles_apply(P))) {
+    // on tiles the dt pass gives alpha too, and without d0 four lanes per row compute it where they stage
+    if (alpha && !(quads && !d0) && !(dt_alpha && tiles_apply(P))) {
         const LaunchCfg& L = P.tune.k[KID_ALPHA];
         timed_begin(P, KID_ALPHA);
         if (tiles_apply(P)) launch_tile_alpha(P, U);
