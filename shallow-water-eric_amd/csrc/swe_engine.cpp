@@ -1131,11 +1131,14 @@ int pool_read_table(Pool* P) {
 }
 
 // ---- autotuner ------------------------------------------------------------------------------
-// Coordinate search over the launch schedule of each kernel the scheme uses: workgroup size
-// (128, 256, 512) and XCD-aware workgroup order (on/off).  Each candidate runs `steps` steps
-// from a saved snapshot of the states and the instance table, timed with HIP events around that
-// kernel's launches; the state and the table are restored afterwards, so tuning changes no
-// result (every schedule computes the same rows with the same arithmetic).
+// First the family of kernels (tiles, or the gather kernels), by whole steps: the kind of k_fct_lo stands for all
+// passes of a step, so its own launches do not tell.  Then a coordinate search over the launch schedule of each
+// kernel the step launches: XCD-aware workgroup order (on/off), and for the gather kernels, whose workgroup size is
+// free, that size (128, 256, 512) and the kind of k_fct_lo.  Last the step form, by whole steps again.  Each candidate runs
+// `steps` steps from a saved snapshot of the states and the instance table, timed with HIP events around that
+// kernel's launches or the whole run; the state and the table are restored afterwards, so tuning changes no
+// result (every schedule computes the same rows with the same arithmetic).  A kernel that a trial does not launch
+// keeps its schedule.
 int pool_tune(Pool* P, int steps, int trials) {
     if (P->nact == 0) return SWE_OK;
     steps = std::max(1, steps);
@@ -1193,46 +1196,98 @@ int pool_tune(Pool* P, int steps, int trials) {
     const char* fa = std::getenv("SWE_TUNE_FAIL_AT");
     const int fail_at = fa ? std::atoi(fa) : 0;
     int trial_no = 0;
-    const int blocks[3] = {128, 256, 512};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    if (!rc) {
+        e = hipEventCreate(&ev[0]);
+        if (e == hipSuccess) e = hipEventCreate(&ev[1]);
+        if (e != hipSuccess) rc = fail(SWE_EHIP, "tuning events: %s", hipGetErrorString(e));
+    }
+    // a trial's steps are queued: counted, waited for
+    auto end_trial = [&]() -> int {
+        if (++trial_no == fail_at)
+            return fail(SWE_EHIP, "tuning run: failure injected at trial %d (SWE_TUNE_FAIL_AT)", trial_no);
+        const hipError_t q = hipStreamSynchronize(P->stream);
+        return (q == hipSuccess) ? SWE_OK : fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(q));
+    };
+    auto undo = [&]() -> int {
+        const hipError_t q = restore();
+        if (q != hipSuccess) return fail(SWE_EHIP, "tuning restore: %s", hipGetErrorString(q));
+        dirty = false;
+        return SWE_OK;
+    };
+    // the least time of `trials` runs of whole steps; a first run is untimed (graph capture, code load)
+    auto time_steps = [&](double& ms_min) -> int {
+        ms_min = std::numeric_limits<double>::infinity();
+        for (int t = 0; t <= trials; ++t) {
+            int r;
+            dirty = true;
+            hipError_t q = hipEventRecord(ev[0], P->stream);
+            if (q != hipSuccess) return fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(q));
+            if ((r = pool_queue_steps(P, steps))) return r;
+            q = hipEventRecord(ev[1], P->stream);
+            if (q != hipSuccess) return fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(q));
+            if ((r = end_trial())) return r;
+            float ms = 0.0f;
+            (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
+            if (t > 0) ms_min = std::min(ms_min, (double)ms);
+            if ((r = undo())) return r;
+        }
+        return SWE_OK;
+    };
+    const int form0 = P->step_form;
+    if (!rc && P->ntile > 0) {
+        int& kind = P->tune.k[KID_FCT_LO].kind;
+        const int kind0 = kind, gather = (kind == 1) ? 1 : 0;
+        P->step_form = 0;       // (the persistent form is the gather kernels')
+        P->timing = false;
+        double tiled = 0.0, gathered = 0.0;
+        kind = 2;
+        rc = time_steps(tiled);
+        kind = gather;
+        if (!rc) rc = time_steps(gathered);
+        if (rc) kind = kind0;
+        else if (tiled <= gathered) kind = 2;
+        P->step_form = form0;
+    }
+    const bool on_tiles = tiles_apply(*P);
     for (int kid : kids) {
         if (rc) break;
+        // on tiles the workgroup size follows from the tile.  A mesh without tiles runs the gather kernels at kind 2
+        // too, lambda inline as at kind 0; 2 is kept for meshes admitted later.
+        std::vector<int> sizes = {128, 256, 512}, kinds = {0};
+        if (on_tiles) sizes = {P->tune.k[kid].block};
+        if (kid == KID_FCT_LO) {
+            if (on_tiles) kinds = {2};
+            else kinds = {P->ntile > 0 ? 0 : 2, 1};
+        }
         LaunchCfg best = P->tune.k[kid];
         double best_ms = std::numeric_limits<double>::infinity();
-        for (int cand = 0; cand < 3 * 2 * kinds_of(kid) && !rc; ++cand) {
-            const int b = blocks[cand % 3], remap = (cand / 3) % 2, kind = cand / 6;
-            {
-                if (!block_supported(kid, b)) continue;
-                if (kid == KID_FCT_LO && kind == 2 && (b != 256 || P->ntile == 0)) continue;   // one workgroup size
-                P->tune.k[kid] = LaunchCfg{b, remap, kind};
-                double ms_min = std::numeric_limits<double>::infinity();
-                for (int t = 0; t < trials && !rc; ++t) {
-                    P->timing = true;
-                    P->timed_name = kKernelNames[kid];
-                    P->tk.used = 0;
-                    dirty = true;
-                    if ((rc = pool_queue_steps(P, steps))) break;
-                    if (++trial_no == fail_at) {
-                        rc = fail(SWE_EHIP, "tuning run: failure injected at trial %d (SWE_TUNE_FAIL_AT)", trial_no);
-                        break;
-                    }
-                    if ((e = hipStreamSynchronize(P->stream)) != hipSuccess) {
-                        rc = fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(e));
-                        break;
-                    }
-                    double sum = 0.0;
-                    for (int q = 0; q < P->tk.used; ++q) {
-                        float ms = 0.0f;
-                        (void)hipEventElapsedTime(&ms, P->tk.ev[(size_t)2 * q], P->tk.ev[(size_t)2 * q + 1]);
-                        sum += ms;
-                    }
-                    ms_min = std::min(ms_min, sum);
-                    if ((e = restore()) != hipSuccess) rc = fail(SWE_EHIP, "tuning restore: %s", hipGetErrorString(e));
-                    else dirty = false;
+        bool launched = true;
+        for (int cand = 0; cand < (int)(sizes.size() * 2 * kinds.size()) && launched && !rc; ++cand) {
+            const int ns = (int)sizes.size(), b = sizes[(size_t)(cand % ns)];
+            if (!block_supported(kid, b)) continue;
+            P->tune.k[kid] = LaunchCfg{b, (cand / ns) % 2, kinds[(size_t)(cand / (2 * ns))]};
+            double ms_min = std::numeric_limits<double>::infinity();
+            for (int t = 0; t < trials && launched && !rc; ++t) {
+                P->timing = true;
+                P->timed_name = kKernelNames[kid];
+                P->tk.used = 0;
+                dirty = true;
+                if ((rc = pool_queue_steps(P, steps))) break;
+                if ((rc = end_trial())) break;
+                double sum = 0.0;
+                for (int q = 0; q < P->tk.used; ++q) {
+                    float ms = 0.0f;
+                    (void)hipEventElapsedTime(&ms, P->tk.ev[(size_t)2 * q], P->tk.ev[(size_t)2 * q + 1]);
+                    sum += ms;
                 }
-                if (ms_min < best_ms) {
-                    best_ms = ms_min;
-                    best = P->tune.k[kid];
-                }
+                launched = P->tk.used > 0;
+                ms_min = std::min(ms_min, sum);
+                rc = undo();
+            }
+            if (launched && !rc && ms_min < best_ms) {
+                best_ms = ms_min;
+                best = P->tune.k[kid];
             }
         }
         P->tune.k[kid] = best;
@@ -1240,50 +1295,23 @@ int pool_tune(Pool* P, int steps, int trials) {
     P->timing = timing0;
     P->timed_name = name0;
     P->tk.used = 0;
-    // the step form, on whole steps: the launch sequence (captured graph when enabled) or the
-    // persistent step; the first run of each form is untimed (graph capture, code load)
+    // the step form: the launch sequence (captured graph when enabled) or the persistent step
     if (!rc && persistent_applies(*P)) {
-        hipEvent_t ev[2] = {nullptr, nullptr};
-        e = hipEventCreate(&ev[0]);
-        if (e == hipSuccess) e = hipEventCreate(&ev[1]);
-        if (e != hipSuccess) rc = fail(SWE_EHIP, "tuning events: %s", hipGetErrorString(e));
-        const int form0 = P->step_form;
         int best_form = form0;
         double best_ms = std::numeric_limits<double>::infinity();
         for (int form = 0; form <= 1 && !rc; ++form) {
             P->step_form = form;
-            double ms_min = std::numeric_limits<double>::infinity();
-            for (int t = 0; t <= trials && !rc; ++t) {
-                dirty = true;
-                if ((e = hipEventRecord(ev[0], P->stream)) != hipSuccess) {
-                    rc = fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(e));
-                    break;
-                }
-                if ((rc = pool_queue_steps(P, steps))) break;
-                if (++trial_no == fail_at) {
-                    rc = fail(SWE_EHIP, "tuning run: failure injected at trial %d (SWE_TUNE_FAIL_AT)", trial_no);
-                    break;
-                }
-                if ((e = hipEventRecord(ev[1], P->stream)) == hipSuccess) e = hipStreamSynchronize(P->stream);
-                if (e != hipSuccess) {
-                    rc = fail(SWE_EHIP, "tuning run: %s", hipGetErrorString(e));
-                    break;
-                }
-                float ms = 0.0f;
-                (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
-                if (t > 0) ms_min = std::min(ms_min, (double)ms);
-                if ((e = restore()) != hipSuccess) rc = fail(SWE_EHIP, "tuning restore: %s", hipGetErrorString(e));
-                else dirty = false;
-            }
-            if (ms_min < best_ms) {
+            double ms_min = 0.0;
+            rc = time_steps(ms_min);
+            if (!rc && ms_min < best_ms) {
                 best_ms = ms_min;
                 best_form = form;
             }
         }
         P->step_form = rc ? form0 : best_form;
-        for (hipEvent_t x : ev)
-            if (x) (void)hipEventDestroy(x);
     }
+    for (hipEvent_t x : ev)
+        if (x) (void)hipEventDestroy(x);
     if (dirty) {
         // a trial failed part-way: wait for what it queued, then restore the snapshot; a failed
         // restore is reported on its own (the tuning error is kept in the message)

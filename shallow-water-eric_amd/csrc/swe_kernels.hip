@@ -1586,10 +1586,12 @@ int launch_euler_stage(Pool& P, const Node* U, const Node* Uo, Node* out, const 
             timed_end(P, KID_APPLY);
         }
     } else {  // entropy_visc
+        timed_begin(P, KID_FCT_LO);
         if (quads) launch_quad_lo(P, U, d0, alpha, false);
         else if (tiles_apply(P)) launch_tile_lo(P, U, d0, alpha, false);
         else if (alpha) launch_fct_lo<true, false>(P, U, d0);
         else launch_fct_lo<false, false>(P, U, d0);
+        timed_end(P, KID_FCT_LO);
         timed_begin(P, KID_EV);
         if (quads) {
             launch_quad_ev(P, U, Uo, out, stage, bdy);
