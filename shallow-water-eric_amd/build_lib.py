@@ -20,7 +20,7 @@ CSRC = os.path.join(PKG, "csrc")
 SOURCES = [os.path.join(CSRC, f) for f in ("swe_kernels.hip", "swe_tiles.hip", "swe_quads.hip", "swe_engine.cpp", "swe_capi.cpp", "swe_setup.cpp",
                                                               "swe_setup_device.hip", "swe_errors.hip")]
 HEADERS = [os.path.join(REPO, "include", "swe_amd.h")] + [os.path.join(CSRC, f) for f in
-                                                          ("swe_kernels.h", "swe_rows.h", "swe_tile.h", "swe_layout.h", "swe_engine.h", "swe_p1.h")]
+                                                          ("swe_kernels.h", "swe_rows.h", "swe_tile.h", "swe_layout.h", "swe_order.h", "swe_engine.h", "swe_p1.h")]
 
 
 def hipcc():

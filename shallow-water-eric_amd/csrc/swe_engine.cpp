@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "swe_engine.h"
+#include "swe_order.h"
 
 namespace swe {
 
@@ -235,76 +236,6 @@ int validate_mesh(const swe_mesh_desc& d) {
     return SWE_OK;
 }
 
-namespace {
-
-// Locality order of the CSR graph, for a mesh handed over without coordinates: the rows are bisected
-// recursively, each part in the order of a breadth-first sweep from an end of it, so that every cut goes
-// across the part's longer dimension and runs of consecutive rows are compact in every direction.  Cuts
-// fall on multiples of the largest tile's rows while a part is larger than that, of a slice's below.  (A
-// reverse Cuthill-McKee order makes runs thin strips: the 256 rows of a tile of a 50,000-node mesh then
-// border on about 450 rows instead of 80.)
-struct Bisector {
-    const swe_mesh_desc& d;
-    std::vector<int> order;
-    std::vector<int> mark;             // stamp of the part or sweep that holds the node
-    std::atomic<int> stamp{0};
-
-    explicit Bisector(const swe_mesh_desc& m) : d(m), order((size_t)m.np), mark((size_t)m.np, -1) {
-        for (int i = 0; i < m.np; ++i) order[(size_t)i] = i;
-    }
-    // Breadth-first sweep from s over the nodes stamped `from`, restamped `to`, appended to seq.
-    void sweep(int s, int from, int to, std::vector<int>& seq) {
-        size_t h = seq.size();
-        seq.push_back(s);
-        mark[(size_t)s] = to;
-        for (; h < seq.size(); ++h)
-            for (int p = d.ia[seq[h]] - 1; p < d.ia[seq[h] + 1] - 1; ++p) {
-                const int v = d.ja[p] - 1;
-                if (mark[(size_t)v] == from) {
-                    mark[(size_t)v] = to;
-                    seq.push_back(v);
-                }
-            }
-    }
-    void run(int b, int e, int depth) {
-        const int n = e - b;
-        if (n <= 64) return;
-        const int part = stamp.fetch_add(3), seen = part + 1, done = part + 2;
-        for (int q = b; q < e; ++q) mark[(size_t)order[(size_t)q]] = part;
-        std::vector<int> seq, first;
-        seq.reserve((size_t)n);
-        for (int q = b; q < e; ++q) {                      // one connected piece after another
-            if (mark[(size_t)order[(size_t)q]] != part) continue;
-            first.clear();
-            sweep(order[(size_t)q], part, seen, first);
-            sweep(first.back(), seen, done, seq);
-            for (int u : first)                            // (one-way references may leave some behind)
-                if (mark[(size_t)u] == seen) sweep(u, seen, done, seq);
-        }
-        std::copy(seq.begin(), seq.end(), order.begin() + b);
-        std::vector<int>().swap(seq);
-        const int unit = (n > 64 * kMaxTileSlices) ? 64 * kMaxTileSlices : 64;
-        const int m = b + std::max(1, (n / 2 + unit / 2) / unit) * unit;
-        if (m >= e) return;
-        if (depth < 5 && n > (1 << 15)) {
-            std::thread t([=] { run(b, m, depth + 1); });
-            run(m, e, depth + 1);
-            t.join();
-        } else {
-            run(b, m, depth + 1);
-            run(m, e, depth + 1);
-        }
-    }
-};
-
-std::vector<int> locality_order(const swe_mesh_desc& d) {
-    Bisector B(d);
-    B.run(0, d.np, 0);
-    return std::move(B.order);
-}
-
-}  // namespace
-
 bool reorder_enabled() {
     const char* v = std::getenv("SWE_REORDER");
     return !v || std::atoi(v) != 0;
@@ -339,7 +270,7 @@ int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostL
     L.iperm.resize((size_t)np);
     std::vector<int> base((size_t)np);
     for (int i = 0; i < np; ++i) base[(size_t)i] = i;
-    if (reorder_enabled()) base = locality_order(d);
+    if (reorder_enabled()) base = locality_order(d, 64, 64 * kMaxTileSlices);
     const int W = sort_window > 0 ? sort_window : 64 * tile_slices;
     const int nwin = (np + W - 1) / W;
     parallel_for(nwin, [&](int64_t b, int64_t e) {
