@@ -255,7 +255,9 @@ int tile_slices_for(int64_t rows) { return rows <= 48 * 1024 ? 1 : rows <= 128 *
 // length.  Within a tile the order costs nothing, its rows being staged in LDS as a whole, and a wave
 // iterates to the longest of 64 rows of about one length instead of the longest of any 64 (per 100 steps
 // against windows of 64: FCT run of 100k nodes 14.7 -> 14.0 ms, of 1M 70.7 -> 67.6, first order 500k 21.8 ->
-// 20.7).  Only the processing order and placement change; each row keeps its entries in the caller's order,
+// 20.7).  A mesh whose halos do not fit its tiles is run by the gather kernels, which want the 64 rows of a slice to
+// be neighbours: windows of 64 there (FCT step of a row-numbered lattice under SWE_REORDER=0, 490k nodes 584 -> 573 us,
+// 4M 3723 -> 3531).  Only the processing order and placement change; each row keeps its entries in the caller's order,
 // which is the order of every row sum.
 int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostLayout& L) {
     int rc = validate_mesh(d);
@@ -389,6 +391,7 @@ int build_layout(const swe_mesh_desc& d, int sort_window, int tile_slices, HostL
         }
     }, 64);
     L.max_halo = fits ? longest.load() : -1;
+    if (L.max_halo < 0 && W > 64 && sort_window <= 0) return build_layout(d, 64, tile_slices, L);
     const int* src[3] = {d.h_dir, d.ux_dir, d.uy_dir};
     const int ns[3] = {d.n_h_dir, d.n_ux_dir, d.n_uy_dir};
     for (int k = 0; k < 3; ++k) {

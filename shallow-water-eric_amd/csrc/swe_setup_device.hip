@@ -374,19 +374,57 @@ __global__ void k_lay_len(int np, const int64_t* __restrict__ ia0, int* __restri
     if (l > swe::kMaxRow || l < 1) atomicOr(bad, 1);
 }
 
+// A set of rows in LDS, filled by a workgroup (open addressing; far past a halo's capacity it takes no more).
+constexpr int kTileHash = 1024;
+static_assert(kTileHash == 1024, "tile_hash gives 10 bits");
+__device__ __forceinline__ int tile_hash(int j) { return (int)(((unsigned)j * 2654435761u) >> 22); }
+__device__ __forceinline__ void tile_insert(int* key, int* count, int j) {
+    for (int h = tile_hash(j), n = 0; n < kTileHash; ++n, h = (h + 1) & (kTileHash - 1)) {
+        const int old = atomicCAS(key + h, -1, j);
+        if (old == j) return;
+        if (old == -1) {
+            atomicAdd(count, 1);
+            return;
+        }
+    }
+}
+
+// One workgroup per tile of the caller's numbering: sets *wide where its entries refer to more outside rows than a
+// tile may have (which does not depend on the order of the rows within the tile).
+__global__ void __launch_bounds__(256)
+k_lay_fits(int np, int tile_slices, const int64_t* __restrict__ ia0, const int* __restrict__ ja, int* __restrict__ wide) {
+    __shared__ int key[kTileHash];
+    __shared__ int count;
+    const int nsl = (np + 63) / 64, t0 = (int)blockIdx.x * tile_slices;
+    const int ns = (nsl - t0 < tile_slices) ? nsl - t0 : tile_slices;
+    const int row0 = t0 * 64, row1 = (row0 + 64 * ns < np) ? row0 + 64 * ns : np;
+    for (int q = threadIdx.x; q < kTileHash; q += blockDim.x) key[q] = -1;
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    for (int r = row0 + (int)threadIdx.x; r < row1; r += blockDim.x)
+        for (int64_t p = ia0[r]; p < ia0[r + 1]; ++p) {
+            const int j = ja[p] - 1;
+            if (j < row0 || j >= row1) tile_insert(key, &count, j);
+        }
+    __syncthreads();
+    if (threadIdx.x == 0 && count > swe::tile_halo_cap(tile_slices, ns)) atomicOr(wide, 1);
+}
+
 // One workgroup per tile, one thread per row of it in the base order (base[p], or p when base is null): each
-// row's rank among the tile's by (length, position in the base order).
+// row's rank among the tile's by (length, position in the base order); among its slice's where *wide is set.
 __global__ void __launch_bounds__(64 * swe::kMaxTileSlices)
-k_lay_sort(int np, const int* __restrict__ lenc, const int* __restrict__ base, int* __restrict__ perm) {
+k_lay_sort(int np, const int* __restrict__ lenc, const int* __restrict__ base, const int* __restrict__ wide,
+           int* __restrict__ perm) {
     __shared__ int key[64 * swe::kMaxTileSlices];
     const int n = (int)blockDim.x, k = (int)threadIdx.x;
     const int w0 = (int)blockIdx.x * n, pos = w0 + k;
     const int i = (pos < np) ? (base ? base[pos] : pos) : 0;
     const int mine = (pos < np) ? lenc[i] * n + k : 0x7fffffff;
+    const int first = *wide ? (k & ~63) : 0, end = *wide ? first + 64 : n;
     key[k] = mine;
     __syncthreads();
-    int rank = 0;
-    for (int m = 0; m < n; ++m) rank += (key[m] < mine) ? 1 : 0;
+    int rank = first;
+    for (int m = first; m < end; ++m) rank += (key[m] < mine) ? 1 : 0;
     if (pos < np) perm[w0 + rank] = i;
 }
 
@@ -592,10 +630,9 @@ __global__ void k_lay_slice_info(int nsl, int64_t s0, int64_t p0, int64_t e0, in
 }
 
 // One workgroup per tile: the distinct rows outside the tile that its entries refer to, collected in a hash
-// set in LDS (open addressing; a tile past the halo capacity gives up),
+// set in LDS (a tile past the halo capacity gives up),
 // ranked by counting (ascending, as the host layout sorts them), every entry's column within the tile,
 // and the longest list (INT_MAX: one past the capacity).  Runs after k_lay_fill (global columns) and k_lay_slice_info.
-constexpr int kTileHash = 1024;
 __global__ void __launch_bounds__(256)
 k_lay_tiles(int nsl, int64_t s0, int tile_slices, const uint8_t* __restrict__ len8, const int* __restrict__ col,
             swe::SliceInfo* __restrict__ sl, uint16_t* __restrict__ lcol, int* __restrict__ halo,
@@ -612,22 +649,13 @@ k_lay_tiles(int nsl, int64_t s0, int tile_slices, const uint8_t* __restrict__ le
     for (int q = threadIdx.x; q < kTileHash; q += blockDim.x) key[q] = -1;
     if (threadIdx.x == 0) count = 0;
     __syncthreads();
-    auto slot_of = [&](int j) { return (int)(((unsigned)j * 2654435761u) >> 22); };   // 10 bits
-    static_assert(kTileHash == 1024, "slot_of gives 10 bits");
     for (int r = threadIdx.x; r < 64 * ns; r += blockDim.x) {
         const int L = len8[row0 + r];
         const int64_t base = sl[g0 + (r >> 6)].sbase + (r & 63);
         for (int q = 0; q < L; ++q) {
             const int j = col[base + 64 * (int64_t)q];
             if (j >= row0 && j < row1) continue;
-            for (int h = slot_of(j), n = 0; n < kTileHash; ++n, h = (h + 1) & (kTileHash - 1)) {
-                const int old = atomicCAS(key + h, -1, j);
-                if (old == j) break;
-                if (old == -1) {
-                    atomicAdd(&count, 1);
-                    break;
-                }
-            }
+            tile_insert(key, &count, j);
         }
     }
     __syncthreads();
@@ -658,7 +686,7 @@ k_lay_tiles(int nsl, int64_t s0, int tile_slices, const uint8_t* __restrict__ le
             const int j = col[p];
             int l = j - row0;
             if (j < row0 || j >= row1) {
-                int h = slot_of(j);
+                int h = tile_hash(j);
                 while (key[h] != j) h = (h + 1) & (kTileHash - 1);
                 l = 64 * tile_slices + pos[h];
             }
@@ -768,7 +796,7 @@ int build_layout_device(const swe_assembly* a, int tile_slices, DeviceLayout& DL
     keep.add(&DL.len, (size_t)np_pad);
     keep.add(&DL.sptr, (size_t)nsl + 1);
     keep.add(&DL.eoff, (size_t)nsl + 1);
-    temp.add(&flag, 2);
+    temp.add(&flag, 3);        // row-length check, longest row, halos too long
     const size_t zeroed = temp.bytes();
     temp.add(&sums, 4);
     temp.add(&lenc, (size_t)np);
@@ -785,8 +813,12 @@ int build_layout_device(const swe_assembly* a, int tile_slices, DeviceLayout& DL
     int64_t h[4] = {0, 0, 0, 0};
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_lay_len, dim3(grid_of(np, 256)), dim3(256), 0, s, np, (const int64_t*)a->ia0, lenc, flag);
+        // a numbering of the caller's may be no order for tiles (build_layout says why the windows are slices there)
+        if (!base && tile_slices > 1)
+            hipLaunchKernelGGL(k_lay_fits, dim3(grid_of(nsl, tile_slices)), dim3(256), 0, s, np, tile_slices,
+                               (const int64_t*)a->ia0, (const int*)a->ja, flag + 2);
         hipLaunchKernelGGL(k_lay_sort, dim3(grid_of(nsl, tile_slices)), dim3(64 * tile_slices), 0, s, np,
-                           (const int*)lenc, base, DL.perm);
+                           (const int*)lenc, base, (const int*)(flag + 2), DL.perm);
         hipLaunchKernelGGL(k_lay_iperm, dim3(grid_of(np_pad, 256)), dim3(256), 0, s, np, np_pad, (const int*)DL.perm,
                            (const int*)lenc, DL.iperm, DL.len);
         hipLaunchKernelGGL(k_lay_slices, dim3(grid_of(nsl + 1, 256)), dim3(256), 0, s, nsl, np, (const int*)DL.len, slots,
