@@ -953,6 +953,7 @@ int ensure_graph(Pool* P) {
         P->wmax,
         P->mode.viscosity_type * 128 + P->mode.viscous_type * 16 + P->mode.alpha * 4 + P->mode.roundoff * 2 +
             (P->any_src ? 1 : 0),
+        P->mode.sgn,
         tuning_hash(P->tune),
         (P->one < 0) ? -1 : (int64_t)P->one * (1ll << 32) + P->inst[(size_t)P->one].slice0};
     if (P->gexec && key == P->graph_key) return SWE_OK;

@@ -49,7 +49,7 @@ struct Tuning {
 bool block_supported(int kid, int block);
 
 // Words of Pool::graph_key.
-constexpr int kGraphKey = 10;
+constexpr int kGraphKey = 11;
 // Words of Pool::done: one per group of workgroups and one for the groups, a cache line each.
 constexpr unsigned kDoneGroups = 64, kDoneStride = 32;
 

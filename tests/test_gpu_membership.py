@@ -61,3 +61,24 @@ def test_other_meshes_of_as_many_slices(oracle, rows, first, then):
                 b.remove(k)
         ref, rt = state_of(big, total)
         assert b.status(kb)[1] == rt and same_bits(b.get_state(kb), ref)
+
+
+def test_another_model_on_the_same_rows(oracle):
+    """An emptied batch takes another model: the five components of test 13 after the three of test 11, whose step has
+    the same launch extents and scheme."""
+    from conftest import golden
+    from swe_amd.batch import Batch
+    from swe_amd.solver import MeshArrays, make_params
+    z = golden("sgn_run.npz")
+    g, htiny, hmax, cfl = z["scalars"]
+    kw = dict(gravity=g, htiny=htiny, cfl=cfl, max_water_h=hmax, alpha_limit=True)
+    with Batch(8192, 80000, 64, 2) as b:
+        for tt, lam, u in ((11, 0.0, np.ascontiguousarray(z["states"][1][:, :3])), (13, float(z["lambda_sgn"]), z["states"][1])):
+            ref, _, rt, err = oracle.Oracle(z["ia"], z["ja"], z["cij"], z["lumped"], z["bath"], type_test=tt, lambda_sgn=lam,
+                                            viscosity_type=oracle.VISCOUS, **kw).run(u, 4)
+            assert err == 0
+            k = b.add(MeshArrays(z["ia"], z["ja"], z["cij"], z["lumped"], z["bath"]),
+                      make_params(viscosity="viscous", type_test=tt, lambda_sgn=lam, **kw), u)
+            b.step(4)
+            assert b.status(k)[1] == rt and same_bits(b.get_state(k), ref), tt
+            b.remove(k)
