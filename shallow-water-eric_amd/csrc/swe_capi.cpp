@@ -27,6 +27,7 @@ struct swe_handle {
     long long queued = 0;           // steps queued so far (the instance's step counter)
     bool state_set = false;
     bool step_open = false;         // swe_step_begin ran; swe_step_finish completes the step
+    bool dij_kept = false;          // and no call has changed what its d_ij were evaluated from, nor used their memory
     int bc_kind = SWE_BC_NONE;
 };
 
@@ -319,6 +320,7 @@ int swe_destroy(swe_handle* h) {
 
 int swe_set_params(swe_handle* h, const swe_params* prm) {
     if (!h || !prm) return fail(SWE_EINVAL, "null argument");
+    h->dij_kept = false;
     return pool_set_params(h->P, kId, *prm);
 }
 
@@ -336,6 +338,7 @@ int swe_set_bc_values(swe_handle* h, const double* hv, const double* uxv, const 
 
 int swe_set_state(swe_handle* h, const double* un) {
     if (!h || !un) return fail(SWE_EINVAL, "null argument");
+    h->dij_kept = false;
     int rc = pool_upload_state(h->P, kId, un, h->P->S[0]);
     if (rc) return rc;
     SWE_HIPCHK(hipStreamSynchronize(h->P->stream));
@@ -393,6 +396,7 @@ int swe_euler(swe_handle* h, const double* un, double* unext, double dt) {
 
 int swe_fct_positivity(swe_handle* h, const double* us, const double* f, double* lij) {
     if (!h || !us || !f || !lij) return fail(SWE_EINVAL, "null argument");
+    h->dij_kept = false;
     Pool* P = h->P;
     const InstHost& I = P->inst[kId];
     double htiny = 0.0;
@@ -519,6 +523,7 @@ int swe_run(swe_handle* h, int nsteps, double* time, double* dts) {
     if (!h) return fail(SWE_EINVAL, "null handle");
     if (nsteps < 0) return fail(SWE_EINVAL, "nsteps < 0");
     if (!h->state_set) return fail(SWE_EINVAL, "no state has been set");
+    h->dij_kept = false;
     int rc;
     if (time && (rc = swe_set_time(h, *time))) return rc;
     if (dts && (rc = ensure_dt_log(h, nsteps))) return rc;
@@ -557,6 +562,7 @@ int swe_step_begin(swe_handle* h, double* dt) {
     }
     if ((rc = read_field(P, kId, offsetof(InstDev, dt), dt, sizeof *dt))) return rc;
     h->step_open = true;
+    h->dij_kept = true;
     h->queued += 1;
     return SWE_OK;
 }
@@ -574,8 +580,8 @@ int swe_step_finish(swe_handle* h, const double* vals) {
             SWE_HIPCHK(hipMemcpyAsync(P->bcv + st * P->bcv_stride + I.bc0, vals + st * n, sizeof(double) * (size_t)n,
                                       hipMemcpyHostToDevice, P->stream));
     }
-    // (the caller may have set a schedule or parameters, or run swe_euler, since swe_step_begin)
-    int rc = record_stages(P, false);
+    // (no alpha factors: the caller may have set a schedule or run swe_euler since swe_step_begin)
+    int rc = record_stages(P, h->dij_kept, false);
     if (rc) return rc;
     SWE_HIPCHK(hipGetLastError());
     return check_flags(P, kId);
@@ -585,6 +591,7 @@ int swe_run_async(swe_handle* h, int nsteps) {
     if (!h) return fail(SWE_EINVAL, "null handle");
     if (nsteps < 0) return fail(SWE_EINVAL, "nsteps < 0");
     if (!h->state_set) return fail(SWE_EINVAL, "no state has been set");
+    h->dij_kept = false;
     const int rc = pool_queue_steps(h->P, nsteps);
     if (!rc) h->queued += nsteps;
     return rc;
@@ -610,6 +617,7 @@ int swe_kernel_timing(swe_handle* h, const char* kernel, int* launches, double* 
 int swe_tune(swe_handle* h, int steps) {
     if (!h) return fail(SWE_EINVAL, "null handle");
     if (!h->state_set) return fail(SWE_EINVAL, "no state has been set");
+    h->dij_kept = false;
     return pool_tune(h->P, steps, 2);
 }
 

@@ -909,8 +909,8 @@ int record_dt(Pool* P) {
     return SWE_OK;
 }
 
-int record_stages(Pool* P, bool same_call) {
-    const bool lam = P->mode.viscosity_type != SWE_GALERKIN;
+int record_stages(Pool* P, bool dij, bool alpha) {
+    const bool lam = dij && P->mode.viscosity_type != SWE_GALERKIN;
     Node* A = P->S[0];
     Node* B = P->S[1];
     Node* C = P->S[2];
@@ -919,7 +919,8 @@ int record_stages(Pool* P, bool same_call) {
     Node* out[3] = {B, C, A};
     for (int stage = 0; stage < 3; ++stage) {
         const bool first = lam && stage == 0;
-        const int rc = launch_euler_stage(*P, in[stage], A, out[stage], first ? P->d0 : nullptr, first && same_call, stage, true);
+        const int rc = launch_euler_stage(*P, in[stage], A, out[stage], first ? P->d0 : nullptr, first && alpha, stage,
+                                          true);
         if (rc) return rc;
         if (lists) launch_bdy(*P, out[stage], stage);
     }
@@ -930,7 +931,7 @@ namespace {
 
 int record_step(Pool* P) {
     const int rc = record_dt(P);
-    return rc ? rc : record_stages(P, true);
+    return rc ? rc : record_stages(P, true, true);
 }
 
 int64_t tuning_hash(const Tuning& t) {

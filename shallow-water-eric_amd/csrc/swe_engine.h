@@ -267,8 +267,9 @@ int pool_queue_steps(Pool* P, int nsteps);
 // The parts of one step, launched on the compute stream: the dt pass and its bookkeeping, then the
 // three stages with bdy.
 int record_dt(Pool* P);
-// same_call: nothing came between this and record_dt, so what the dt pass left beside d0 still holds.
-int record_stages(Pool* P, bool same_call);
+// dij, alpha: the first stage may take the d_ij and, on tiles, the alpha factors that record_dt left (its state,
+// parameters and memory are as they were).
+int record_stages(Pool* P, bool dij, bool alpha);
 // Rebuild the launch list from the instances marked listed (ordered on the compute stream).
 int pool_update_active(Pool* P);
 int pool_read_table(Pool* P);         // sync, then tab_host / flags_host hold the table
