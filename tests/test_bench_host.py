@@ -44,3 +44,15 @@ def test_fifo_replay():
     before it ends, whichever is later."""
     fin = bench.replay_fifo([0.0, 0.5, 10.0], [2.0, 1.0, 1.0])
     assert fin == pytest.approx([2.0, 3.0, 11.0])
+
+
+def test_profile_figures_are_those_of_the_kernel_that_runs():
+    """The counters beside a launch time are of the kernel launched: k_tile_lo where the schedule's kind is 2."""
+    sched = {"k_fct_lo": (256, 1, 2), "k_stage_lo": (256, 1, 0)}
+    assert bench.launched_kernel("k_fct_lo", sched) == "k_tile_lo"
+    assert bench.launched_kernel("k_stage_lo", sched) == "k_stage_lo"
+    assert bench.launched_kernel("k_fct_lo", {"k_fct_lo": (256, 1, 0)}) == "k_fct_lo"
+    tile, gather = (bench.measured_traffic(k, "bumps_pd", 16716273) for k in ("k_tile_lo", "k_fct_lo"))
+    assert tile is not None and tile != gather
+    busy, lanes = bench.measured_valu("k_tile_lo", "bumps_pd", 16716273)
+    assert 0.0 < busy <= 1.0 and 0.0 < lanes <= 1.0
