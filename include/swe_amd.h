@@ -114,7 +114,9 @@ int swe_assembly_destroy(swe_assembly *a);
  * state built by construct_matrices (SOURCES/update.f90:18-132) and construct_mesh.
  * The environment variable SWE_SORT_WINDOW (default: the rows of a tile, 64 to 256) sets the
  * window of rows inside which the internal numbering sorts rows by length; SWE_REORDER=0 keeps the
- * caller's numbering as the base order instead of a locality order of the mesh graph.  These are layout choices; results do not depend on them. */
+ * caller's numbering as the base order instead of a locality order of the mesh graph (a mesh whose
+ * halos are then too long for tiles is sorted inside windows of 64).  These are layout choices; results
+ * do not depend on them. */
 int swe_create(const swe_mesh_desc *mesh, const swe_params *prm, swe_handle **out);
 /* swe_create over a mesh assembled by swe_assemble_device, without taking the matrices to the
  * host: the solver's layout is built on the GPU from the assembly (rows sorted by length inside
@@ -244,21 +246,25 @@ int swe_stream_bandwidth(unsigned long long bytes, int reps, double *read_gbs, d
 
 /* Launch schedules: per kernel, the workgroup size (128, 256 or 512) and whether workgroups are
  * ordered XCD-aware (1) or in dispatch order (0).  Kernels, in this order: k_compute_dt, k_alpha,
- * k_stage_lo, k_fct_lo, k_fct_rminus, k_fct_apply, k_ev_update.  swe_tune times every schedule
- * of each kernel the scheme uses on the handle's own mesh and state (the state and time are
- * restored afterwards) and keeps the fastest; results do not depend on the schedule.  The
- * first-order and SGN stages (k_stage_lo) take their workgroup size and order from the same entry.
+ * k_stage_lo, k_fct_lo, k_fct_rminus, k_fct_apply, k_ev_update.  swe_tune decides between the tile and
+ * the gather kernels by whole steps, then times the schedules of each kernel the step launches, on the
+ * handle's own mesh and state (the state and time are restored afterwards), and keeps the fastest;
+ * results do not depend on the schedule.  On tiles the workgroup size follows from the tile: the
+ * schedule's is the gather kernels'.  The first-order and SGN stages (k_stage_lo) take their order, and
+ * in the gather kernels their workgroup size, from the same entry.
  * SWE_TUNE_FAIL_AT=n (environment, for the test of the restore path) makes the n-th trial fail
  * after its steps are queued; unset or 0 never. */
 #define SWE_NUM_KERNELS 7
 int swe_tune(swe_handle *h, int steps);
 int swe_get_schedule(swe_handle *h, int *blocks, int *remap);
 int swe_set_schedule(swe_handle *h, const int *blocks, const int *remap);
-/* The schedule kind per kernel (same order), a third axis of swe_tune: k_fct_lo in stages 2 and 3
- * has kind 0 (lambda_ij evaluated per entry inside each lane's row loop) and kind 1 (lambda_ij
- * evaluated first entry-parallel, one off-diagonal entry per lane, into LDS, then read by the row
- * loop); every other kernel has kind 0 only.  swe_set_schedule_kinds returns SWE_EINVAL for a kind
- * a kernel does not have.  Results do not depend on the kind. */
+/* The schedule kind per kernel (same order).  The kind of k_fct_lo chooses the kernels of every pass, in
+ * every scheme: 2 (the default) the tile kernels, which stage the rows of a tile and their neighbours in
+ * LDS (a mesh with a halo too long for its tiles, and every mesh of its batch with it, runs the gather
+ * kernels with lambda inline); 0 and 1 the gather kernels, with lambda_ij evaluated in the low-order pass of
+ * stages 2 and 3 per entry inside each lane's row loop (0) or first entry-parallel, one off-diagonal
+ * entry per lane, into LDS (1).  Every other kernel has kind 0 only.  swe_set_schedule_kinds returns
+ * SWE_EINVAL for a kind a kernel does not have.  Results do not depend on the kind. */
 int swe_get_schedule_kinds(swe_handle *h, int *kinds);
 int swe_set_schedule_kinds(swe_handle *h, const int *kinds);
 /* Queue steps as one captured HIP graph per step (1, the default) or as individual launches (0).
