@@ -295,7 +295,7 @@ def bench_batch(count, steps, warmup, workers, tune=True, seed=20261202, nmin=50
     compute_dij and euler per stage, `dropin_steps` steps per mesh, on the first `dropin_count`
     meshes, a random sample of the family, when given).  device_setup: the batch and the
     device-resident loop admit each mesh from its element list (assembly and layout on the GPU, with
-    the Hilbert locality order) rather than from the host assembly and layout (reverse Cuthill-McKee)."""
+    the Hilbert locality order) rather than from the host assembly and layout (order by bisection)."""
     from swe_amd import problems
     from swe_amd.batch import Batch
     t0 = time.perf_counter()
