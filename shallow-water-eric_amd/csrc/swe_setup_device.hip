@@ -293,7 +293,8 @@ extern "C" int swe_assemble_device(int np, int me, const int* jj, const double* 
     if (e == hipSuccess) e = hipMemcpyAsync(&total, a->ia0 + np, sizeof total, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     int rc = SWE_OK;
-    if (e == hipSuccess && (bad & kFlagRange)) {
+    if (e != hipSuccess || (bad & kFlagRange)) {
+        // (also where the device failed: an entry out of range is refused as such on any machine)
         for (int64_t q = 0; q < n3 && rc == SWE_OK; ++q)
             if (jj[q] < 1 || jj[q] > np) rc = swe::fail(SWE_EINVAL, "jj(%lld)=%d out of range", (long long)q + 1, jj[q]);
     } else if (e == hipSuccess && bad) {
@@ -319,7 +320,7 @@ extern "C" int swe_assemble_device(int np, int me, const int* jj, const double* 
         if (e == hipSuccess) e = hipStreamSynchronize(s);
     }
     dfree(work, s);
-    if (e != hipSuccess) rc = swe::fail(SWE_EHIP, "device assembly: %s", hipGetErrorString(e));
+    if (e != hipSuccess && rc == SWE_OK) rc = swe::fail(SWE_EHIP, "device assembly: %s", hipGetErrorString(e));
     if (rc != SWE_OK) {
         release(a);
         return rc;

@@ -107,3 +107,17 @@ def test_assemble_rejects_bad_elements():
     from swe_amd.solver import SweError, assemble
     with pytest.raises(SweError):
         assemble(np.array([[0, 1, 7]]), np.zeros((3, 2)))
+
+
+@pytest.mark.parametrize("bad", [0, 5, -1])
+def test_device_assembly_refuses_an_entry_out_of_range_on_any_machine(bad):
+    """swe_assemble_device names the entry also where there is no device to assemble on."""
+    import ctypes as C
+    from swe_amd.solver import SWE_EINVAL, load_library
+    lib = load_library()
+    jj = np.array([[1, 2, 3], [2, 4, bad]], np.int32)
+    rr = np.array([[0.0, 0.0], [1.0, 0.0], [0.0, 1.0], [1.0, 1.0]])
+    a, n = C.c_void_p(), C.c_longlong()
+    rc = lib.swe_assemble_device(4, 2, jj.ctypes.data_as(C.c_void_p), rr.ctypes.data_as(C.c_void_p), C.byref(a), C.byref(n))
+    assert rc == SWE_EINVAL and not a.value
+    assert lib.swe_last_error() == b"jj(6)=%d out of range" % bad
